@@ -210,6 +210,55 @@ char reduction_schedule(uint32_t mask, int32_t rank) {
   return 'g';
 }
 
+// The entries of a reduction with kept axes after a reduced one or reduced ones around a kept one
+// (schedules 'm' and 'g'), plain or over NI inputs (`x` prefixes the symbols' tails): xreduce_inner
+// when the innermost axis is reduced, a block or a wave per output; xreduce_outer when it is kept.
+// Eight waves a block and up to eight 16-byte loads in flight per lane put 64 KiB in flight per CU
+// (column sums of an 8192 x 4096 f32: one such block per CU reads at 79% of a plain read; 2 to 4
+// blocks, 256 or 1024 threads and 4 or 16 loads measured no better).  The inner entries take two
+// blocks per CU, so that one block's closing fold runs under the other's loads.
+static void emit_split(std::ostringstream& src, Lowered& L, int32_t dtype, int NI, int op, const std::string& ops,
+                const std::string& x) {
+  const char* T = ctype(dtype);
+  const int V = vec_of(dtype), U = std::max(1, 8 / NI);
+  const bool inner = (L.axes_mask >> (L.form.rank - 1)) & 1u;
+  L.threads = 512;
+  L.blocks_per_cu = inner ? 2 : 1;
+  for (int team = 0; team <= (inner ? 1 : 0); ++team)
+    for (int fast = 1; fast >= 0; --fast) {
+      Entry e;
+      e.fast = fast;
+      e.vec = fast ? V : 1;
+      e.team = team;
+      e.symbol = L.name + "_" + x + (inner ? (team ? "gw" : "g") : "m") + (fast ? "v" : "s");
+      src << "extern \"C\" __global__ void __launch_bounds__(512) " << e.symbol << "(";
+      for (int k = 0; k < NI; ++k) src << "const " << T << "* in" << k << ", ";
+      src << T << "* out, unp::red_axes d, long long S, " << (inner ? "" : "int lpr, ")
+          << "unsigned long long* partials, unsigned* counters, "
+          << "unsigned epoch, unp::waits wt) {\n  const " << T << "* in[" << NI << "] = {";
+      for (int k = 0; k < NI; ++k) src << (k ? ", " : "") << "in" << k;
+      src << "};\n  unp::" << (inner ? "xreduce_inner<" : "xreduce_outer<") << T << ", " << NI << ", " << op << ", "
+          << ops << ", " << e.vec << ", ";
+      if (inner) src << (team ? 1 : 8) << ", ";
+      src << "512, " << U << ">(in, out, d, S, " << (inner ? "" : "lpr, ") << "partials, counters, epoch, wt);\n}\n";
+      L.entries.push_back(e);
+    }
+}
+static const char* split_policy(uint32_t mask, int32_t rank) {
+  return (mask >> (rank - 1)) & 1u
+             ? "blocks stride over (chunk of the reduced positions, output) items, the last-ticket block of an "
+               "output folds its chunk partials; short reductions: waves stride over the outputs"
+             : "a wave per 64 x vec columns (or whole rows of fewer), blocks stride over (chunk of the reduced "
+               "rows, column strip) items, the last-ticket block of a strip folds its chunk partials";
+}
+static std::string split_when(const Entry& e) {
+  return std::string(e.team ? "few positions per output, or many outputs; " : "") +
+         (e.fast ? "innermost run >= vec elements" : "otherwise");
+}
+static const char* const kSplitWorkspace =
+    "{\"partials\":\"(outputs, or strips * 64 * vec) * chunks * 8 bytes per 4-byte accumulator word (tagged with the "
+    "launch epoch)\",\"counters\":\"(outputs or strips) * 4\",\"stall\":4,\"host_state\":[\"epoch\"]}";
+
 // When the executor picks an entry that reads through storage-image strides.
 static const char* const kStridedWhen =
     "a storage image that is not dense row-major (unp_hip_exec_launch_views): the view's strides";
@@ -263,24 +312,10 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
   L.name = name.str();
   std::ostringstream src;
   src << header(L.name, f);
-  if (sched == 'm') {
-    // Eight waves per block, one block per CU, 8 rows in flight per lane; blocks split the
-    // reduced extent so that a launch has about cu_count blocks (measured best for an
-    // 8192 x 4096 f32 column sum: more chunks cost more in the partials' final fold than they
-    // add in parallelism).
-    L.threads = 512;
-    L.blocks_per_cu = 1;
-    for (int fast = 1; fast >= 0; --fast) {
-      Entry e;
-      e.fast = fast;
-      e.vec = fast ? V : 1;
-      e.symbol = L.name + (fast ? "_mv" : "_ms");
-      src << "extern \"C\" __global__ void __launch_bounds__(512) " << e.symbol << "(const " << T << "* in, " << T
-          << "* out, long long A, long long R, long long B, long long S, "
-          << "unsigned long long* partials, unsigned* counters, unsigned epoch, unp::waits wt) {\n  unp::reduce_mid<" << T
-          << ", " << f.op0 << ", " << e.vec << ", 512, 8>(in, out, A, R, B, S, partials, counters, epoch, wt);\n}\n";
-      L.entries.push_back(e);
-    }
+  if (sched == 'm' || sched == 'g') {
+    std::ostringstream ops;
+    ops << "unp::plain_ops<" << T << ", " << f.op0 << ">";
+    emit_split(src, L, f.dtype, 1, f.op0, ops.str(), "");
   } else if (sched == 'q') {
     L.threads = 256;
     L.blocks_per_cu = 8;
@@ -290,16 +325,6 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
     e.symbol = L.name + "_q";
     src << "extern \"C\" __global__ void __launch_bounds__(256) " << e.symbol << "(const " << T << "* in, " << T
         << "* out, unp::red_view d) {\n  unp::reduce_serial<" << T << ", " << f.op0 << ", 256>(in, out, d);\n}\n";
-    L.entries.push_back(e);
-  } else if (sched == 'g') {
-    L.threads = 256;
-    L.blocks_per_cu = 8;
-    Entry e;
-    e.fast = false;
-    e.vec = 1;
-    e.symbol = L.name + "_g";
-    src << "extern \"C\" __global__ void __launch_bounds__(256) " << e.symbol << "(const " << T << "* in, " << T
-        << "* out, unp::axes_desc d) {\n  unp::reduce_generic<" << T << ", " << f.op0 << ", 256>(in, out, d);\n}\n";
     L.entries.push_back(e);
   } else if (L.reduce_all) {
     // One block per CU (8 waves): the read rate peaks with few streams per CU.
@@ -372,9 +397,7 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
   j << "],\"launch\":{\"block\":[" << L.threads << ",1,1],\"grid\":\"cu_count*" << L.blocks_per_cu
     << "\",\"grid_policy\":\"device-class constant; "
     << (sched == 'a'   ? "blocks stride over 16-byte vectors, last-ticket block folds the partials"
-        : sched == 'm' ? "the input as A x R x B: a wave per 64 x vec columns, blocks split R into chunks, the "
-                         "last-ticket block of a column strip folds the chunk partials in chunk order"
-        : sched == 'g' ? "one wave per output element, lanes stride over the reduced positions"
+        : (sched == 'm' || sched == 'g') ? split_policy(mask, f.rank)
         : sched == 'q' ? "one lane per output element, the reduced positions folded in the serial lift's "
                          "order (the serial accumulator, row-major over the reduced axes)"
                        : "waves stride over rows (one wave per row); rows longer than 32768 elements: one block per row")
@@ -383,13 +406,13 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
     j << (i ? "," : "") << "{\"symbol\":\"" << L.entries[i].symbol << "\",\"vec\":" << L.entries[i].vec
       << ",\"when\":\"" << (L.entries[i].wide ? "reduced extent > 32768; " : "")
       << (L.entries[i].strided ? kStridedWhen
-          : (sched == 'g' || sched == 'q') ? "always"
-          : sched == 'm' ? (L.entries[i].fast ? "B % vec == 0 and in0 16-byte aligned" : "otherwise")
+          : sched == 'q' ? "always"
+          : (sched == 'm' || sched == 'g') ? split_when(L.entries[i])
                          : (L.entries[i].fast ? "reduced extent % vec == 0 and in0 16-byte aligned" : "otherwise"))
       << "\"}";
   j << "],\"workspace\":"
     << (L.reduce_all   ? "{\"partials\":\"grid * 8 bytes per 4-byte accumulator word (tagged with the launch epoch)\",\"counter\":4,\"stall\":4,\"host_state\":[\"epoch\"]}"
-        : sched == 'm' ? "{\"partials\":\"strips * chunks * 64 * vec * 8 bytes per 4-byte accumulator word (tagged with the launch epoch)\",\"counters\":\"strips * 4\",\"stall\":4,\"host_state\":[\"epoch\"]}"
+        : (sched == 'm' || sched == 'g') ? kSplitWorkspace
                        : "null")
     << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
     << ",\"fidelity_notes\":["
@@ -1904,17 +1927,7 @@ int32_t lower_reduction_x(const unp_form& f, const ReductionExpr& rx, Lowered& L
       L.entries.push_back(e);
     }
   } else {
-    L.blocks_per_cu = 8;
-    Entry e;
-    e.fast = false;
-    e.vec = 1;
-    e.symbol = L.name + "_xg";
-    src << "extern \"C\" __global__ void __launch_bounds__(256) " << e.symbol << "(";
-    sig(src);
-    src << ", unp::axes_desc d) {\n";
-    ins(src);
-    src << "  unp::xreduce_generic<" << T << ", " << NI << ", " << f.op0 << ", " << ops << ", 256>(in, out, d);\n}\n";
-    L.entries.push_back(e);
+    emit_split(src, L, f.dtype, NI, f.op0, ops, "x");
   }
   L.source = src.str();
   std::ostringstream j;
@@ -1930,16 +1943,17 @@ int32_t lower_reduction_x(const unp_form& f, const ReductionExpr& rx, Lowered& L
   j << "],\"launch\":{\"block\":[" << L.threads << ",1,1],\"grid_policy\":\""
     << (sched == 'r'   ? "one wave per row, waves stride over rows"
         : sched == 'a' ? "blocks stride over 16-byte vectors of every input, last-ticket block folds the partials"
-                       : "one wave per output element, lanes stride over the reduced positions")
+                       : split_policy(mask, f.rank))
     << "\"},\"entries\":[";
   for (size_t i = 0; i < L.entries.size(); ++i)
     j << (i ? "," : "") << "{\"symbol\":\"" << L.entries[i].symbol << "\",\"vec\":" << L.entries[i].vec
       << ",\"when\":\""
-      << (sched == 'm' || sched == 'g' ? "always"
+      << (sched == 'm' || sched == 'g' ? split_when(L.entries[i])
           : L.entries[i].fast         ? "reduced extent % vec == 0 and every input 16-byte aligned"
                                       : "otherwise")
       << "\"}";
-  j << "],\"workspace\":" << (sched == 'a' ? "{\"partials\":\"grid * 16 (f64, tagged with the launch epoch)\",\"counter\":4,\"stall\":4,\"host_state\":[\"epoch\"]}" : "null")
+  j << "],\"workspace\":" << (sched == 'a' ? "{\"partials\":\"grid * 16 (f64, tagged with the launch epoch)\",\"counter\":4,\"stall\":4,\"host_state\":[\"epoch\"]}"
+        : sched == 'r' ? "null" : kSplitWorkspace)
     << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
     << ",\"fidelity_notes\":["
     << json_str(int_body ? "the body evaluates at the element type by the total integer rule (Add/Sub/Mul wrap, a zero "

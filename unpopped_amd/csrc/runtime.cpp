@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 
@@ -85,6 +86,15 @@ struct unp_event {
   hipEvent_t e = nullptr;
 };
 
+// One stream's workspace of a split reduction: launches on a stream follow one another, so each may
+// use the words of the one before it, told apart by the epoch.
+struct StreamWs {
+  hipStream_t stream = nullptr;
+  bool bound = false;             // to `stream`
+  uint8_t* base = nullptr;        // ticket counters (left zero by every launch), then the partials
+  uint32_t epoch = 0;
+};
+
 struct unp_exec {
   unp::Lowered l;
   hipModule_t mod = nullptr;
@@ -96,8 +106,8 @@ struct unp_exec {
   void* ws = nullptr;  // scan: tile status words; full reduction: block partials
   size_t ws_bytes = 0;
   uint32_t* counter = nullptr;
-  uint32_t* counters = nullptr;  // reduce_mid: one ticket counter per column strip, left zero
-  size_t n_counters = 0;
+  // The workspaces of a split reduction, one per stream the executor has launched it on.
+  std::vector<StreamWs> stream_ws;
   uint32_t epoch = 0;
   uint32_t ticket_base = 0;
   // Bounded waits: the word a kernel that gave up waiting counts into, read and cleared by
@@ -119,6 +129,39 @@ struct unp_exec {
   std::vector<void*> stage;
   std::vector<size_t> stage_cap;
 };
+
+namespace {
+
+// A split reduction's workspace.  The items (outputs or column strips, times chunks) of a launch that
+// splits are at most kSplitItems = 4 rounds of its grid (split_chunks): each has a ticket counter
+// at most, and its partials: one value, or a strip's 64 * vec of them, in 16 bytes at most.
+constexpr size_t kSplitRounds = 4, kMaxStreams = 4;
+bool inner_reduced(const unp::Lowered& l) { return (l.axes_mask >> (l.form.rank - 1)) & 1u; }
+size_t split_items(const unp_exec* x) { return kSplitRounds * (size_t)x->cu_count * (size_t)x->l.blocks_per_cu; }
+size_t split_counter_bytes(const unp_exec* x) { return (split_items(x) * sizeof(uint32_t) + 255) / 256 * 256; }
+size_t split_bytes(const unp_exec* x) {
+  const size_t values = inner_reduced(x->l) ? 1 : 64 * (16 / unp::kind_bytes(x->l.form.dtype));
+  return split_counter_bytes(x) + split_items(x) * values * 16;
+}
+
+bool splits(const unp_exec* x) {
+  return x->l.form.kind == UNP_FORM_REDUCTION && (x->l.red_schedule == 'g' || x->l.red_schedule == 'm');
+}
+
+hipError_t add_stream_ws(unp_exec* x) {
+  StreamWs w;
+  hipError_t e = hipMalloc((void**)&w.base, split_bytes(x));
+  if (e != hipSuccess) return e;
+  if ((e = hipMemset(w.base, 0, split_bytes(x))) == hipSuccess) e = hipDeviceSynchronize();
+  if (e != hipSuccess) {
+    hipFree(w.base);
+    return e;
+  }
+  x->stream_ws.push_back(w);
+  return hipSuccess;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -453,6 +496,10 @@ int32_t unp_hip_exec_create(const unp_generated* g, unp_exec** out, unp_error* e
       per_cu = 0;
     x->resident.push_back(per_cu);
   }
+  if (splits(x) && (e = add_stream_ws(x)) != hipSuccess) {
+    unp_hip_exec_destroy(x);
+    return hip_fail(err, "hipMalloc(split reduction workspace)", e);
+  }
   set_error(err, UNP_OK, "");
   *out = x;
   return UNP_OK;
@@ -462,7 +509,8 @@ void unp_hip_exec_destroy(unp_exec* x) {
   if (!x) return;
   if (x->ws) hipFree(x->ws);
   if (x->counter) hipFree(x->counter);
-  if (x->counters) hipFree(x->counters);
+  for (const StreamWs& w : x->stream_ws)
+    if (w.base) hipFree(w.base);
   if (x->stall) hipFree(x->stall);
   for (void* p : x->stage)
     if (p) hipFree(p);
@@ -602,15 +650,20 @@ struct Ws {
   uint32_t* counters = nullptr;
 };
 
-int32_t ensure_counters(unp_exec* x, size_t n, unp_error* err);
+size_t up256(size_t v) { return (v + 255) / 256 * 256; }
+size_t scratch_need(size_t bytes, bool need_counter, size_t n_counters) {
+  return (need_counter ? 256 : 0) + up256(n_counters * sizeof(uint32_t)) + up256(bytes);
+}
+// The last 256 bytes stay unused, so no piece ends at the region's very end.
+bool static_fits(const unp_exec* x, size_t bytes, bool need_counter, size_t n_counters) {
+  return x->fixed->cap >= 256 && scratch_need(bytes, need_counter, n_counters) <= x->fixed->cap - 256;
+}
 
 int32_t workspace(unp_exec* x, size_t bytes, bool need_counter, size_t n_counters, hipStream_t s, Ws& w,
                   unp_error* err) {
   if (x->fixed) {
-    const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t need = (need_counter ? 256 : 0) + up(n_counters * sizeof(uint32_t)) + up(bytes);
-    // The last 256 bytes stay unused, so no piece ends at the region's very end.
-    if (x->fixed->cap < 256 || need > x->fixed->cap - 256) {
+    const size_t need = scratch_need(bytes, need_counter, n_counters);
+    if (!static_fits(x, bytes, need_counter, n_counters)) {
       set_error(err, UNP_INVALID_ARGUMENT,
                 "this launch needs " + std::to_string(need) + " bytes of workspace; the static scratch holds " +
                     std::to_string(x->fixed->cap) + " (" + std::to_string(x->fixed->cap - 256) + " usable)");
@@ -623,19 +676,17 @@ int32_t workspace(unp_exec* x, size_t bytes, bool need_counter, size_t n_counter
     }
     if (n_counters) {
       w.counters = reinterpret_cast<uint32_t*>(p);
-      p += up(n_counters * sizeof(uint32_t));
+      p += up256(n_counters * sizeof(uint32_t));
     }
     if (bytes) w.ws = p;
     // A kernel, not hipMemsetAsync: a call under graph capture then records no memset node.
     if (need) return unp::scratch_clear(x->fixed->base, need, s, err);
     return UNP_OK;
   }
-  int32_t rc = ensure_ws(x, bytes, need_counter, err);
-  if (rc == UNP_OK && n_counters) rc = ensure_counters(x, n_counters, err);
+  const int32_t rc = ensure_ws(x, bytes, need_counter, err);
   if (rc != UNP_OK) return rc;
   w.ws = x->ws;
   w.counter = x->counter;
-  w.counters = x->counters;
   return UNP_OK;
 }
 
@@ -659,30 +710,124 @@ int32_t next_epoch(unp_exec* x, hipStream_t s, uint32_t& ep, unp_error* err) {
 
 waits_host waits_of(const unp_exec* x) { return waits_host{x->stall, x->wait_ticks, 0}; }
 
-// The kept and the reduced axes of a row-major input with their element strides, outermost
-// first, adjacent axes of a kind merged (a merged run's stride is its innermost axis's).
-void fill_axes_desc(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask, unp::axes_desc_host& d) {
-  long long stride = 1;
-  std::vector<long long> str((size_t)rank);
-  for (int32_t k = rank - 1; k >= 0; --k) {
-    str[(size_t)k] = stride;
-    stride *= ext[(size_t)k];
-  }
-  for (int32_t k = 0; k < rank;) {
+// The axes of a row-major input for a split reduction: the innermost run of one kind as L, the kept
+// and the reduced axes before it with their element strides, outermost first.  Axes of extent 1 are
+// dropped and adjacent axes of a kind merged (a merged run's stride is its innermost axis's).
+void fill_red_axes(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask, unp::red_axes_host& d) {
+  const bool last = (mask >> (rank - 1)) & 1u;
+  d.L = d.outs = d.count = 1;
+  for (int32_t k = 0; k < rank; ++k) ((mask >> k) & 1u ? d.count : d.outs) *= ext[(size_t)k];
+  int32_t k = rank - 1;
+  for (; k >= 0 && (((mask >> k) & 1u) != 0) == last; --k) d.L *= ext[(size_t)k];
+  long long stride = d.L;
+  bool prev = last;  // the kind of the axis that ended the list's newest run
+  for (; k >= 0; --k) {
+    const long long e = ext[(size_t)k];
+    if (e == 1) continue;
     const bool red = (mask >> k) & 1u;
-    long long e_ = 1;
-    int32_t e = k;
-    while (e < rank && (((mask >> e) & 1u) != 0) == red) e_ *= ext[(size_t)e++];
-    const long long st = str[(size_t)(e - 1)];
-    if (red) {
-      d.rext[d.nr] = e_;
-      d.rstr[d.nr++] = st;
+    long long& n = red ? d.nr : d.nk;
+    long long* const xs = red ? d.rext : d.kext;
+    long long* const ss = red ? d.rstr : d.kstr;
+    if (n > 0 && red == prev) {
+      xs[n - 1] *= e;  // the run goes on outwards: its stride stays its innermost axis's
     } else {
-      d.kext[d.nk] = e_;
-      d.kstr[d.nk++] = st;
+      xs[n] = e;
+      ss[n++] = stride;
     }
-    k = e;
+    prev = red;
+    stride *= e;
   }
+  std::reverse(d.kext, d.kext + d.nk);
+  std::reverse(d.kstr, d.kstr + d.nk);
+  std::reverse(d.rext, d.rext + d.nr);
+  std::reverse(d.rstr, d.rstr + d.nr);
+  for (long long i = 0; i < d.nk; ++i) d.kinv[i] = 1.0 / (double)d.kext[i];
+  for (long long i = 0; i < d.nr; ++i) d.rinv[i] = 1.0 / (double)d.rext[i];
+  const long long total = last ? d.count : d.outs;
+  d.runs = d.L > 0 ? total / d.L : 0;
+}
+
+// What a split reduction's launch takes, in microseconds, up to a constant: `items` over `grid` blocks
+// of eight waves that stride over them, `loads` 16-byte loads of each lane per item, `folds` rounds
+// of loads of the partials in the closing fold (0: not split).  Blocks read `speed` times the 5
+// TB/s they reach together (8 KiB a load and block), or, where few run, the 27 GB/s one reaches, and
+// wait about 1.2 us for every eight loads; an item pays about 2 us for its start and its fold over
+// the block, a split launch 3.5 us for publishing, the ticket and the store.  Against measurement:
+// 6000 x 2050 f32 column norms 19.4 us at 28 chunks of 256 columns (here 17.9 + the launch), 30.0 at
+// 85; 12158 x 90 I32 column maxima 13.6 at 64 chunks, 15.1 at 256; the means of 256 channels of 25088
+// f32 each 9.5 (7.0 + the launch).
+double split_cost(long long items, long long grid, double loads, double speed, long long folds) {
+  const double together = 8192.0 / 5.0e6 * (double)std::min(items, grid) / speed;
+  const double item = std::max(1.2 * std::ceil(loads / 8.0), loads * std::max(0.3, together)) + 2.0;
+  return (double)((items + grid - 1) / grid) * item + (folds ? 3.5 + 1.3 * (double)folds : 0.0);
+}
+
+// The number of chunks (1 .. kMaxChunks, at most kSplitRounds whole rounds of items, at least
+// `least` loads each) with the least cost, for `units` outputs or strips of `loads` loads each of
+// which `slots` partials are folded in a round; `best` starts at the cost to beat.
+long long split_chunks(long long units, long long grid, double loads, double speed, long long slots, double& best) {
+  long long S = 1;
+  const auto take = [&](long long s) {
+    if (s < 1 || s > unp::kMaxChunks || (s > 1 && (units * s > (long long)kSplitRounds * grid || loads / (double)s < 1.0)))
+      return;
+    const double c = split_cost(units * s, grid, loads / (double)s, speed, s > 1 ? (s + slots - 1) / slots : 0);
+    if (c < best) {
+      best = c;
+      S = s;
+    }
+  };
+  take(1);
+  for (long long s = 2; s <= unp::kMaxChunks; s *= 2) take(s);
+  for (long long m = 1; m <= (long long)kSplitRounds; ++m) take(m * grid / units);
+  return S;
+}
+
+// The workspace of a split launch on stream s: the stream's own, bound on its first launch (the
+// one made with the executor first, then up to kMaxStreams).  None (null words) for a stream past
+// those, for the per-thread stream (one handle, a stream per thread), under capture (a replay
+// would carry one epoch for ever, and the graph the addresses) and in a no-allocation launch; the
+// kernel then folds all chunks of an output in one block, to the same bits.
+struct SplitWs {
+  void* partials = nullptr;
+  void* counters = nullptr;
+  uint32_t epoch = 0;
+};
+
+SplitWs stream_workspace(unp_exec* x, hipStream_t s) {
+  SplitWs w;
+  if (x->fixed || s == hipStreamPerThread) return w;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();  // the null stream while another stream captures: not an error of this launch
+    return w;
+  }
+  if (st != hipStreamCaptureStatusNone) return w;
+  StreamWs* own = nullptr;
+  for (StreamWs& c : x->stream_ws)
+    if (c.bound && c.stream == s) own = &c;
+  for (StreamWs& c : x->stream_ws)
+    if (!own && !c.bound) own = &c;
+  if (!own) {
+    if (x->stream_ws.size() >= kMaxStreams || add_stream_ws(x) != hipSuccess) {
+      (void)hipGetLastError();
+      return w;
+    }
+    own = &x->stream_ws.back();
+  }
+  own->bound = true;
+  own->stream = s;
+  if (own->epoch == 0xffffffffu) {
+    // The words start zeroed and no launch has epoch 0; clear them before the epoch wraps.
+    if (hipMemsetAsync(own->base, 0, split_bytes(x), s) != hipSuccess) {
+      (void)hipGetLastError();
+      return w;
+    }
+    own->epoch = 0;
+  }
+  w.epoch = ++own->epoch;
+  w.counters = own->base;
+  w.partials = own->base + split_counter_bytes(x);
+  return w;
 }
 
 // Appends axis (e, is, os) to a descriptor's list, merged into the previous axis when the two
@@ -725,24 +870,7 @@ void fill_red_view(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask,
 static_assert(sizeof(unp::red_view_host) == 44 * 8, "red_view_host mirrors the device's red_view");
 static_assert(sizeof(unp::scan_view_host) == 29 * 8, "scan_view_host mirrors the device's scan_view");
 static_assert(sizeof(unp::gather_view_host) == 35 * 8, "gather_view_host mirrors the device's gather_view");
-static_assert(sizeof(unp::axes_desc_host) == 36 * 8, "axes_desc_host mirrors the device's axes_desc");
-
-// At least n zeroed ticket counters.  Kernels leave every counter they use at zero, so a
-// larger array is allocated afresh (and zeroed) only when a launch needs more strips.
-int32_t ensure_counters(unp_exec* x, size_t n, unp_error* err) {
-  if (n <= x->n_counters) return UNP_OK;
-  if (x->counters) {
-    hipFree(x->counters);
-    x->counters = nullptr;
-    x->n_counters = 0;
-  }
-  hipError_t e = hipMalloc((void**)&x->counters, n * sizeof(uint32_t));
-  if (e != hipSuccess) return hip_fail(err, "hipMalloc(counters)", e);
-  e = hipMemset(x->counters, 0, n * sizeof(uint32_t));
-  if (e != hipSuccess) return hip_fail(err, "hipMemset(counters)", e);
-  x->n_counters = n;
-  return UNP_OK;
-}
+static_assert(sizeof(unp::red_axes_host) == 54 * 8, "red_axes_host mirrors the device's red_axes");
 
 int32_t launch(unp_exec* x, size_t entry, uint32_t grid, void** params, hipStream_t s, unp_error* err) {
   const uint32_t threads = (uint32_t)(x->l.entries[entry].threads ? x->l.entries[entry].threads : x->l.threads);
@@ -786,6 +914,84 @@ int64_t product(const std::vector<int64_t>& v, size_t from, size_t to) {
   int64_t p = 1;
   for (size_t i = from; i < to; ++i) p *= v[i];
   return p;
+}
+
+// A reduction with kept axes after a reduced one, or reduced ones around a kept one: `ptrs` the
+// inputs, then the output.
+int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint64_t> ptrs, hipStream_t s,
+                  unp_error* err) {
+  const unp_form& f = x->l.form;
+  const bool inner = inner_reduced(x->l);
+  unp::red_axes_host d{};
+  fill_red_axes(ext, f.rank, x->l.axes_mask, d);
+  const long long grid = (long long)x->cu_count * x->l.blocks_per_cu;
+  const long long vec = 16 / (long long)unp::kind_bytes(f.dtype);
+  const bool fast = d.L >= vec;
+  const long long v = fast ? vec : 1;
+  long long S = 1, units = d.outs;
+  bool team = false;
+  int lpr = 64;
+  double best = 1e300;
+  if (inner) {
+    // A block per (chunk of an) output, or a wave per output.
+    const double loads = (double)(d.runs * ((d.L + v - 1) / v)) / 64.0;
+    S = split_chunks(units, grid, loads / 8.0, 1.0, 64, best);
+    const long long waves = 8 * grid, busy = std::min(units, waves);
+    team = (double)((units + waves - 1) / waves) *
+               std::max(1.2 * std::ceil(loads / 8.0), (double)busy * loads * 1024.0 / 5.0e6) + 2.0 < best;
+    if (team) S = 1;
+  } else {
+    // Strips of 64 lanes' columns, or of 32 or 16 where that gives more blocks without splitting rows:
+    // narrower ones read slower (28.9, 31.5, 33.8 us for 2000 x 16001 f32 column norms at 64, 32 and
+    // 16 lanes; 53.6 at 8).
+    const long long whole = std::min(64LL, (d.L + v - 1) / v);
+    const struct { long long lanes; double speed; } widths[] = {{64, 1.0}, {32, 0.9}, {16, 0.8}};
+    for (const auto& w : widths) {
+      const long long lanes = std::min(w.lanes, whole);
+      if (w.lanes < 64 && w.lanes >= whole) continue;
+      const long long n = d.runs * ((d.L + lanes * v - 1) / (lanes * v)), rpi = 64 / lanes;
+      const double before = best;
+      const long long s = split_chunks(n, grid, (double)d.count / (double)(8 * rpi), w.speed, 4 * 8 * rpi, best);
+      if (best < before) {
+        S = s;
+        units = n;
+        lpr = (int)lanes;
+      }
+    }
+  }
+  size_t entry = 0;
+  while (x->l.entries[entry].strided || x->l.entries[entry].fast != fast || x->l.entries[entry].team != team) ++entry;
+  SplitWs w;
+  if (S > 1) {
+    if (units * S > (long long)split_items(x)) {
+      set_error(err, UNP_INVALID_ARGUMENT, "a split reduction beyond its workspace");
+      return UNP_INVALID_ARGUMENT;
+    }
+    const size_t bytes = (size_t)(units * S * (inner ? 1 : 64 * v)) * 16;
+    if (!x->fixed) {
+      w = stream_workspace(x, s);
+    } else if (f.kind == UNP_FORM_REDUCTION && x->l.red_schedule == 'm' && x->l.rx.plain &&
+               static_fits(x, bytes, false, (size_t)units)) {
+      // The plain column reduction takes the static scratch; the others never shared it.
+      Ws own;
+      const int32_t rc = workspace(x, bytes, false, (size_t)units, s, own, err);
+      if (rc != UNP_OK) return rc;
+      w.partials = own.ws;
+      w.counters = own.counters;
+      w.epoch = 1;
+    }
+  }
+  waits_host wt = waits_of(x);
+  std::vector<void*> params;
+  for (uint64_t& p : ptrs) params.push_back(&p);
+  params.push_back(&d);
+  params.push_back(&S);
+  if (!inner) params.push_back(&lpr);
+  params.push_back(&w.partials);
+  params.push_back(&w.counters);
+  params.push_back(&w.epoch);
+  params.push_back(&wt);
+  return launch(x, entry, (uint32_t)grid, params.data(), s, err);
 }
 
 // A reduction with a pre-map body over NI inputs or a fused post: NI input buffers of the same
@@ -833,13 +1039,7 @@ int32_t run_xreduction(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, u
     params.push_back(&wt);
     return launch(x, aligned ? 0 : 1, grid, params.data(), s, err);
   }
-  unp::axes_desc_host d{};
-  fill_axes_desc(A.ext, f.rank, mask, d);
-  d.outs = outs;
-  d.count = count;
-  params.push_back(&d);
-  const long long cap = (long long)x->cu_count * x->l.blocks_per_cu;
-  return launch(x, 0, (uint32_t)cap, params.data(), s, err);
+  return run_split(x, A.ext, ptrs, s, err);
 }
 
 int32_t run_reduction(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_error* err) {
@@ -859,68 +1059,23 @@ int32_t run_reduction(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, un
     for (int32_t d = 0; d < f.rank; ++d) ((mask >> d) & 1u ? count : outs) *= A.ext[(size_t)d];
     if ((rc = need_buffers(A, outs > 0, err)) != UNP_OK) return rc;
     if (outs == 0) return UNP_OK;
+    if (sched != 'q') return run_split(x, A.ext, A.buf, s, err);
     uint64_t in = A.buf[0], out = A.buf[1];
-    if (sched == 'm') {
-      // A x R x B: the kept axes before the reduced run, the run, the kept axes after it.
-      int32_t fr = 0, lr = f.rank - 1;
-      while (!((mask >> fr) & 1u)) ++fr;
-      while (!((mask >> lr) & 1u)) --lr;
-      long long a = product(A.ext, 0, (size_t)fr), r = product(A.ext, (size_t)fr, (size_t)lr + 1),
-                b = product(A.ext, (size_t)lr + 1, (size_t)f.rank);
-      const size_t entry = (b % vec == 0 && aligned16(in)) ? 0 : 1;
-      const long long cw = 64LL * x->l.entries[entry].vec;
-      const long long strips = a * ((b + cw - 1) / cw);
-      // The grid is the device-class constant (cu_count * blocks_per_cu); the work is strips x S
-      // items, S chunks of R: about one item per block, at least 16 rows per chunk, at most 1024
-      // chunks.  Blocks stride over the items.
-      const long long grid = (long long)x->cu_count * x->l.blocks_per_cu;
-      long long S = (grid + strips - 1) / strips;
-      S = std::min(S, std::max(1LL, r / 16));
-      S = std::max(1LL, std::min(S, 1024LL));
-      // A partial is one 8-byte tagged word per 4 bytes of accumulator.
-      const size_t acc_bytes = (unp::kind_is_float(f.dtype) && (f.op0 == UNP_OP_SUM || f.op0 == UNP_OP_MEAN))
-                                   ? 8
-                                   : unp::kind_bytes(f.dtype);
-      const size_t word_bytes = acc_bytes == 8 ? 16 : 8;
-      void* ws = nullptr;
-      void* cnt = nullptr;
-      uint32_t ep = 0;
-      if (S > 1) {
-        Ws w;
-        if ((rc = workspace(x, (size_t)(strips * S * cw) * word_bytes, false, (size_t)strips, s, w, err)) != UNP_OK)
-          return rc;
-        if ((rc = next_epoch(x, s, ep, err)) != UNP_OK) return rc;
-        ws = w.ws;
-        cnt = w.counters;
-      }
-      waits_host wt = waits_of(x);
-      void* params[] = {&in, &out, &a, &r, &b, &S, &ws, &cnt, &ep, &wt};
-      return launch(x, entry, (uint32_t)grid, params, s, err);
-    }
     const long long cap = (long long)x->cu_count * x->l.blocks_per_cu;
-    if (sched == 'q') {
-      // The serial product (a lane per output) takes the storage-image descriptor, here with the
-      // row-major strides of the input and of the kept-axes output.
-      std::vector<long long> in_str((size_t)f.rank), out_str((size_t)f.rank, 0);
-      long long si = 1, so = 1;
-      for (int32_t k = f.rank - 1; k >= 0; --k) {
-        in_str[(size_t)k] = si;
-        si *= A.ext[(size_t)k];
-        if (!((mask >> k) & 1u)) {
-          out_str[(size_t)k] = so;
-          so *= A.ext[(size_t)k];
-        }
+    // The serial product (a lane per output) takes the storage-image descriptor, here with the
+    // row-major strides of the input and of the kept-axes output.
+    std::vector<long long> in_str((size_t)f.rank), out_str((size_t)f.rank, 0);
+    long long si = 1, so = 1;
+    for (int32_t k = f.rank - 1; k >= 0; --k) {
+      in_str[(size_t)k] = si;
+      si *= A.ext[(size_t)k];
+      if (!((mask >> k) & 1u)) {
+        out_str[(size_t)k] = so;
+        so *= A.ext[(size_t)k];
       }
-      unp::red_view_host d{};
-      fill_red_view(A.ext, f.rank, mask, in_str.data(), out_str.data(), d);
-      d.outs = outs;
-      d.count = count;
-      void* params[] = {&in, &out, &d};
-      return launch(x, 0, (uint32_t)cap, params, s, err);
     }
-    // Any other mask: a wave per output.
-    unp::axes_desc_host d{};
-    fill_axes_desc(A.ext, f.rank, mask, d);
+    unp::red_view_host d{};
+    fill_red_view(A.ext, f.rank, mask, in_str.data(), out_str.data(), d);
     d.outs = outs;
     d.count = count;
     void* params[] = {&in, &out, &d};

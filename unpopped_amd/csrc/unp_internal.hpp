@@ -30,6 +30,7 @@ struct Entry {
   bool wide = false;  // reduction: the block-per-row schedule (long rows)
   int threads = 0;    // block size of this entry (0: the form's)
   int blocks_per_cu = 0;  // persistent blocks per CU of this entry (0: the form's)
+  bool team = false;      // split reduction, innermost run reduced: a wave per output
   int cols = 0;           // output columns per block (dequant GEMM decode entries)
   // Reads and writes its buffers through storage-image strides (unp_hip_exec_launch_views with a
   // view that is not dense row-major); never picked for a pointer launch.
@@ -48,13 +49,18 @@ constexpr long long kWideRow = 32768;
 uint32_t reduction_mask(const unp_form& f);
 char reduction_schedule(uint32_t mask, int32_t rank);
 
-// The host image of the device's axes_desc (reduce_generic's argument, passed by value).
-struct axes_desc_host {
+// The host image of the device's red_axes (the split reductions' argument, passed by value).
+struct red_axes_host {
   long long nk, nr;
   long long kext[8], kstr[8];
   long long rext[8], rstr[8];
+  double kinv[8], rinv[8];
+  long long L, runs;
   long long outs, count;
 };
+
+// The most chunks a split reduction cuts one output's (or column strip's) positions into.
+constexpr long long kMaxChunks = 256;
 
 // Host images of the storage-image descriptors (red_view, scan_view, gather_view; passed by
 // value): extents and signed element strides of the views, axes outermost first.
