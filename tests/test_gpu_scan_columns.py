@@ -1,0 +1,47 @@
+"""Scans along an axis with kept axes after it, whose rows stream through LDS tiles: strips of 64 columns
+and their ragged last groups, tiles' last rows, several strips per block, unaligned buffers, in place."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+import unpopped_amd as u
+from unpopped_amd import forms as H, synth
+
+pytestmark = pytest.mark.gpu
+NT = {"F32": np.float32, "F64": np.float64, "I32": np.int32, "I64": np.int64}
+
+
+def values(dtype, n):
+    return synth.normal_f32(5, n).astype(NT[dtype]) if dtype[0] == "F" else synth.int16_i32(5, n).astype(NT[dtype])
+
+
+@pytest.mark.parametrize("a,s,b", [(1, 16, 32), (3, 33, 63), (2, 64, 64), (1, 65, 65), (2, 129, 130), (1, 600, 67),
+                                   (5, 700, 256), (300, 20, 33), (7, 40, 8001), (1, 15, 64), (2, 50, 31)])
+@pytest.mark.parametrize("dtype,op,exclusive,reverse", [("F32", "Sum", False, False), ("F32", "Sum", True, True),
+                                                        ("F32", "Mean", False, True), ("F32", "Max", True, False),
+                                                        ("F64", "Sum", False, True), ("I32", "Sum", True, False),
+                                                        ("I64", "Min", False, False)])
+def test_every_prefix_is_the_serial_ones(hip_device, a, s, b, dtype, op, exclusive, reverse):
+    """Bit-exact against the serial scan, at aligned and unaligned addresses and in place."""
+    if op == "Mean" and dtype[0] == "I":
+        pytest.skip("an integer Mean")
+    x = values(dtype, a * s * b).reshape(a, s, b)
+    rows = np.ascontiguousarray(np.moveaxis(x, 1, -1)).reshape(-1, s)
+    want = np.ascontiguousarray(np.moveaxis(oracle.scan_rows(rows, op, exclusive, reverse).reshape(a, b, s), -1, 1))
+    ex = H.executor(kind="scan", dtype=dtype, rank=3, op=op, axis=1, exclusive=exclusive, reverse=reverse)
+    H.say(f"[case] column scan {a}x{s}x{b} {dtype} {op} exclusive={exclusive} reverse={reverse}")
+    for shift in (0, x.itemsize):
+        buf = u.DeviceBuffer(x.nbytes + 64)
+        dst = u.DeviceBuffer(x.nbytes + 64)
+        dst.fill(0x5A)
+        buf.at(shift).upload(x)
+        ex.launch(buf.at(shift), dst.at(shift), a, s, b)
+        u.synchronize()
+        assert np.array_equal(dst.at(shift).download(NT[dtype], x.size).reshape(x.shape), want, equal_nan=True)
+        edge = dst.at(shift + x.nbytes).download(np.uint8, 64 - shift)
+        assert (edge == 0x5A).all()
+        ex.launch(buf.at(shift), buf.at(shift), a, s, b)
+        u.synchronize()
+        assert np.array_equal(buf.at(shift).download(NT[dtype], x.size).reshape(x.shape), want, equal_nan=True)

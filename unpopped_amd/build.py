@@ -100,6 +100,7 @@ extern "C" __global__ void __launch_bounds__(512) c_ro(const float* a, float* b,
 extern "C" __global__ void KB c_rq(const float* a, float* b, unp::red_view d) { unp::reduce_serial<float, unp::OP_MAXNUM, 256>(a, b, d); }
 extern "C" __global__ void KB c_rq2(const long long* a, long long* b, unp::red_view d) { unp::reduce_serial<long long, unp::OP_XOR, 256>(a, b, d); }
 extern "C" __global__ void KB c_rv(const float* a, float* b, unp::red_view d) { unp::reduce_strided<float, unp::OP_SUM, 256>(a, b, d); }
+extern "C" __global__ void __launch_bounds__(576) c_sc(const double* a, double* b, long long S, long long B, long long n, long long c, int wide) { __shared__ __attribute__((aligned(16))) unsigned char ring[9 * 16384]; if (wide) unp::scan_cols<double, unp::OP_MEAN, true, true, true, 8>(a, b, S, B, n, c, ring); else unp::scan_cols<double, unp::OP_MEAN, true, true, false, 8>(a, b, S, B, n, c, ring); }
 extern "C" __global__ void KB c_sv(const double* a, double* b, unp::scan_view v) { unp::scan_strided<double, unp::OP_MEAN, true, true>(a, b, v); }
 extern "C" __global__ void KB c_gv(const unsigned short* t, const long long* i, unsigned short* o, unp::gather_view v, long long x) { unp::gather_strided<unsigned short, long long, unp::OOB_ZEROFILL>(t, i, o, v, x); }
 extern "C" __global__ void KB c_si(const int* a, int* b, long long r, long long c, unsigned long long* s, unsigned* k, unsigned t, unsigned e, unp::waits w) { unp::scan_lookback<int, unp::OP_SUM, true, true, 4, 16, 4, 32>(a, b, r, c, s, k, t, e, w); }

@@ -488,21 +488,36 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
        << (f.reverse ? "rev_" : "") << op_name(f.op0) << "_" << lower_name(f.dtype);
   L.name = name.str();
   if (serial) {
+    // _q: a lane per column, 8 loads each in flight.
+    // _c: rows of at least 32 columns, streamed through LDS by eight mover waves around one that scans.
     Entry e;
     e.fast = false;
     e.vec = 1;
-    e.threads = 256;
-    e.blocks_per_cu = 8;
+    e.threads = 1024;
+    e.blocks_per_cu = 1;
     e.symbol = L.name + "_q";
+    Entry c = e;
+    c.fast = true;
+    c.threads = 64 * 9;
+    c.symbol = L.name + "_c";
+    const std::string how = std::string(f.exclusive ? "true" : "false") + ", " + (f.reverse ? "true" : "false");
     std::ostringstream src;
     src << header(L.name, f);
-    src << "extern \"C\" __global__ void __launch_bounds__(256) " << e.symbol << "(const " << T << "* in, " << T
+    src << "extern \"C\" __global__ void __launch_bounds__(1024) " << e.symbol << "(const " << T << "* in, " << T
         << "* out, long long A, long long S, long long B) {\n  unp::scan_seq<" << T << ", " << f.op0 << ", "
-        << (f.exclusive ? "true" : "false") << ", " << (f.reverse ? "true" : "false") << ", 8>(in, out, A, S, B);\n}\n";
+        << how << ", 8>(in, out, A, S, B);\n}\n";
+    src << "extern \"C\" __global__ void __launch_bounds__(" << c.threads << ") " << c.symbol << "(const " << T << "* in, "
+        << T << "* out, long long S, long long B, long long nstrips, long long ncb, int wide) {\n"
+        << "  __shared__ __attribute__((aligned(16))) unsigned char ring[9 * 16384];\n";
+    for (int wide = 1; wide >= 0; --wide)
+      src << (wide ? "  if (wide) " : "  else ") << "unp::scan_cols<" << T << ", " << f.op0 << ", " << how << ", "
+          << (wide ? "true" : "false") << ", 8>(in, out, S, B, nstrips, ncb, ring);\n";
+    src << "}\n";
     L.entries.push_back(e);
+    L.entries.push_back(c);
     src << scan_strided_entry(f, L);
-    L.threads = 256;
-    L.blocks_per_cu = 8;
+    L.threads = e.threads;
+    L.blocks_per_cu = e.blocks_per_cu;
     L.source = src.str();
     std::ostringstream j;
     j << "{\"backend\":\"hip\",\"target\":\"rocm:gfx950\",\"form\":\"scan\",\"dtype\":\"" << kind_name(f.dtype)
@@ -511,9 +526,11 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
       << ",\"schedule\":\"serial\",\"params\":[{\"name\":\"in0\",\"kind\":\"buffer\",\"role\":\"Read\"},"
       << "{\"name\":\"out\",\"kind\":\"buffer\",\"role\":\"Write\"}";
     for (int d = 0; d < f.rank; ++d) j << ",{\"name\":\"n" << d << "\",\"kind\":\"scalar\",\"dtype\":\"I32\"}";
-    j << "],\"launch\":{\"block\":[256,1,1],\"grid\":\"cu_count*8\",\"grid_policy\":\"device-class constant; one "
-      << "lane per column of the input seen as A x S x B around the scanned axis, lanes stride over columns\"},"
-      << "\"entries\":[{\"symbol\":\"" << e.symbol << "\",\"when\":\"always\"},{\"symbol\":\""
+    j << "],\"launch\":{\"block\":[1024,1,1],\"grid\":\"cu_count*1\",\"grid_policy\":\"device-class constant; one "
+      << "lane per column of the input seen as A x S x B around the scanned axis, lanes or blocks of 64 columns stride "
+      << "over the columns\"},\"entries\":[{\"symbol\":\"" << c.symbol
+      << "\",\"block\":576,\"when\":\"B >= 32, S >= 16 and at most 4 strips of 64 columns per CU\"},{\"symbol\":\"" << e.symbol
+      << "\",\"when\":\"otherwise\"},{\"symbol\":\""
       << L.entries.back().symbol << "\",\"when\":\"" << kStridedWhen << "\"}],\"workspace\":null"
       << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
       << ",\"fidelity_notes\":[" << json_str("the serial lift's own order: each column's prefix folds ascending (descending "

@@ -218,6 +218,10 @@ template <class T, int N> UNP_DEV vec<T, N> ld_any(const T* p) {
     return ld_nt<T, N>(p);
   }
 }
+template <class T, int N> UNP_DEV void st_any(T* p, const vec<T, N>& v) {
+  static_assert(sizeof(T) * N == 16, "16-byte vectors");
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_any*>(p));
+}
 template <class T, int N> UNP_DEV void st_nt(T* p, const vec<T, N>& v) {
   if constexpr (sizeof(T) * N == 16) {
     __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(p));
@@ -1238,8 +1242,10 @@ UNP_DEV void scan_seq(const T* __restrict__ in, T* __restrict__ out, i64 A, i64 
   typedef typename serial_acc<T>::type Ac;
   typedef fold<Ac, OP> F;
   const i64 cols = A * B;
+  // Groups of 256 columns go round the blocks first, so that a few hundred of them still reach every
+  // CU and a group's rows are read in whole kilobytes.
   const i64 stride = (i64)gridDim.x * blockDim.x;
-  for (i64 c = (i64)blockIdx.x * blockDim.x + threadIdx.x; c < cols; c += stride) {
+  for (i64 c = ((i64)(threadIdx.x >> 8) * gridDim.x + blockIdx.x) * 256 + (threadIdx.x & 255); c < cols; c += stride) {
     const i64 a = c / B, b = c - a * B;
     const i64 base = a * S * B + b;
     Ac v = F::identity();
@@ -1271,6 +1277,234 @@ UNP_DEV void scan_seq(const T* __restrict__ in, T* __restrict__ out, i64 A, i64 
         out[off] = scan_out<T, OP>(v, i + 1);
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The same scan of A x S x B in the same order, for rows of at least 32 columns: a strip of 64
+// columns per block, its rows streamed through a ring of LDS tiles.  The serial order leaves a
+// column one chain of S folds, so one wave (lanes on columns) runs nothing but that chain, out of
+// LDS, while NM mover waves keep the rows coming and going: a lane that loads its own rows waits
+// for memory once per group of loads instead.  2048 x 3000 f32: 34.5 us, 111.6 with scan_seq; 4096 x
+// 8192: 66 us (4.0 TB/s), 355.  What bounds a few strips is the chain: a conversion, an add and a
+// conversion in f64 per row, 11 to 12 ns.  From about four strips per CU on a lane per column keeps
+// as much in flight (16 x 300 x 5000: 55 us here, 53 there; 32 x 100 x 8001: 74, 51).
+//
+// Tiles of 16 KiB (64 rows of 4-byte elements) follow each other through NB buffers, across the
+// block's strips (strip = blockIdx.x, += gridDim.x) without a break.  Round r:
+//   movers  issue the global->LDS DMA of tile r + D, store tile r - 1, and wait until tile r + 1 has
+//           landed (every tile issues the same operations, clamped to its last row, so the wait is
+//           an exact count that leaves the younger tiles in flight);
+//   scanner folds tile r in place;
+//   barrier (LDS only: nothing waits for global stores).
+// A tile's buffer is written again NB rounds later, D = NB - 2: after its stores have read it.
+// Seven tiles ahead are 112 KiB in flight per CU.
+//
+// A row's 64 slots are 16-byte groups of columns; a strip's last group starts at B - VEC, so that
+// every group is whole, and scans the columns it shares with the one before it a second time, to
+// the same values.  `wide`: B % VEC == 0 and `in` 16-byte aligned, the rows move by 16-byte DMA;
+// otherwise by 4-byte DMA (one row of 4-byte slots per operation).  Stores are 16 bytes at any
+// element alignment.
+// ---------------------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void lds_void;
+
+// Wait until at most N vector memory operations of this wave are outstanding (gfx9
+// s_waitcnt encoding: vmcnt bits 3:0 and 15:14; expcnt and lgkmcnt left at their maximum).
+template <int N> UNP_DEV void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt is six bits");
+  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | 0x0F70);
+}
+
+// fn(ic<0>{}), fn(ic<1>{}), ..., fn(ic<N - 1>{}): a loop whose index is a constant expression
+// in the body (for immediates such as a wait count).
+template <int N, int I = 0, class Fn> UNP_DEV void unroll_for(Fn&& fn) {
+  if constexpr (I < N) {
+    fn(ic<I>{});
+    unroll_for<N, I + 1>(fn);
+  }
+}
+
+template <class T, int OP, bool EXCL, bool REV, bool WIDE, int NM>
+UNP_DEV void scan_cols(const T* __restrict__ in, T* __restrict__ out, i64 S, i64 B, i64 nstrips, i64 ncb, u8* ring) {
+  typedef typename serial_acc<T>::type Ac;
+  typedef fold<Ac, OP> F;
+  constexpr int VEC = 16 / sizeof(T), RB = 64 * (int)sizeof(T), TILE = 16384, TR = TILE / RB, NB = 9, D = NB - 2;
+  constexpr int GPR = RB / 16;                         // 16-byte groups per row
+  constexpr int LB = WIDE ? 16 : 4;                    // bytes a lane moves per DMA operation
+  constexpr int DMA = TILE / (64 * LB) / NM, ST = TILE / 1024 / NM;  // operations per mover wave and tile
+  static_assert((D - 1) * DMA + D * ST < 64, "the wait counts fit vmcnt");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const i64 nt = (S + TR - 1) / TR;
+  const i64 mine = nstrips > blockIdx.x ? (nstrips - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;
+  const i64 N = mine * nt;  // this block's tiles
+  if (N == 0) return;
+  struct Cursor {  // a tile: its strip, its number in the strip and its buffer
+    i64 strip, t;
+    int b;
+  };
+  auto next = [&](Cursor& c) {
+    if (++c.t == nt) {
+      c.t = 0;
+      c.strip += gridDim.x;
+    }
+    c.b = c.b + 1 == NB ? 0 : c.b + 1;
+  };
+  const Cursor first = {(i64)blockIdx.x, 0, 0};
+
+  if (wave < NM) {
+    const divisor by_ncb(ncb);
+    // The element offset of scan row `row` of a strip at this lane's 16-byte group g, and whether the
+    // group is the strip's (the offset of one that is not is that of its last).
+    auto offset = [&](i64 strip, i64 row, int g, bool& live) {
+      i64 a, cb;
+      by_ncb(strip, a, cb);
+      const i64 c = cb * 64 + g * VEC;
+      live = c < B;
+      return a * S * B + (REV ? S - 1 - row : row) * B + (c + VEC <= B ? c : B - VEC);
+    };
+    // Each lane keeps the address of its rows in the tile at hand: worked out at a strip's start and
+    // in its last tile (whose rows are clamped), else a tile's stride further.  With the addresses
+    // worked out for every tile the movers, not the chain, set the round: 1.28 us instead of 0.8.
+    const i64 stride = (REV ? -(i64)TR : (i64)TR) * B;
+    i64 lo[DMA], so[ST];
+    bool llive = false, slive = false;
+    auto issue = [&](const Cursor& c) {
+      if (c.t == 0 || c.t == nt - 1) {
+#pragma unroll
+        for (int k = 0; k < DMA; ++k) {
+          const int at = ((wave + NM * k) * 64 + lane) * LB;  // this lane's byte of the tile
+          const i64 i = c.t * TR + at / RB;
+          lo[k] = offset(c.strip, i < S ? i : S - 1, at / 16 % GPR, llive);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < DMA; ++k) {
+        const int o = wave + NM * k;  // operation o fills LDS bytes o * 64 * LB ..
+        const T* p = in + lo[k];
+        lds_void* const to = (lds_void*)(ring + c.b * TILE + o * 64 * LB);
+        // Groups past the row (their column is clamped too) are skipped only where an operation also
+        // covers the first group: one without a live lane would not be issued, and the count be off.
+        if constexpr (WIDE) {
+          if (llive) __builtin_amdgcn_global_load_lds(p, to, 16, 0, 2 /* nt */);
+        } else {
+          __builtin_amdgcn_global_load_lds(reinterpret_cast<const u8*>(p) + lane * LB % 16, to, 4, 0, 2);
+        }
+        lo[k] += stride;
+      }
+    };
+    auto store = [&](const Cursor& c) {
+      const int g = lane % GPR;
+      int r[ST];  // this lane's rows of the tile
+#pragma unroll
+      for (int k = 0; k < ST; ++k) r[k] = (wave + NM * k) * (1024 / RB) + lane / GPR;
+      if (c.t == 0 || c.t == nt - 1) {
+        const int rows = S - c.t * TR < TR ? (int)(S - c.t * TR) : TR;
+#pragma unroll
+        for (int k = 0; k < ST; ++k) {
+          r[k] = r[k] < rows ? r[k] : rows - 1;
+          so[k] = offset(c.strip, c.t * TR + r[k], g, slive);
+        }
+      }
+      // Inline: for an ordinary LDS read the compiler would wait for every DMA of this wave.
+      const u32 lds = (u32)(size_t)(lds_void*)(ring + c.b * TILE) + (u32)(g * 16);
+      u32x4_t v[ST];
+      static_assert(ST == 2, "two reads under one wait");
+      asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(v[0]), "=&v"(v[1])
+                   : "v"(lds + (u32)(r[0] * RB)), "v"(lds + (u32)(r[1] * RB))
+                   : "memory");
+#pragma unroll
+      for (int k = 0; k < ST; ++k) {
+        if (slive) st_any<T, VEC>(out + so[k], __builtin_bit_cast(vec<T, VEC>, v[k]));
+        so[k] += stride;
+      }
+    };
+    // Tile r + 1 has landed once at most this many operations are outstanding: the DMA of the `rem`
+    // younger tiles, and D rounds' stores (in the first D rounds some, counted as none).
+    auto wait_tile = [&](i64 rem, bool stores) {
+      unroll_for<D>([&](auto n) {
+        constexpr int M = decltype(n)::value;
+        if (rem == M || (M == D - 1 && rem > M)) {
+          if (stores) wait_vm<M * DMA + D * ST>();
+          else wait_vm<M * DMA>();
+        }
+      });
+    };
+    Cursor ld = first, st = first;
+    for (i64 r = 0; r < D && r < N; ++r) {
+      issue(ld);
+      next(ld);
+    }
+    wait_tile(N - 1, false);
+    asm volatile("s_barrier" ::: "memory");
+    // Rolled: the compiler would peel the first D rounds, each then fetched cold.
+#pragma unroll 1
+    for (i64 r = 0; r <= N; ++r) {
+      int full = (int)(r >= D);
+      asm volatile("" : "+v"(full));
+      full = __builtin_amdgcn_readfirstlane(full);
+      if (r + D < N) {
+        issue(ld);
+        next(ld);
+      }
+      if (r > 0) {
+        store(st);
+        next(st);
+      }
+      if (r == N) break;
+      if (r + 1 < N) wait_tile(N - 2 - r, full != 0);
+      asm volatile("s_barrier" ::: "memory");
+    }
+    return;
+  }
+
+  // ---- the scanner ----
+  __builtin_amdgcn_s_setprio(3);
+  constexpr int Q = 16, NQ = TR / Q;  // rows per batch, batches per tile
+  Cursor c = first;
+  Ac v = F::identity();
+  asm volatile("s_barrier" ::: "memory");
+  for (i64 r = 0; r < N; ++r) {
+    if (c.t == 0) v = F::identity();
+    T* const tile = reinterpret_cast<T*>(ring + c.b * TILE) + lane;
+    const i64 i0 = c.t * TR;
+    auto fold_row = [&](int at, T raw) {
+      const i64 i = i0 + at;
+      const Ac e = (Ac)raw;
+      if constexpr (EXCL) {
+        tile[at * 64] = scan_out<T, OP>(v, i);
+        v = F::apply(v, e);
+      } else {
+        v = F::apply(v, e);
+        tile[at * 64] = scan_out<T, OP>(v, i + 1);
+      }
+    };
+    if (i0 + TR <= S) {
+      // A batch's rows are read while the one before it is folded.
+      T x[2][Q];
+#pragma unroll
+      for (int u = 0; u < Q; ++u) x[0][u] = tile[u * 64];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        if (q + 1 < NQ) {
+#pragma unroll
+          for (int u = 0; u < Q; ++u) x[(q + 1) & 1][u] = tile[((q + 1) * Q + u) * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < Q; ++u) fold_row(q * Q + u, x[q & 1][u]);
+      }
+    } else {
+      // Whole groups of 8 rows: those past the end are folded too and never stored.
+      for (int at = 0; i0 + at < S; at += 8) {
+        T x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = tile[(at + u) * 64];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) fold_row(at + u, x[u]);
+      }
+    }
+    next(c);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
 }
 
@@ -1871,24 +2105,7 @@ UNP_DEV void xscan_lookback(const T* const* __restrict__ in, T* __restrict__ out
 // differently from the within-stripe prefixes; every output is still one f64 fold of exactly
 // its prefix, held to the declared bound.
 // ---------------------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void;
-
-// Wait until at most N vector memory operations of this wave are outstanding (gfx9
-// s_waitcnt encoding: vmcnt bits 3:0 and 15:14; expcnt and lgkmcnt left at their maximum).
-template <int N> UNP_DEV void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt is six bits");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | 0x0F70);
-}
 UNP_DEV void wait_vm_all() { wait_vm<0>(); }
-
-// fn(ic<0>{}), fn(ic<1>{}), ..., fn(ic<N - 1>{}): a loop whose index is a constant expression
-// in the body (for immediates such as a wait count).
-template <int N, int I = 0, class Fn> UNP_DEV void unroll_for(Fn&& fn) {
-  if constexpr (I < N) {
-    fn(ic<I>{});
-    unroll_for<N, I + 1>(fn);
-  }
-}
 
 // A block barrier that orders LDS only: no wait on outstanding global stores.  A wave with
 // global->LDS DMA in flight must wait for it first (the DMA counts as LDS writes).

@@ -1174,8 +1174,18 @@ int32_t run_scan(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_err
     if ((rc = need_buffers(A, a0 > 0 && S > 0 && b0 > 0, err)) != UNP_OK) return rc;
     if (a0 == 0 || S == 0 || b0 == 0) return UNP_OK;
     uint64_t in = A.buf[0], out = A.buf[1];
+    const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
+    // Up to four strips of 64 columns per CU stream through LDS (rows of at least half a strip); more
+    // columns than that keep enough loads in flight with a lane each.
+    const long long ncb = (b0 + 63) / 64, strips = a0 * ncb;
+    if (b0 >= 32 && S >= 16 && strips <= 4LL * x->cu_count) {
+      int32_t wide = b0 % (16 / (long long)unp::kind_bytes(f.dtype)) == 0 && aligned16(in);
+      long long n = strips, c = ncb;
+      void* params[] = {&in, &out, &S, &b0, &n, &c, &wide};
+      return launch(x, 1, grid, params, s, err);
+    }
     void* params[] = {&in, &out, &a0, &S, &b0};
-    return launch(x, 0, (uint32_t)(x->cu_count * x->l.blocks_per_cu), params, s, err);
+    return launch(x, 0, grid, params, s, err);
   }
   long long rows = product(A.ext, 0, (size_t)f.rank - 1);
   long long cols = A.ext[(size_t)f.rank - 1];
