@@ -89,6 +89,7 @@ static_assert(sizeof(unp::red_axes) == 54 * 8, "red_axes");
 static_assert(sizeof(unp::red_view) == 44 * 8, "red_view");
 static_assert(sizeof(unp::scan_view) == 29 * 8, "scan_view");
 static_assert(sizeof(unp::gather_view) == 35 * 8, "gather_view");
+static_assert(sizeof(unp::ew_tile_view) == 114 * 8, "ew_tile_view");
 extern "C" __global__ void KB c_rr(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce<float, unp::OP_SUM, unp::OP_MAX, 2, 4, 256, 4>(a, b, c, r, n); }
 extern "C" __global__ void KB c_rw(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce_wave<float, unp::OP_SUM, unp::OP_MAX, 2, 4, 256, 8>(a, b, c, r, n); }
 extern "C" __global__ void KB c_rri(const long long* a, long long* b, long long* c, long long r, long long n) { unp::rowreduce<long long, unp::OP_PROD, unp::OP_MIN, 2, 1, 256, 8>(a, b, c, r, n); }

@@ -1609,6 +1609,50 @@ int32_t lower_elementwise(const unp_form& f, const ElementwiseExpr& ew, Lowered&
       << "    const ew_t a[" << N << "] = " << loads("static_cast<const ew_t*>(in#)[off[#]]") << ";\n"
       << "    static_cast<ew_t*>(out)[oo] = ew_cell(a);\n"
       << "  }\n}\n";
+  // The tiled entry: 64 x TJ elements of (D0, J) per 256-thread block, U of each input per lane in flight.
+  // Bound by the reads and the writes: out[i][j] = a[i][j] + b[j][i] over 4096 x 3000 f32 (147 MB) takes
+  // 30 us, 36 with cached stores (whose lines are written back under the next launch's reads) and 139
+  // in the strided entry, whose lanes divide out every element's coordinates and read b down its
+  // columns.  A lane holds at most about 32 registers of inputs (half of them: 38 us).
+  const int words = n * (int)std::max<size_t>(1, eb / 4);
+  const int U = words <= 2 ? 16 : words <= 4 ? 8 : words <= 8 ? 4 : 2, TJ = 4 * U;
+  const std::string TE = L.name + "_t_e";
+  src << "extern \"C\" __global__ void " << kLaunchBounds << " " << TE << "(" << params() << ", unp::ew_tile_view v) {\n"
+      << "  constexpr int TJ = " << TJ << ", U = " << U << ";\n"
+      << "  __shared__ ew_t turn[64 * (TJ + 1)];\n"
+      << "  const int dd = threadIdx.x & 63, jd = threadIdx.x >> 6;   // along D0: lane dd, rows jd + 4 u\n"
+      << "  const int jj = threadIdx.x % TJ, dj = threadIdx.x / TJ;   // along J: lane jj, columns dj + (256 / TJ) u\n"
+      << "  for (long long item = blockIdx.x; item < v.items; item += gridDim.x) {\n"
+      << "    const unp::ew_tile<" << N << "> t(v, item, 64, TJ);\n"
+      << "    const int n0 = (int)(v.e0 - t.d0 < 64 ? v.e0 - t.d0 : 64), nj = (int)(v.ej - t.j0 < TJ ? v.ej - t.j0 : TJ);\n"
+      << "    ew_t r[" << N << "][U];\n"
+      << "    // Past the tile's edge the last element inside is read.\n"
+      << "    auto load = [&](const ew_t* in, int k, ew_t (&x)[U]) {\n"
+      << "      const ew_t* p = in + t.in[k] + t.d0 * v.i0[k] + t.j0 * v.ij[k];\n"
+      << "      const bool tr = (v.tr >> k) & 1u;\n"
+      << "#pragma unroll\n"
+      << "      for (int u = 0; u < U; ++u) {\n"
+      << "        const int d = tr ? dj + (256 / TJ) * u : dd, j = tr ? jj : jd + 4 * u;\n"
+      << "        x[u] = p[(d < n0 ? d : n0 - 1) * v.i0[k] + (j < nj ? j : nj - 1) * v.ij[k]];\n"
+      << "      }\n    };\n"
+      << "    auto transpose = [&](int k, ew_t (&x)[U]) {\n"
+      << "      if (!((v.tr >> k) & 1u)) return;\n"
+      << "      __syncthreads();\n"
+      << "#pragma unroll\n"
+      << "      for (int u = 0; u < U; ++u) turn[(dj + (256 / TJ) * u) * (TJ + 1) + jj] = x[u];\n"
+      << "      __syncthreads();\n"
+      << "#pragma unroll\n"
+      << "      for (int u = 0; u < U; ++u) x[u] = turn[dd * (TJ + 1) + jd + 4 * u];\n"
+      << "    };\n";
+  for (int k = 0; k < n; ++k) src << "    load(static_cast<const ew_t*>(in" << k << "), " << k << ", r[" << k << "]);\n";
+  for (int k = 0; k < n; ++k) src << "    transpose(" << k << ", r[" << k << "]);\n";
+  src << "    ew_t* o = static_cast<ew_t*>(out) + t.out + t.d0 + dd + t.j0 * v.oj;\n"
+      << "#pragma unroll\n"
+      << "    for (int u = 0; u < U; ++u) {\n"
+      << "      const ew_t a[" << N << "] = " << loads("r[#][u]") << ";\n"
+      << "      if (dd < n0 && jd + 4 * u < nj) "
+      << (eb <= 8 ? "__builtin_nontemporal_store(ew_cell(a), o + (jd + 4 * u) * v.oj);\n" : "o[(jd + 4 * u) * v.oj] = ew_cell(a);\n")
+      << "    }\n  }\n}\n";
   Entry ev;
   ev.symbol = V;
   ev.fast = true;
@@ -1620,7 +1664,11 @@ int32_t lower_elementwise(const unp_form& f, const ElementwiseExpr& ew, Lowered&
   Entry ee = es;
   ee.symbol = E;
   ee.strided = true;
-  L.entries = {ev, es, ee};
+  Entry et = ee;
+  et.symbol = TE;
+  et.team = true;
+  et.vec = TJ;
+  L.entries = {ev, es, ee, et};
   L.source = src.str();
   std::ostringstream j;
   j << "{\"backend\":\"hip\",\"target\":\"rocm:gfx950\",\"form\":\"elementwise\",\"dtype\":\"" << kind_name(f.dtype)
@@ -1639,7 +1687,9 @@ int32_t lower_elementwise(const unp_form& f, const ElementwiseExpr& ew, Lowered&
        "\"lanes stride over the elements (16-byte packs on the _v entry)\"},\"entries\":["
     << "{\"symbol\":\"" << V << "\",\"when\":\"every buffer dense row-major, no permuted input, every base 16-byte aligned\"},"
     << "{\"symbol\":\"" << S << "\",\"when\":\"every buffer dense row-major and no permuted input, any alignment\"},"
-    << "{\"symbol\":\"" << E << "\",\"when\":\"a permuted input, or storage images that are not dense row-major\"}]"
+    << "{\"symbol\":\"" << TE << "\",\"when\":\"a permuted input, or storage images that are not dense row-major, with "
+       "two merged axes or more and an output axis of stride 1 and at least 16 elements\"},"
+    << "{\"symbol\":\"" << E << "\",\"when\":\"any other permuted input or storage images\"}]"
     << ",\"workspace\":null,\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
     << ",\"fidelity_notes\":["
     << json_str(leaf ? "a raw bit move: bit-exact for every grid and block"

@@ -371,6 +371,33 @@ UNP_DEV u32 draw_ticket(u32* counter) {
   return __builtin_amdgcn_atomic_inc32(counter, 0xffffffffu, __ATOMIC_RELAXED, "agent");
 }
 
+// Division of 0 <= q < 2^53 by e >= 1 through 1 / e in f64 (a 64-bit integer division is a sequence
+// of well over a hundred instructions): q * inv is within one of the quotient, so the truncation is
+// off by one at most and the remainder says which way.
+struct divisor {
+  i64 e;
+  double inv;
+  UNP_DEV divisor(i64 e_) : e(e_), inv(1.0 / (double)e_) {}
+  UNP_DEV divisor(i64 e_, double inv_) : e(e_), inv(inv_) {}
+  UNP_DEV void operator()(i64 q, i64& quo, i64& rem) const {
+    i64 t = (i64)((double)q * inv), r = q - t * e;
+    if (r < 0) {
+      --t;
+      r += e;
+    } else if (r >= e) {
+      ++t;
+      r -= e;
+    }
+    quo = t;
+    rem = r;
+  }
+  UNP_DEV i64 quo(i64 q) const {
+    i64 t, r;
+    (*this)(q, t, r);
+    return t;
+  }
+};
+
 // ---------------------------------------------------------------------------------------
 // Bounded waits.  A wave that waits for another block (a scan tile for its predecessors'
 // status, a full reduction's folding block for the other blocks' partials, a staged scan's
@@ -844,33 +871,6 @@ struct red_axes {
   i64 L;
   i64 runs;             // innermost runs: of one output's positions (xreduce_inner), of the outputs
   i64 outs, count;      // output elements, reduced positions per output
-};
-
-// Division of 0 <= q < 2^53 by e >= 1 through 1 / e in f64 (a 64-bit integer division is a sequence
-// of well over a hundred instructions): q * inv is within one of the quotient, so the truncation is
-// off by one at most and the remainder says which way.
-struct divisor {
-  i64 e;
-  double inv;
-  UNP_DEV divisor(i64 e_) : e(e_), inv(1.0 / (double)e_) {}
-  UNP_DEV divisor(i64 e_, double inv_) : e(e_), inv(inv_) {}
-  UNP_DEV void operator()(i64 q, i64& quo, i64& rem) const {
-    i64 t = (i64)((double)q * inv), r = q - t * e;
-    if (r < 0) {
-      --t;
-      r += e;
-    } else if (r >= e) {
-      ++t;
-      r -= e;
-    }
-    quo = t;
-    rem = r;
-  }
-  UNP_DEV i64 quo(i64 q) const {
-    i64 t, r;
-    (*this)(q, t, r);
-    return t;
-  }
 };
 
 // The element offset of position q over n axes, row-major.
@@ -2507,6 +2507,43 @@ struct gather_x_view {
   i64 ext[8], ostr[8];
   i64 istr[8][8];
   i64 outs;
+};
+
+// An elementwise op over strided buffers in tiles of two axes: D0 (the output's axis of stride 1) and J.
+// Inputs of stride 1 along J instead (bit k of `tr`) are read along J and turned in LDS; the others
+// and the output go by their strides, along D0.  The remaining axes number the tiles' planes.
+struct ew_tile_view {
+  i64 n;                    // remaining axes, outermost first
+  i64 ext[8], ostr[8];
+  double inv[8];            // 1 / ext
+  i64 istr[8][8];           // [input][axis]
+  i64 e0, ej;               // extents of D0 and J
+  i64 oj, i0[8], ij[8];     // the output's stride along J; the inputs' along D0 and J
+  i64 t0, items;            // tiles along D0, tiles in all
+  double inv_t0, inv_tj;    // 1 / tiles along D0 and along J
+  i64 tj;
+  u32 tr, pad;
+};
+
+// Where tile `item` lies: its first coordinates along D0 and J and the buffers' offsets of its plane.
+template <int N> struct ew_tile {
+  i64 d0, j0, out, in[N];
+  UNP_DEV ew_tile(const ew_tile_view& v, i64 item, int td, int tj) : out(0) {
+    i64 q, t;
+    divisor(v.t0, v.inv_t0)(item, q, t);
+    d0 = t * td;
+    divisor(v.tj, v.inv_tj)(q, q, t);
+    j0 = t * tj;
+#pragma unroll
+    for (int k = 0; k < N; ++k) in[k] = 0;
+    for (i64 d = v.n - 1; d >= 0; --d) {
+      i64 c;
+      divisor(v.ext[d], v.inv[d])(q, q, c);
+      out += c * v.ostr[d];
+#pragma unroll
+      for (int k = 0; k < N; ++k) in[k] += c * v.istr[k][d];
+    }
+  }
 };
 
 template <class E, class IDX, int POLICY>

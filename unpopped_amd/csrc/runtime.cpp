@@ -869,6 +869,7 @@ void fill_red_view(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask,
 
 static_assert(sizeof(unp::red_view_host) == 44 * 8, "red_view_host mirrors the device's red_view");
 static_assert(sizeof(unp::scan_view_host) == 29 * 8, "scan_view_host mirrors the device's scan_view");
+static_assert(sizeof(unp::ew_tile_view_host) == 114 * 8, "ew_tile_view_host mirrors the device's ew_tile_view");
 static_assert(sizeof(unp::gather_view_host) == 35 * 8, "gather_view_host mirrors the device's gather_view");
 static_assert(sizeof(unp::red_axes_host) == 54 * 8, "red_axes_host mirrors the device's red_axes");
 
@@ -1366,6 +1367,56 @@ int32_t run_gather(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_e
   return launch(x, entry, grid, params, s, err);
 }
 
+// The tiled entry's descriptor for strided buffers, if its tiles suit them: an output axis of stride 1
+// and at least 16 elements (D0), and a second axis (J): the one along which the inputs that are not
+// of stride 1 (or 0) along D0 have it, when it has 16 elements too, else the next one outwards.
+// Axes of extent 1 are dropped and adjacent axes that every buffer walks as one are merged.
+bool tile_axes(const unp::gather_x_view_host& v, size_t ni, int tj, unp::ew_tile_view_host& d) {
+  std::vector<std::vector<long long>> ax;  // per merged axis: extent, output stride, input strides
+  for (long long a = 0; a < v.rank; ++a) {
+    std::vector<long long> x{v.ext[a], v.ostr[a]};
+    for (size_t k = 0; k < ni; ++k) x.push_back(v.istr[k][a]);
+    if (x[0] == 1) continue;
+    bool merge = !ax.empty();
+    for (size_t i = 1; merge && i < x.size(); ++i) merge = ax.back()[i] == x[0] * x[i];
+    if (merge) x[0] *= ax.back()[0], ax.back() = x;
+    else ax.push_back(x);
+  }
+  size_t d0 = ax.size(), j = ax.size();
+  for (size_t a = 0; a < ax.size(); ++a)
+    if (ax[a][1] == 1) d0 = a;
+  if (ax.size() < 2 || d0 == ax.size() || ax[d0][0] < 16) return false;
+  d = unp::ew_tile_view_host{};
+  for (size_t k = 0; k < ni; ++k) {
+    if (ax[d0][2 + k] == 1 || ax[d0][2 + k] == 0) continue;
+    for (size_t a = 0; a < ax.size(); ++a)
+      if (a != d0 && ax[a][2 + k] == 1 && ax[a][0] >= 16 && (j == ax.size() || j == a)) {
+        j = a;
+        d.tr |= 1u << k;
+      }
+  }
+  if (j == ax.size()) j = d0 > 0 ? d0 - 1 : d0 + 1;
+  d.e0 = ax[d0][0];
+  d.ej = ax[j][0];
+  d.oj = ax[j][1];
+  for (size_t k = 0; k < ni; ++k) d.i0[k] = ax[d0][2 + k], d.ij[k] = ax[j][2 + k];
+  d.t0 = (d.e0 + 63) / 64;
+  d.tj = (d.ej + tj - 1) / tj;
+  d.items = d.t0 * d.tj;
+  for (size_t a = 0; a < ax.size(); ++a) {
+    if (a == d0 || a == j) continue;
+    d.ext[d.n] = ax[a][0];
+    d.inv[d.n] = 1.0 / (double)ax[a][0];
+    d.ostr[d.n] = ax[a][1];
+    for (size_t k = 0; k < ni; ++k) d.istr[k][d.n] = ax[a][2 + k];
+    d.items *= ax[a][0];
+    ++d.n;
+  }
+  d.inv_t0 = 1.0 / (double)d.t0;
+  d.inv_tj = 1.0 / (double)d.tj;
+  return true;
+}
+
 // The elementwise op's strided launch: the descriptor holds the output's extents and strides and
 // every input's strides over the output's axes.
 int32_t launch_elementwise_strided(unp_exec* x, const std::vector<uint64_t>& ptrs, const unp::gather_x_view_host& v,
@@ -1374,6 +1425,13 @@ int32_t launch_elementwise_strided(unp_exec* x, const std::vector<uint64_t>& ptr
   std::vector<uint64_t> p(ptrs);
   std::vector<void*> params;
   for (auto& q : p) params.push_back(&q);
+  unp::ew_tile_view_host tv;
+  const size_t tiled = x->l.entries.size() - 1;
+  if (tile_axes(v, ptrs.size() - 1, x->l.entries[tiled].vec, tv)) {
+    params.push_back(&tv);
+    return launch(x, tiled, (uint32_t)std::min<long long>(tv.items, (long long)x->cu_count * x->l.blocks_per_cu),
+                  params.data(), s, err);
+  }
   unp::gather_x_view_host vv = v;
   params.push_back(&vv);
   const long long blocks = (v.outs + 255) / 256;

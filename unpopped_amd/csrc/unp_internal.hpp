@@ -30,7 +30,8 @@ struct Entry {
   bool wide = false;  // reduction: the block-per-row schedule (long rows)
   int threads = 0;    // block size of this entry (0: the form's)
   int blocks_per_cu = 0;  // persistent blocks per CU of this entry (0: the form's)
-  bool team = false;      // split reduction, innermost run reduced: a wave per output
+  bool team = false;      // split reduction, innermost run reduced: a wave per output; elementwise: the
+                          // tiled entry (vec: its tile's rows)
   int cols = 0;           // output columns per block (dequant GEMM decode entries)
   // Reads and writes its buffers through storage-image strides (unp_hip_exec_launch_views with a
   // view that is not dense row-major); never picked for a pointer launch.
@@ -86,6 +87,20 @@ struct gather_x_view_host {
   long long ext[8], ostr[8];
   long long istr[8][8];
   long long outs;
+};
+
+// The host image of the device's ew_tile_view (the tiled elementwise entry's argument).
+struct ew_tile_view_host {
+  long long n;
+  long long ext[8], ostr[8];
+  double inv[8];
+  long long istr[8][8];
+  long long e0, ej;
+  long long oj, i0[8], ij[8];
+  long long t0, items;
+  double inv_t0, inv_tj;
+  long long tj;
+  uint32_t tr, pad;
 };
 
 // An Access::RowReduce (crates/unpopped/src/ir.rs:2114-2125): the stages' pre expressions and
