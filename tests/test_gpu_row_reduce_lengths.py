@@ -1,0 +1,66 @@
+"""Row reductions over rows of every kind of length: ragged rows in registers, rows in chunks with a launch
+per stage, rows of chunks in one block; unaligned buffers, in place, and the same bits without a
+workspace."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+import unpopped_amd as u
+from tests.test_gpu_parity import f64_order_tolerance, ulps
+from unpopped_amd import expr as X, forms as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 1), (5, 3), (4, 4), (3, 5), (2, 1023), (2300, 37), (3, 4095), (3, 4097),
+                                       (2, 8191), (2, 8193), (600, 8195), (2, 16383), (2, 16385), (1, 50001),
+                                       (3, 20480), (1, 300001), (520, 16388)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("which", ["softmax", "rms_norm"])
+def test_rows_of_any_length(hip_device, rows, cols, dtype, which):
+    stages, epi = getattr(X, which)()
+    x = np.random.default_rng(41).normal(size=(rows, cols)).astype(dtype)
+    want = oracle.row_reduce([x], stages, epi)
+    ex = H.row_reduce_executor("F32" if dtype == np.float32 else "F64", 2, stages, epi)
+    H.say(f"[case] row_reduce length {which} {rows}x{cols} {np.dtype(dtype).name}")
+
+    def near(got):
+        # F32: 2 ulps.  F64: 4 ulps, or what another order of the row's sum allows: the serial fold and
+        # this one are each within gamma_(n-1) * sum|x| of the exact sum.
+        if dtype == np.float32:
+            return ulps(got, want).max() <= 2
+        far = ulps(got, want) > 4
+        return (np.abs(got - want)[far] <= f64_order_tolerance(x, want, which)[far]).all()
+
+    for shift in (0, x.itemsize):
+        src, dst = u.DeviceBuffer(x.nbytes + 64), u.DeviceBuffer(x.nbytes + 64)
+        dst.fill(0x5A)
+        src.at(shift).upload(x)
+        ex.launch(src.at(shift), dst.at(shift), rows, cols)
+        u.synchronize()
+        got = dst.at(shift).download(dtype, x.size).reshape(x.shape)
+        assert near(got)
+        assert (dst.at(shift + x.nbytes).download(np.uint8, 64 - shift) == 0x5A).all()
+        ex.launch_static(src.at(shift), dst.at(shift), rows, cols)
+        u.synchronize()
+        assert dst.at(shift).download(dtype, x.size).tobytes() == got.tobytes()
+        ex.launch(src.at(shift), src.at(shift), rows, cols)  # in place
+        u.synchronize()
+        assert src.at(shift).download(dtype, x.size).tobytes() == got.tobytes()
+
+
+def test_two_inputs_nan_and_infinities_in_chunks(hip_device):
+    """Max and Sum stages over two inputs, in chunks, with a NaN row, an infinite one and one of the lowest
+    values: the oracle's values, the NaNs where it has them."""
+    r = np.random.default_rng(42)
+    a, b = r.integers(-8, 9, (4, 20001)).astype(np.float32), r.integers(-8, 9, (4, 20001)).astype(np.float32)
+    a[1, 19999], a[2, 5], a[3, :] = np.nan, np.inf, np.finfo(np.float32).min
+    b[3, :] = 0
+    stages = [(X.input(0) * X.input(1), "Sum"), (X.input(0) - X.reduced(0), "Max")]
+    epi = X.fma(X.input(0), X.reduced(1), X.input(1) - X.reduced(0))
+    H.say("[case] row_reduce chunks, two inputs, special values")
+    with np.errstate(all="ignore"):
+        want = oracle.row_reduce([a, b], stages, epi)
+    assert np.array_equal(H.row_reduce([a, b], stages, epi), want, equal_nan=True)

@@ -1797,23 +1797,50 @@ int32_t lower_row_reduce(const RowReduceSpec& sp, Lowered& L, std::string& why) 
     src << "template <> __device__ __forceinline__ double " << ops << "::pre<" << st
         << ">(const double* x, const double* r) { (void)x; (void)r; return " << pre[st] << "; }\n";
   const int vec = vec_of(sp.dtype);
+  // The row in registers: four or eight vectors per thread of 256, or eight of 512 (f32 softmax of 918 x
+  // 10955: 26.4 us, 54.2 re-read element by element; of 200 x 10000: 7.1, 16.5 in chunks).  The `rag`
+  // ones take any row of a vector or more at any alignment (f32 RMS norm of 8192 x 4095: 50.3 us, 89.9
+  // element by element; the whole-vector entry takes 45 for 8192 x 4096).
   struct E {
     const char* suffix;
     int vec, r;
     bool fast;
-  } es[] = {{"_c4", vec, 4, true}, {"_c", vec, 8, true}, {"_v", vec, 0, true}, {"_s", 1, 0, false}};
+    bool rag;
+    int threads;
+  } es[] = {{"_c4", vec, 4, true, false, 256},    {"_c", vec, 8, true, false, 256},   {"_c512_v", vec, 8, true, false, 512},
+            {"_c4_s", vec, 4, false, true, 256},  {"_c_s", vec, 8, false, true, 256}, {"_c512_s", vec, 8, false, true, 512},
+            {"_s", 1, 0, false, false, 256}};
   for (const E& e : es) {
     Entry en;
     en.symbol = L.name + e.suffix;
     en.vec = e.vec;
     en.k = e.r;  // vectors per thread held in registers (0: re-read)
     en.fast = e.fast;
-    src << "extern \"C\" __global__ void " << kLaunchBounds << " " << en.symbol << "(";
+    en.threads = e.threads;
+    src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << en.symbol << "(";
     for (int k = 0; k < sp.n_inputs; ++k) src << "const " << T << "* in" << k << ", ";
     src << T << "* out, long long rows, long long cols) {\n  const " << T << "* in[" << sp.n_inputs << "] = {";
     for (int k = 0; k < sp.n_inputs; ++k) src << (k ? ", " : "") << "in" << k;
-    src << "};\n  unp::row_reduce_staged<" << T << ", " << sp.n_inputs << ", " << NS << ", " << ops << ", 256, " << e.vec
-        << ", " << e.r << ">(in, out, rows, cols);\n}\n";
+    src << "};\n  unp::row_reduce_staged<" << T << ", " << sp.n_inputs << ", " << NS << ", " << ops << ", " << e.threads
+        << ", " << e.vec << ", " << e.r << (e.rag ? ", true" : "") << ">(in, out, rows, cols);\n}\n";
+    L.entries.push_back(en);
+  }
+  // Rows beyond the registers, in chunks: a launch per stage and one for the epilogue, or (_a_v) all of
+  // it in one block per row.
+  for (size_t st = 0; st <= NS + 1; ++st) {
+    Entry en;
+    en.symbol = L.name + (st < NS ? "_p" + std::to_string(st) : st == NS ? "_p_v" : "_a_v");
+    en.vec = vec;
+    en.team = true;
+    src << "extern \"C\" __global__ void " << kLaunchBounds << " " << en.symbol << "(";
+    for (int k = 0; k < sp.n_inputs; ++k) src << "const " << T << "* in" << k << ", ";
+    src << T << "* out, long long rows, long long cols, long long chunks" << (st <= NS ? ", double* part" : "") << ") {\n  const "
+        << T << "* in[" << sp.n_inputs << "] = {";
+    for (int k = 0; k < sp.n_inputs; ++k) src << (k ? ", " : "") << "in" << k;
+    src << "};\n  unp::" << (st < NS ? "rr_chunk_stage<" : st == NS ? "rr_chunk_epilogue<" : "rr_chunk_rows<") << T << ", "
+        << sp.n_inputs << ", " << NS << ", " << ops << ", 256, " << vec;
+    if (st < NS) src << ", " << st;
+    src << ">(in, out, rows, cols, chunks" << (st <= NS ? ", part" : "") << ");\n}\n";
     L.entries.push_back(en);
   }
   L.source = src.str();
@@ -1831,14 +1858,18 @@ int32_t lower_row_reduce(const RowReduceSpec& sp, Lowered& L, std::string& why) 
   for (int d = 0; d < sp.rank; ++d) j << ",{\"name\":\"n" << d << "\",\"kind\":\"scalar\",\"dtype\":\"I32\"}";
   j << "],\"launch\":{\"block\":[256,1,1],\"grid\":\"cu_count*min(8, blocks one CU holds)\",\"grid_policy\":\"one "
        "block per row, rows block-strided; the next row's loads issued before this row's stages\"},\"entries\":[";
-  for (size_t i = 0; i < L.entries.size(); ++i)
-    j << (i ? "," : "") << "{\"symbol\":\"" << L.entries[i].symbol << "\",\"vec\":" << L.entries[i].vec
-      << ",\"row_in_registers\":" << (L.entries[i].k ? "true" : "false") << ",\"when\":\""
-      << (L.entries[i].k == 4 ? "cols % vec == 0, every buffer 16-byte aligned and cols <= 256 * vec * 4"
-          : L.entries[i].k     ? "cols % vec == 0, every buffer 16-byte aligned and 256 * vec * 4 < cols <= 256 * vec * 8"
-                               : (L.entries[i].fast ? "cols % vec == 0 and every buffer 16-byte aligned" : "otherwise"))
-      << "\"}";
-  j << "],\"workspace\":null"
+  for (size_t i = 0; i < L.entries.size(); ++i) {
+    const Entry& e = L.entries[i];
+    j << (i ? "," : "") << "{\"symbol\":\"" << e.symbol << "\",\"vec\":" << e.vec
+      << ",\"row_in_registers\":" << (e.k ? "true" : "false") << ",\"when\":\""
+      << (e.team ? (e.symbol == L.name + "_a_v" ? "longer rows, two or more per CU, or without a workspace"
+                                                : "longer rows: the stages in order, then the epilogue")
+          : e.threads == 512 ? "256 * vec * 8 < cols <= 512 * vec * 8"
+          : e.k      ? (e.k == 4 ? "vec <= cols <= 256 * vec * 4" : "256 * vec * 4 < cols <= 256 * vec * 8")
+                     : "cols < vec")
+      << (e.k ? (e.fast ? ", cols % vec == 0 and every buffer 16-byte aligned" : ", otherwise") : "") << "\"}";
+  }
+  j << "],\"workspace\":{\"partials\":\"stages * rows * chunks * 8\"}"
     << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
     << ",\"fidelity_notes\":["
     << json_str("expressions evaluate in f64 and round once per statement, as the kernel evaluator runs the lifted "

@@ -218,6 +218,11 @@ template <class T, int N> UNP_DEV vec<T, N> ld_any(const T* p) {
     return ld_nt<T, N>(p);
   }
 }
+// The same through the caches, for data that is read again.
+template <class T, int N> UNP_DEV vec<T, N> ld_cached(const T* p) {
+  static_assert(sizeof(T) * N == 16, "16-byte vectors");
+  return __builtin_bit_cast(vec<T, N>, (u32x4_t)*reinterpret_cast<const u32x4_any*>(p));
+}
 template <class T, int N> UNP_DEV void st_any(T* p, const vec<T, N>& v) {
   static_assert(sizeof(T) * N == 16, "16-byte vectors");
   __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_any*>(p));
@@ -3702,7 +3707,30 @@ template <class T> UNP_DEV T bit_or(T a, T b) { return (T)(a | b); }
 template <class T> UNP_DEV T bit_xor(T a, T b) { return (T)(a ^ b); }
 }  // namespace xi
 
-template <class T, int NI, int NS, class OPS, int THREADS, int VEC, int R, int S>
+// Where a row's vector vi lies with rows of any length >= VEC (RAG): a last one that would run past
+// the row starts at cols - VEC and its first `skip` elements are the vector before's; one past the
+// row is skipped whole.  Without RAG the rows hold whole vectors.
+template <int VEC, bool RAG> struct row_vec {
+  int at, skip;
+  UNP_DEV row_vec(int vi, i64 cols) : at(vi * VEC), skip(0) {
+    if constexpr (RAG) {
+      const int c = (int)cols;
+      skip = at >= c ? VEC : (at + VEC > c ? at + VEC - c : 0);
+      if (at < c) at -= skip;
+    } else {
+      skip = at < (int)cols ? 0 : VEC;
+    }
+  }
+};
+
+// A stage's fold of a whole row, finished and rounded to T.
+template <class T, int OP> UNP_DEV double rr_finish(double a, i64 cols) {
+  if constexpr (OP == OP_MEAN) a = a / (double)cols;
+  if constexpr (OP == OP_MAX || OP == OP_MIN) a = cols == 0 ? 0.0 : a;
+  return (double)(T)a;
+}
+
+template <class T, int NI, int NS, class OPS, int THREADS, int VEC, int R, int S, bool RAG = false>
 UNP_DEV void rr_stage(const T* const* rin, const vec<T, VEC> (&xr)[NI][R > 0 ? R : 1], i64 cols, double (&red)[NS],
                       double* part, double* redsh, double (&cv)[R > 0 ? R : 1][VEC]) {
   if constexpr (S < NS) {
@@ -3712,21 +3740,23 @@ UNP_DEV void rr_stage(const T* const* rin, const vec<T, VEC> (&xr)[NI][R > 0 ? R
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const i64 nvec = cols / VEC;
     double acc = F::identity();
-    auto fold_vec = [&](const vec<T, VEC> (&v)[NI]) {
+    auto fold_vec = [&](const vec<T, VEC> (&v)[NI], int skip) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         double x[NI];
 #pragma unroll
         for (int k = 0; k < NI; ++k) x[k] = (double)v[k].e[e];
-        acc = F::apply(acc, (double)(T)OPS::template pre<S>(x, red));
+        const double b = F::apply(acc, (double)(T)OPS::template pre<S>(x, red));
+        acc = !RAG || e >= skip ? b : acc;
       }
     };
     if constexpr (R > 0 && S == OPS::cached) {
       // This stage's per-element value recurs in the epilogue: keep it (in f64, before the
       // stage's rounding to T) for the epilogue to read back.
 #pragma unroll
-      for (int q = 0; q < R; ++q)
-        if ((i64)q * THREADS + tid < nvec) {
+      for (int q = 0; q < R; ++q) {
+        const row_vec<VEC, RAG> w(q * THREADS + tid, cols);
+        if (w.skip < VEC) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
             double x[NI];
@@ -3734,24 +3764,28 @@ UNP_DEV void rr_stage(const T* const* rin, const vec<T, VEC> (&xr)[NI][R > 0 ? R
             for (int k = 0; k < NI; ++k) x[k] = (double)xr[k][q].e[e];
             const double p = OPS::template pre<S>(x, red);
             cv[q][e] = p;
-            acc = F::apply(acc, (double)(T)p);
+            const double b = F::apply(acc, (double)(T)p);
+            acc = !RAG || e >= w.skip ? b : acc;
           }
         }
+      }
     } else if constexpr (R > 0) {
 #pragma unroll
-      for (int q = 0; q < R; ++q)
-        if ((i64)q * THREADS + tid < nvec) {
+      for (int q = 0; q < R; ++q) {
+        const row_vec<VEC, RAG> w(q * THREADS + tid, cols);
+        if (w.skip < VEC) {
           vec<T, VEC> xv[NI];
 #pragma unroll
           for (int k = 0; k < NI; ++k) xv[k] = xr[k][q];
-          fold_vec(xv);
+          fold_vec(xv, RAG ? w.skip : 0);
         }
+      }
     } else {
       for (i64 v = tid; v < nvec; v += THREADS) {
         vec<T, VEC> xv[NI];
 #pragma unroll
         for (int k = 0; k < NI; ++k) xv[k] = ld<T, VEC>(rin[k] + v * VEC);
-        fold_vec(xv);
+        fold_vec(xv, 0);
       }
     }
     acc = wave_reduce<double, OP>(acc);
@@ -3761,18 +3795,15 @@ UNP_DEV void rr_stage(const T* const* rin, const vec<T, VEC> (&xr)[NI][R > 0 ? R
       double a = part[0];
 #pragma unroll
       for (int w = 1; w < WAVES; ++w) a = F::apply(a, part[w]);
-      double fin = a;
-      if constexpr (OP == OP_MEAN) fin = a / (double)cols;
-      if constexpr (OP == OP_MAX || OP == OP_MIN) fin = cols == 0 ? 0.0 : a;
-      redsh[S] = (double)(T)fin;
+      redsh[S] = rr_finish<T, OP>(a, cols);
     }
     __syncthreads();
     red[S] = redsh[S];
-    rr_stage<T, NI, NS, OPS, THREADS, VEC, R, S + 1>(rin, xr, cols, red, part, redsh, cv);
+    rr_stage<T, NI, NS, OPS, THREADS, VEC, R, S + 1, RAG>(rin, xr, cols, red, part, redsh, cv);
   }
 }
 
-template <class T, int NI, int NS, class OPS, int THREADS, int VEC, int R>
+template <class T, int NI, int NS, class OPS, int THREADS, int VEC, int R, bool RAG = false>
 UNP_DEV void row_reduce_staged(const T* const* in, T* __restrict__ out, i64 rows, i64 cols) {
   __shared__ double part[THREADS / 64];
   __shared__ double redsh[NS];
@@ -3797,7 +3828,7 @@ UNP_DEV void row_reduce_staged(const T* const* in, T* __restrict__ out, i64 rows
         const __amdgpu_buffer_rsrc_t rk = row_rsrc(in[k], row);
 #pragma unroll
         for (int q = 0; q < R; ++q)
-          xr[k][q] = __builtin_bit_cast(vec<T, VEC>, __builtin_amdgcn_raw_buffer_load_b128(rk, (q * THREADS + tid) * 16, 0, 2));
+          xr[k][q] = __builtin_bit_cast(vec<T, VEC>, __builtin_amdgcn_raw_buffer_load_b128(rk, row_vec<VEC, RAG>(q * THREADS + tid, cols).at * (int)sizeof(T), 0, 2));
       }
     }
   };
@@ -3808,7 +3839,7 @@ UNP_DEV void row_reduce_staged(const T* const* in, T* __restrict__ out, i64 rows
     T* __restrict__ rout = out + row * cols;
     double red[NS];
     double cv[R > 0 ? R : 1][VEC];
-    rr_stage<T, NI, NS, OPS, THREADS, VEC, R, 0>(rin, xr, cols, red, part, redsh, cv);
+    rr_stage<T, NI, NS, OPS, THREADS, VEC, R, 0, RAG>(rin, xr, cols, red, part, redsh, cv);
     auto emit = [&](const vec<T, VEC> (&v)[NI], i64 at) {
       vec<T, VEC> o;
 #pragma unroll
@@ -3834,7 +3865,7 @@ UNP_DEV void row_reduce_staged(const T* const* in, T* __restrict__ out, i64 rows
           if constexpr (OPS::cached >= 0) o.e[e] = (T)OPS::epi_c(x, red, cv[q][e]);
           else o.e[e] = (T)OPS::epi(x, red);
         }
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4b, o), ro, (q * THREADS + tid) * 16, 0, 2);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4b, o), ro, row_vec<VEC, RAG>(q * THREADS + tid, cols).at * (int)sizeof(T), 0, 2);
       }
     } else {
       for (i64 v = tid; v < nvec; v += THREADS) {
@@ -3862,6 +3893,148 @@ UNP_DEV void row_reduce_staged(const T* const* in, T* __restrict__ out, i64 rows
   } else {
     RowRegs none;
     for (i64 row = blockIdx.x; row < rows; row += G) one_row(row, none);
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The same over rows too long for a block's registers: each row's vectors are cut into C chunks and
+// the stages run one after another over all (row, chunk) items, blocks striding over them, so a few
+// long rows reach every CU.  Stage S leaves each chunk's partial fold in part[S][row][chunk]; what
+// follows it (the next stages, the epilogue) folds a row's partials first: lane l the chunks l, l +
+// 64, ..., then the lanes.  rr_chunk_stage and rr_chunk_epilogue are a launch each, so a stage's
+// partials are whole before they are read; rr_chunk_rows walks the chunks of its rows in one block
+// instead, for a launch that has no workspace, with the same partials in the same order.
+// Rows have any length >= VEC and any alignment (row_vec).
+//
+// Bound by the f64 arithmetic of the pre expressions, once the row's reads after the first come from
+// the caches: softmax over 64 rows of 50001 f32 takes 20 us, 132 with one block per row that reads
+// it element by element.
+// ---------------------------------------------------------------------------------------
+template <class T, int NI, int NS, class OPS, int THREADS, int VEC> struct rr_chunks {
+  static constexpr int R = 4;  // vectors per thread and pass
+  const T* const* in;
+  T* out;
+  i64 cols, C, nvec;
+  UNP_DEV rr_chunks(const T* const* in_, T* out_, i64 cols_, i64 C_)
+      : in(in_), out(out_), cols(cols_), C(C_), nvec((cols_ + VEC - 1) / VEC) {}
+
+  // fn(vector's first element, its leading elements that are another vector's, the inputs) over
+  // chunk c of a row, R vectors of each input in flight.
+  template <class Fn> UNP_DEV void each(i64 row, i64 c, Fn&& fn) const {
+    const i64 v0 = nvec * c / C, v1 = nvec * (c + 1) / C;
+    for (i64 v = v0; v < v1; v += THREADS * R) {
+      vec<T, VEC> x[R][NI];
+      i64 at[R];
+      int skip[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const i64 i = v + q * THREADS + (i64)threadIdx.x;
+        const i64 w = (i < v1 ? i : v1 - 1) * VEC;  // past the chunk its last vector is read and ignored
+        at[q] = w + VEC <= cols ? w : cols - VEC;
+        skip[q] = i < v1 ? (int)(w - at[q]) : VEC;
+#pragma unroll
+        for (int k = 0; k < NI; ++k) x[q][k] = ld_cached<T, VEC>(in[k] + row * cols + at[q]);
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q) fn(at[q], skip[q], x[q]);
+    }
+  }
+
+  // Chunk c of a row folded by stage S, in every thread (`sh`: a slot per wave).
+  template <int S> UNP_DEV double fold(i64 row, i64 c, const double (&red)[NS], double* sh) const {
+    typedef unp::fold<double, OPS::op[S]> F;
+    double acc = F::identity();
+    each(row, c, [&](i64, int skip, const vec<T, VEC> (&v)[NI]) {
+      if (skip == VEC) return;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        double x[NI];
+#pragma unroll
+        for (int k = 0; k < NI; ++k) x[k] = (double)v[k].e[e];
+        const double b = F::apply(acc, (double)(T)OPS::template pre<S>(x, red));
+        acc = e >= skip ? b : acc;
+      }
+    });
+    return block_reduce<double, OPS::op[S], THREADS>(acc, sh);
+  }
+
+  // Stage S of a row from its chunks' partials, in every lane.
+  template <int S> UNP_DEV double finish(const double* part) const {
+    typedef unp::fold<double, OPS::op[S]> F;
+    double a = F::identity();
+    for (i64 c = threadIdx.x & 63; c < C; c += 64) a = F::apply(a, part[c]);
+    return rr_finish<T, OPS::op[S]>(wave_reduce<double, OPS::op[S]>(a), cols);
+  }
+
+  UNP_DEV void epilogue(i64 row, i64 c, const double (&red)[NS]) const {
+    each(row, c, [&](i64 at, int skip, const vec<T, VEC> (&v)[NI]) {
+      if (skip == VEC) return;
+      vec<T, VEC> o;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        double x[NI];
+#pragma unroll
+        for (int k = 0; k < NI; ++k) x[k] = (double)v[k].e[e];
+        o.e[e] = (T)OPS::epi(x, red);
+      }
+      // A shifted vector's first elements are another lane's to store: in place, this one may have
+      // read them after that.
+      T* const p = out + row * cols + at;
+      if (skip == 0) {
+        st_any<T, VEC>(p, o);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          if (e >= skip) p[e] = o.e[e];
+      }
+    });
+  }
+};
+
+template <class T, int NI, int NS, class OPS, int THREADS, int VEC, int S>
+UNP_DEV void rr_chunk_stage(const T* const* in, T* out, i64 rows, i64 cols, i64 C, double* part) {
+  const rr_chunks<T, NI, NS, OPS, THREADS, VEC> ch(in, out, cols, C);
+  __shared__ double sh[THREADS / 64];
+  const divisor by_chunks(C);
+  for (i64 item = blockIdx.x; item < rows * C; item += gridDim.x) {
+    i64 row, c;
+    by_chunks(item, row, c);
+    double red[NS] = {};
+    unroll_for<S>([&](auto t) { red[t.value] = ch.template finish<t.value>(part + (t.value * rows + row) * C); });
+    const double a = ch.template fold<S>(row, c, red, sh);
+    if (threadIdx.x == 0) part[(S * rows + row) * C + c] = a;
+  }
+}
+
+template <class T, int NI, int NS, class OPS, int THREADS, int VEC>
+UNP_DEV void rr_chunk_epilogue(const T* const* in, T* out, i64 rows, i64 cols, i64 C, const double* part) {
+  const rr_chunks<T, NI, NS, OPS, THREADS, VEC> ch(in, out, cols, C);
+  const divisor by_chunks(C);
+  for (i64 item = blockIdx.x; item < rows * C; item += gridDim.x) {
+    i64 row, c;
+    by_chunks(item, row, c);
+    double red[NS];
+    unroll_for<NS>([&](auto t) { red[t.value] = ch.template finish<t.value>(part + (t.value * rows + row) * C); });
+    ch.epilogue(row, c, red);
+  }
+}
+
+template <class T, int NI, int NS, class OPS, int THREADS, int VEC>
+UNP_DEV void rr_chunk_rows(const T* const* in, T* out, i64 rows, i64 cols, i64 C) {
+  const rr_chunks<T, NI, NS, OPS, THREADS, VEC> ch(in, out, cols, C);
+  __shared__ double sh[THREADS / 64], part[kMaxChunks];
+  for (i64 row = blockIdx.x; row < rows; row += gridDim.x) {
+    double red[NS] = {};
+    unroll_for<NS>([&](auto t) {
+      for (i64 c = 0; c < C; ++c) {
+        const double a = ch.template fold<t.value>(row, c, red, sh);
+        if (threadIdx.x == 0) part[c] = a;
+      }
+      __syncthreads();
+      red[t.value] = ch.template finish<t.value>(part);
+      __syncthreads();  // `part` is the next stage's
+    });
+    for (i64 c = 0; c < C; ++c) ch.epilogue(row, c, red);
   }
 }
 

@@ -139,12 +139,16 @@ constexpr size_t kSplitRounds = 4, kMaxStreams = 4;
 bool inner_reduced(const unp::Lowered& l) { return (l.axes_mask >> (l.form.rank - 1)) & 1u; }
 size_t split_items(const unp_exec* x) { return kSplitRounds * (size_t)x->cu_count * (size_t)x->l.blocks_per_cu; }
 size_t split_counter_bytes(const unp_exec* x) { return (split_items(x) * sizeof(uint32_t) + 255) / 256 * 256; }
+// A row reduction's chunked rows: a partial per stage and chunk, up to kRowChunks chunks in a launch.
+constexpr long long kRowChunks = 32768;
 size_t split_bytes(const unp_exec* x) {
+  if (x->l.form.kind == UNP_FORM_ROW_REDUCE) return split_counter_bytes(x) + (size_t)kRowChunks * x->l.rr.ops.size() * 8;
   const size_t values = inner_reduced(x->l) ? 1 : 64 * (16 / unp::kind_bytes(x->l.form.dtype));
   return split_counter_bytes(x) + split_items(x) * values * 16;
 }
 
 bool splits(const unp_exec* x) {
+  if (x->l.form.kind == UNP_FORM_ROW_REDUCE) return true;
   return x->l.form.kind == UNP_FORM_REDUCTION && (x->l.red_schedule == 'g' || x->l.red_schedule == 'm');
 }
 
@@ -1241,20 +1245,37 @@ int32_t run_row_reduce(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, u
   const int vec = 16 / (int)unp::kind_bytes(sp.dtype);
   bool aligned = cols % vec == 0;
   for (uint64_t p : A.buf) aligned = aligned && aligned16(p);
-  // entries: 0 the row in registers (4 vectors per thread), 1 in registers (8 vectors per
-  // thread), 2 vector passes, 3 scalar passes
-  const size_t entry = !aligned ? 3 : (cols <= 256LL * vec * 4 ? 0 : (cols <= 256LL * vec * 8 ? 1 : 2));
+  std::vector<uint64_t> ptrs(A.buf.begin(), A.buf.end());
+  std::vector<void*> params;
+  for (size_t i = 0; i < ptrs.size(); ++i) params.push_back(&ptrs[i]);
+  params.push_back(&rows);
+  params.push_back(&cols);
+  // entries: the row in registers (4 vectors per thread, 8, or 8 of 512 threads; 0 .. 2 whole aligned
+  // vectors, 3 .. 5 any row of a vector or more), 6 scalar passes, then the chunked rows: a launch per
+  // stage, the epilogue, and the whole row in one block.
+  const size_t held_by = cols <= 256LL * vec * 4 ? 0 : cols <= 256LL * vec * 8 ? 1 : 2;
+  if (cols > 512LL * vec * 8) {
+    // Two rows per CU or more: each in one block, which finds them in its caches again (600 x 40000 f32
+    // softmax 86 us, 96 in chunks of 4096); fewer: chunks of up to four vectors per thread of a block, on every CU.
+    const bool whole = rows >= 2LL * x->cu_count;
+    const long long nvec = (cols + vec - 1) / vec, most = whole ? 8192 : 1024;
+    long long chunks = std::min(unp::kMaxChunks, (nvec + most - 1) / most);
+    params.push_back(&chunks);
+    const size_t first = 7, stages = sp.ops.size();
+    const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
+    SplitWs w;
+    if (!whole && rows <= kRowChunks / chunks) w = stream_workspace(x, s);
+    if (!w.partials) return launch(x, first + stages + 1, grid, params.data(), s, err);
+    params.push_back(&w.partials);
+    for (size_t st = 0; st <= stages && rc == UNP_OK; ++st) rc = launch(x, first + st, grid, params.data(), s, err);
+    return rc;
+  }
+  const size_t entry = cols < vec ? 6 : (aligned ? 0 : 3) + held_by;
   // As many blocks as the CUs hold at once (at most blocks_per_cu each), so no blocks start late
   // as a tail that runs at a fraction of the occupancy.
   const int held = x->resident[entry];
   const long long cap = (long long)x->cu_count * (held > 0 && held < x->l.blocks_per_cu ? held : x->l.blocks_per_cu);
-  const uint32_t grid = (uint32_t)cap;
-  std::vector<void*> params;
-  std::vector<uint64_t> ptrs(A.buf.begin(), A.buf.end());
-  for (size_t i = 0; i < ptrs.size(); ++i) params.push_back(&ptrs[i]);
-  params.push_back(&rows);
-  params.push_back(&cols);
-  return launch(x, entry, grid, params.data(), s, err);
+  return launch(x, entry, (uint32_t)cap, params.data(), s, err);
 }
 
 // The general gather's launch: the descriptor from each input's strides (istr[k][d] over the output
