@@ -1687,9 +1687,9 @@ int32_t lower_elementwise(const unp_form& f, const ElementwiseExpr& ew, Lowered&
        "\"lanes stride over the elements (16-byte packs on the _v entry)\"},\"entries\":["
     << "{\"symbol\":\"" << V << "\",\"when\":\"every buffer dense row-major, no permuted input, every base 16-byte aligned\"},"
     << "{\"symbol\":\"" << S << "\",\"when\":\"every buffer dense row-major and no permuted input, any alignment\"},"
-    << "{\"symbol\":\"" << TE << "\",\"when\":\"a permuted input, or storage images that are not dense row-major, with "
-       "two merged axes or more and an output axis of stride 1 and at least 16 elements\"},"
-    << "{\"symbol\":\"" << E << "\",\"when\":\"any other permuted input or storage images\"}]"
+    << "{\"symbol\":\"" << E << "\",\"when\":\"a permuted input, or storage images that are not dense row-major\"}]"
+    << ",\"tiled_entries\":[{\"symbol\":\"" << TE << "\",\"when\":\"the same with two merged axes or more and an output "
+       "axis of stride 1 and at least 16 elements, in place of the strided entry\"}]"
     << ",\"workspace\":null,\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
     << ",\"fidelity_notes\":["
     << json_str(leaf ? "a raw bit move: bit-exact for every grid and block"
@@ -1858,17 +1858,28 @@ int32_t lower_row_reduce(const RowReduceSpec& sp, Lowered& L, std::string& why) 
   for (int d = 0; d < sp.rank; ++d) j << ",{\"name\":\"n" << d << "\",\"kind\":\"scalar\",\"dtype\":\"I32\"}";
   j << "],\"launch\":{\"block\":[256,1,1],\"grid\":\"cu_count*min(8, blocks one CU holds)\",\"grid_policy\":\"one "
        "block per row, rows block-strided; the next row's loads issued before this row's stages\"},\"entries\":[";
-  for (size_t i = 0; i < L.entries.size(); ++i) {
-    const Entry& e = L.entries[i];
-    j << (i ? "," : "") << "{\"symbol\":\"" << e.symbol << "\",\"vec\":" << e.vec
-      << ",\"row_in_registers\":" << (e.k ? "true" : "false") << ",\"when\":\""
-      << (e.team ? (e.symbol == L.name + "_a_v" ? "longer rows, two or more per CU, or without a workspace"
-                                                : "longer rows: the stages in order, then the epilogue")
-          : e.threads == 512 ? "256 * vec * 8 < cols <= 512 * vec * 8"
-          : e.k      ? (e.k == 4 ? "vec <= cols <= 256 * vec * 4" : "256 * vec * 4 < cols <= 256 * vec * 8")
-                     : "cols < vec")
-      << (e.k ? (e.fast ? ", cols % vec == 0 and every buffer 16-byte aligned" : ", otherwise") : "") << "\"}";
-  }
+  // "entries" lists the kernels for rows of whole aligned vectors and the scalar one, "ragged_entries"
+  // and "chunk_entries" the others.
+  auto list = [&](auto&& in) {
+    bool first = true;
+    for (const Entry& e : L.entries) {
+      if (!in(e)) continue;
+      j << (first ? "" : ",") << "{\"symbol\":\"" << e.symbol << "\",\"vec\":" << e.vec
+        << ",\"row_in_registers\":" << (e.k ? "true" : "false") << ",\"when\":\""
+        << (e.team ? (e.symbol == L.name + "_a_v" ? "longer rows, two or more per CU, or without a workspace"
+                                                  : "longer rows: the stages in order, then the epilogue")
+            : e.threads == 512 ? "256 * vec * 8 < cols <= 512 * vec * 8"
+            : e.k ? (e.k == 4 ? "vec <= cols <= 256 * vec * 4" : "256 * vec * 4 < cols <= 256 * vec * 8")
+                  : "cols < vec")
+        << (e.k ? (e.fast ? ", cols % vec == 0 and every buffer 16-byte aligned" : ", otherwise") : "") << "\"}";
+      first = false;
+    }
+  };
+  list([](const Entry& e) { return !e.team && (e.fast || e.k == 0); });
+  j << "],\"ragged_entries\":[";
+  list([](const Entry& e) { return !e.team && !e.fast && e.k != 0; });
+  j << "],\"chunk_entries\":[";
+  list([](const Entry& e) { return e.team; });
   j << "],\"workspace\":{\"partials\":\"stages * rows * chunks * 8\"}"
     << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
     << ",\"fidelity_notes\":["
