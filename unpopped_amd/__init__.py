@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes as C
 import json
+import struct
 from dataclasses import dataclass
 
 import numpy as np
@@ -375,6 +376,17 @@ class DeviceBuffer:
             pass
 
 
+class _ArgWords(dict):
+    """The packer of n unp_args (native little-endian words), made on first use."""
+
+    def __missing__(self, n: int):
+        self[n] = struct.Struct(f"{2 * n}Q").pack
+        return self[n]
+
+
+_ARG_WORDS = _ArgWords()
+
+
 class Executor:
     """A lowered kernel compiled, loaded and ready to launch on the current device."""
 
@@ -384,6 +396,10 @@ class Executor:
         err = _lib.Error()
         check(_lib.lib().unp_hip_exec_create(kernel._handle, C.byref(h), C.byref(err)), err)
         self._h = h
+        # One caller at a time: launches share an error and look nothing up.
+        self._err = err
+        self._perr = C.byref(err)
+        self._launch = _lib.lib().unp_hip_exec_launch
 
     @staticmethod
     def _args(args):
@@ -397,8 +413,13 @@ class Executor:
 
     def launch(self, *args, stream: int = 0) -> None:
         """Arguments in the KernelFn's parameter order: buffers, then integer scalars."""
-        err = _lib.Error()
-        check(_lib.lib().unp_hip_exec_launch(self._h, self._args(args), len(args), stream, C.byref(err)), err)
+        # A unp_arg as two words: is_buffer (its low half; the pad is 0), then the value.
+        words = []
+        for a in args:
+            words += (1, a.ptr) if isinstance(a, DeviceBuffer) else (0, int(a) & 0xFFFFFFFFFFFFFFFF)
+        rc = self._launch(self._h, _ARG_WORDS[len(args)](*words), len(args), stream, self._perr)
+        if rc:
+            check(rc, self._err)
 
     def launch_static(self, *args, stream: int = 0) -> None:
         """``launch`` with every workspace in the library's static device scratch

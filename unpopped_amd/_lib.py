@@ -134,7 +134,7 @@ def lib() -> C.CDLL:
         "unp_hip_event_synchronize": (i32, [P]),
         "unp_hip_event_elapsed_ms": (i32, [P, P, C.POINTER(C.c_float)]),
         "unp_hip_exec_create": (i32, [P, C.POINTER(P), E]),
-        "unp_hip_exec_launch": (i32, [P, C.POINTER(Arg), sz, P, E]),
+        "unp_hip_exec_launch": (i32, [P, P, sz, P, E]),  # the arguments: an Arg array, or their words as bytes
         "unp_hip_exec_launch_views": (i32, [P, C.POINTER(View), sz, C.POINTER(C.c_int64), sz, P, E]),
         "unp_hip_exec_launch_static": (i32, [P, C.POINTER(Arg), sz, P, E]),
         "unp_hip_exec_set_timing": (i32, [P, P, P]),
