@@ -90,11 +90,11 @@ static_assert(sizeof(unp::red_view) == 44 * 8, "red_view");
 static_assert(sizeof(unp::scan_view) == 29 * 8, "scan_view");
 static_assert(sizeof(unp::gather_view) == 35 * 8, "gather_view");
 static_assert(sizeof(unp::ew_tile_view) == 114 * 8, "ew_tile_view");
-extern "C" __global__ void KB c_rr(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce<float, unp::OP_SUM, unp::OP_MAX, 2, 4, 256, 4>(a, b, c, r, n); }
-extern "C" __global__ void KB c_rw(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce_wave<float, unp::OP_SUM, unp::OP_MAX, 2, 4, 256, 8>(a, b, c, r, n); }
-extern "C" __global__ void KB c_rri(const long long* a, long long* b, long long* c, long long r, long long n) { unp::rowreduce<long long, unp::OP_PROD, unp::OP_MIN, 2, 1, 256, 8>(a, b, c, r, n); }
+extern "C" __global__ void KB c_rr(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce<float, unp::OP_SUM, unp::OP_MAX, 2, 4, 256, 4, true>(a, b, c, r, n); }
+extern "C" __global__ void KB c_rw(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce_wave<float, unp::OP_SUM, unp::OP_MAX, 2, 4, 256, 8, true>(a, b, c, r, n); }
+extern "C" __global__ void KB c_rri(const long long* a, long long* b, long long* c, long long r, long long n) { unp::rowreduce<long long, unp::OP_PROD, unp::OP_MIN, 2, 2, 256, 8, false>(a, b, c, r, n); }
 extern "C" __global__ void KB c_ra(const double* a, double* b, long long n, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { unp::reduce_all<double, unp::OP_MEAN, 2, 256, 4>(a, b, n, p, k, e, w); }
-extern "C" __global__ void KB c_rn(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce_wave<float, unp::OP_MAXNUM, unp::OP_MINNUM, 2, 4, 256, 8>(a, b, c, r, n); }
+extern "C" __global__ void KB c_rn(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce_wave<float, unp::OP_MAXNUM, unp::OP_MINNUM, 2, 4, 256, 8, false>(a, b, c, r, n); }
 extern "C" __global__ void KB c_rx(const int* a, int* b, long long n, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { unp::reduce_all<int, unp::OP_XOR, 4, 256, 4>(a, b, n, p, k, e, w); }
 extern "C" __global__ void __launch_bounds__(512) c_rb(const long long* a, long long* b, unp::red_axes d, long long S, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { const long long* in[1] = {a}; unp::xreduce_inner<long long, 1, unp::OP_AND, unp::plain_ops<long long, unp::OP_AND>, 2, 8, 512, 8>(in, b, d, S, p, k, e, w); }
 extern "C" __global__ void __launch_bounds__(512) c_ro(const float* a, float* b, unp::red_axes d, long long S, int l, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { const float* in[1] = {a}; unp::xreduce_outer<float, 1, unp::OP_SUM, unp::plain_ops<float, unp::OP_SUM>, 4, 512, 8>(in, b, d, S, l, p, k, e, w); }

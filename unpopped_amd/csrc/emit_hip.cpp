@@ -342,9 +342,10 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
       L.entries.push_back(e);
     }
   } else {
-    // Rows up to kWideRow (32768) elements: one wave per row (no barrier); longer rows: one
-    // block per row with the LDS combine.  Both read the row once and stream it past the caches.
-    // Two blocks of four waves per CU (measured best for an 8192 x 4096 f32 row read).
+    // Rows up to kWideRow (32768) elements: one wave per row (no barrier); longer rows, or long ones (4096
+    // or more) that are no more than the CUs: one block per row with the LDS combine.  Both read the row once, in whole
+    // vectors at any alignment, and stream it past the caches.  Two blocks of four waves per CU
+    // (measured best for an 8192 x 4096 f32 row read); a block per row takes 16 waves.
     L.threads = 256;
     L.blocks_per_cu = 2;
     for (int wide = 0; wide <= 1; ++wide) {
@@ -352,13 +353,15 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
         Entry e;
         e.fast = fast;
         e.wide = wide;
-        e.vec = fast ? V : 1;
+        e.vec = V;
+        e.threads = wide ? 1024 : 256;
         e.symbol = L.name + (wide ? "_b" : "_w") + (fast ? "v" : "s");
-        const int unroll = wide ? (fast ? 4 : 8) : 16;
-        src << "extern \"C\" __global__ void __launch_bounds__(256) " << e.symbol << "(const " << T << "* in, " << T
-            << "* out0, " << T << "* out1, long long rows, long long cols) {\n  unp::"
+        const int unroll = wide ? 4 : 16;
+        src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << e.symbol << "(const " << T << "* in, "
+            << T << "* out0, " << T << "* out1, long long rows, long long cols) {\n  unp::"
             << (wide ? "rowreduce<" : "rowreduce_wave<") << T << ", " << f.op0 << ", " << (two ? f.op1 : f.op0) << ", "
-            << (two ? 2 : 1) << ", " << e.vec << ", 256, " << unroll << ">(in, out0, out1, rows, cols);\n}\n";
+            << (two ? 2 : 1) << ", " << e.vec << ", " << e.threads << ", " << unroll << (fast ? ", false" : ", true")
+            << ">(in, out0, out1, rows, cols);\n}\n";
         L.entries.push_back(e);
       }
     }
@@ -400,11 +403,12 @@ static int32_t lower_reduction(const unp_form& f, Lowered& L, std::string& why) 
         : (sched == 'm' || sched == 'g') ? split_policy(mask, f.rank)
         : sched == 'q' ? "one lane per output element, the reduced positions folded in the serial lift's "
                          "order (the serial accumulator, row-major over the reduced axes)"
-                       : "waves stride over rows (one wave per row); rows longer than 32768 elements: one block per row")
+                       : "waves stride over rows (one wave per row); rows longer than 32768 elements, or few long ones: one "
+                         "block per row")
     << "\"},\"entries\":[";
   for (size_t i = 0; i < L.entries.size(); ++i)
     j << (i ? "," : "") << "{\"symbol\":\"" << L.entries[i].symbol << "\",\"vec\":" << L.entries[i].vec
-      << ",\"when\":\"" << (L.entries[i].wide ? "reduced extent > 32768; " : "")
+      << ",\"when\":\"" << (L.entries[i].wide ? "reduced extent > 32768, or at least 4096 and a row per CU at most; " : "")
       << (L.entries[i].strided ? kStridedWhen
           : sched == 'q' ? "always"
           : (sched == 'm' || sched == 'g') ? split_when(L.entries[i])

@@ -475,9 +475,11 @@ template <class A> struct tagged {
 // Row reduction, one wave per row: waves stride over rows (the outermost kept axis, as
 // kernel_lift/block_reduce.rs:313-338 strides blocks over it); lane l folds the vectors
 // l, l + 64, ... of its row (U of them in flight), then the wave combines by DPP and lane 0
-// stores.  No LDS and no barrier: the schedule for rows up to a few thousand vectors.
+// stores.  No LDS and no barrier: the schedule for rows up to a few thousand vectors.  Without RAG
+// the rows are whole 16-byte-aligned vectors; RAG takes any (8192 x 4095 f32: 30.6 us, 41.2 element by
+// element; 8192 x 4096 whole: 22.2).
 // ---------------------------------------------------------------------------------------
-template <class T, int OP0, int OP1, int NOUT, int VEC, int THREADS, int U>
+template <class T, int OP0, int OP1, int NOUT, int VEC, int THREADS, int U, bool RAG>
 UNP_DEV void rowreduce_wave(const T* __restrict__ in, T* __restrict__ out0, T* __restrict__ out1, i64 rows,
                             i64 cols) {
   typedef typename acc<T, OP0>::type A0;
@@ -492,10 +494,10 @@ UNP_DEV void rowreduce_wave(const T* __restrict__ in, T* __restrict__ out0, T* _
     A0 a0 = F0::identity();
     A1 a1 = F1::identity();
     i64 c = (i64)lane * VEC;
-    for (; c + (U - 1) * STEP < cols; c += U * STEP) {
+    for (; c + (U - 1) * STEP + (RAG ? VEC - 1 : 0) < cols; c += U * STEP) {
       vec<T, VEC> v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = ld_nt<T, VEC>(p + c + u * STEP);
+      for (int u = 0; u < U; ++u) v[u] = RAG ? ld_any<T, VEC>(p + c + u * STEP) : ld_nt<T, VEC>(p + c + u * STEP);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
 #pragma unroll
@@ -505,12 +507,51 @@ UNP_DEV void rowreduce_wave(const T* __restrict__ in, T* __restrict__ out0, T* _
         }
       }
     }
-    for (; c < cols; c += STEP) {
-      const vec<T, VEC> v = ld_nt<T, VEC>(p + c);
+    if constexpr (RAG) {
+      if (cols < VEC) {  // less than a vector: an element per lane
+        if (lane < cols) {
+          a0 = F0::apply(a0, (A0)p[lane]);
+          if constexpr (NOUT > 1) a1 = F1::apply(a1, (A1)p[lane]);
+        }
+        c = cols;
+      }
+      // RAG, the rest: a vector that would run past the row starts at cols - VEC and ignores what the one
+      // before it held.  Four loads in flight, or one where one reaches the row's end.
+      auto rest = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        vec<T, VEC> v[N];
+        int skip[N];
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        a0 = F0::apply(a0, (A0)v.e[e]);
-        if constexpr (NOUT > 1) a1 = F1::apply(a1, (A1)v.e[e]);
+        for (int u = 0; u < N; ++u) {
+          const i64 w = c + u * STEP, at = w + VEC <= cols ? w : cols - VEC;
+          skip[u] = w < cols ? (int)(w - at) : VEC;
+          v[u] = ld_any<T, VEC>(p + at);
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            const A0 b0 = F0::apply(a0, (A0)v[u].e[e]);
+            a0 = e >= skip[u] ? b0 : a0;
+            if constexpr (NOUT > 1) {
+              const A1 b1 = F1::apply(a1, (A1)v[u].e[e]);
+              a1 = e >= skip[u] ? b1 : a1;
+            }
+          }
+        c += N * STEP;
+      };
+      while (c < cols) {
+        if (c + STEP >= cols) rest(ic<1>{});
+        else rest(ic<4>{});
+      }
+    } else {
+      for (; c < cols; c += STEP) {
+        const vec<T, VEC> v = ld_nt<T, VEC>(p + c);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          a0 = F0::apply(a0, (A0)v.e[e]);
+          if constexpr (NOUT > 1) a1 = F1::apply(a1, (A1)v.e[e]);
+        }
       }
     }
     a0 = wave_reduce<A0, OP0>(a0);
@@ -527,9 +568,10 @@ UNP_DEV void rowreduce_wave(const T* __restrict__ in, T* __restrict__ out0, T* _
 // once.  Blocks stride over rows (row = blockIdx.x; += gridDim.x), as the launched reduction
 // lift strides over its outermost kept axis (kernel_lift/block_reduce.rs:313-338).
 // Inside a row, thread t folds the vectors t, t + THREADS, ... (VEC elements each) in
-// ascending order; waves combine by DPP, blocks by LDS in wave order.
+// ascending order; waves combine by DPP, blocks by LDS in wave order.  28 rows of 66304 f32: 6.7 us with
+// 16 waves, 12.5 with four; 10 of 12160: 4.5 (the launch), 8.1 with a wave per row.
 // ---------------------------------------------------------------------------------------
-template <class T, int OP0, int OP1, int NOUT, int VEC, int THREADS, int UNROLL>
+template <class T, int OP0, int OP1, int NOUT, int VEC, int THREADS, int UNROLL, bool RAG>
 UNP_DEV void rowreduce(const T* __restrict__ in, T* __restrict__ out0, T* __restrict__ out1, i64 rows,
                        i64 cols) {
   typedef typename acc<T, OP0>::type A0;
@@ -547,10 +589,10 @@ UNP_DEV void rowreduce(const T* __restrict__ in, T* __restrict__ out0, T* __rest
     A0 a0 = F0::identity();
     A1 a1 = F1::identity();
     i64 c = (i64)tid * VEC;
-    for (; c + (UNROLL - 1) * STEP < cols; c += UNROLL * STEP) {
+    for (; c + (UNROLL - 1) * STEP + (RAG ? VEC - 1 : 0) < cols; c += UNROLL * STEP) {
       vec<T, VEC> v[UNROLL];
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) v[u] = ld_nt<T, VEC>(p + c + u * STEP);
+      for (int u = 0; u < UNROLL; ++u) v[u] = RAG ? ld_any<T, VEC>(p + c + u * STEP) : ld_nt<T, VEC>(p + c + u * STEP);
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
 #pragma unroll
@@ -560,12 +602,38 @@ UNP_DEV void rowreduce(const T* __restrict__ in, T* __restrict__ out0, T* __rest
         }
       }
     }
-    for (; c < cols; c += STEP) {
-      const vec<T, VEC> v = ld_nt<T, VEC>(p + c);
+    if constexpr (RAG) {
+      // Rows here are longer than a vector.
+      // The rest in one pass, as in rowreduce_wave.
+      if (c < cols) {
+        vec<T, VEC> v[UNROLL];
+        int skip[UNROLL];
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        a0 = F0::apply(a0, (A0)v.e[e]);
-        if constexpr (NOUT > 1) a1 = F1::apply(a1, (A1)v.e[e]);
+        for (int u = 0; u < UNROLL; ++u) {
+          const i64 w = c + u * STEP, at = w + VEC <= cols ? w : cols - VEC;
+          skip[u] = w < cols ? (int)(w - at) : VEC;
+          v[u] = ld_any<T, VEC>(p + at);
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            const A0 b0 = F0::apply(a0, (A0)v[u].e[e]);
+            a0 = e >= skip[u] ? b0 : a0;
+            if constexpr (NOUT > 1) {
+              const A1 b1 = F1::apply(a1, (A1)v[u].e[e]);
+              a1 = e >= skip[u] ? b1 : a1;
+            }
+          }
+      }
+    } else {
+      for (; c < cols; c += STEP) {
+        const vec<T, VEC> v = ld_nt<T, VEC>(p + c);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          a0 = F0::apply(a0, (A0)v.e[e]);
+          if constexpr (NOUT > 1) a1 = F1::apply(a1, (A1)v.e[e]);
+        }
       }
     }
     a0 = wave_reduce<A0, OP0>(a0);

@@ -1091,7 +1091,9 @@ int32_t run_reduction(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, un
   if ((rc = need_buffers(A, rows > 0, err)) != UNP_OK) return rc;
   if (rows == 0) return UNP_OK;
   uint64_t in = A.buf[0], o0 = A.buf[1], o1 = two ? A.buf[2] : A.buf[1];
-  const size_t entry = pick(x, cols % vec == 0 && aligned16(in), !x->l.reduce_all && cols > unp::kWideRow);
+  // A block of 16 waves per row where a wave each would leave CUs idle, or the rows are long.
+  const bool wide = !x->l.reduce_all && (cols > unp::kWideRow || (rows <= x->cu_count && cols >= 4096));
+  const size_t entry = pick(x, cols % vec == 0 && aligned16(in), wide);
   const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
   if (x->l.reduce_all) {
     // Up to two 8-byte tagged words per block partial.
