@@ -548,7 +548,9 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
   //  _v  rows of a multiple of 16 bytes, 16-byte aligned: the LDS-staged scan, one producer
   //      wave streaming the next tile into LDS by DMA plus NC consumer waves, one block per
   //      CU (two LDS buffers of one 72 KiB tile each);
-  //  _s  anything else: the register scan, one element per lane-vector.
+  //  _s  anything else: the register scan, 16384-element tiles in 16-byte vectors at any alignment.
+  // Rows of at most 1024 and 16384 elements of 4 bytes (half as many of 8) fit a wave's or a block's
+  // registers and take _r1 and _r8 instead.
   // Measured on MI355X at 2^28 i32 / 2^26 f32: a 4-byte carry runs best with 6 consumer waves
   // of K = 12 vectors, an 8-byte carry (f32 Sum in f64, F64, I64) on the device schedule with 4
   // waves of K = 18, and on the fixed schedule with 6 waves of K = 12 (its grouped look-back
@@ -578,18 +580,33 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
   {
     Entry e;
     e.fast = false;
-    e.vec = 1;
-    e.k = wide_carry ? 16 : 32;
+    e.vec = vec16;
     e.wpb = wide_carry ? 16 : 8;
+    e.k = 16384 / (64 * vec16 * e.wpb);
     e.threads = 64 * e.wpb;
     e.blocks_per_cu = wide_carry ? 1 : 3;
     e.symbol = L.name + "_s";
     src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << e.symbol << "(const " << T
         << "* in, " << T << "* out, long long rows, long long cols, unsigned long long* status, "
         << "unsigned* counter, unsigned ticket_base, unsigned epoch, unp::waits wt) {\n  unp::scan_lookback<" << T << ", " << f.op0
-        << ", " << (f.exclusive ? "true" : "false") << ", " << (f.reverse ? "true" : "false") << ", 1, " << e.k
+        << ", " << (f.exclusive ? "true" : "false") << ", " << (f.reverse ? "true" : "false") << ", " << e.vec << ", " << e.k
         << ", " << e.wpb << ", " << kScanStatusWords << (fixed ? ", true" : "")
         << ">(in, out, rows, cols, status, counter, ticket_base, epoch, wt);\n}\n";
+    L.entries.push_back(e);
+  }
+  for (int wpr : {1, 8}) {
+    Entry e;
+    e.team = true;
+    e.vec = vec16;
+    e.k = wpr == 1 ? 4 : 8;
+    e.wpb = wpr;
+    e.threads = wpr == 1 ? 256 : 512;
+    e.blocks_per_cu = wpr == 1 ? 8 : 4;
+    e.symbol = L.name + "_r" + std::to_string(wpr);
+    src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << e.symbol << "(const " << T << "* in, "
+        << T << "* out, long long rows, long long cols) {\n  unp::scan_rows<" << T << ", " << f.op0 << ", "
+        << (f.exclusive ? "true" : "false") << ", " << (f.reverse ? "true" : "false") << ", " << e.vec << ", " << e.k << ", "
+        << e.wpb << ", " << e.threads << ">(in, out, rows, cols);\n}\n";
     L.entries.push_back(e);
   }
   src << scan_strided_entry(f, L);
@@ -605,15 +622,24 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
   for (int d = 0; d < f.rank; ++d) j << ",{\"name\":\"n" << d << "\",\"kind\":\"scalar\",\"dtype\":\"I32\"}";
   j << "],\"launch\":{\"block\":[" << L.threads << ",1,1],\"grid\":\"cu_count*" << L.blocks_per_cu
     << "\",\"grid_policy\":\"persistent blocks draw one block-tile ticket per round\"},\"entries\":[";
-  for (size_t i = 0; i < L.entries.size(); ++i)
-    j << (i ? "," : "") << "{\"symbol\":\"" << L.entries[i].symbol << "\",\"vec\":" << L.entries[i].vec
-      << ",\"k\":" << L.entries[i].k << ",\"waves\":" << L.entries[i].wpb
-      << ",\"block\":" << L.entries[i].threads << ",\"blocks_per_cu\":" << L.entries[i].blocks_per_cu
-      << ",\"block_tile\":" << 64 * L.entries[i].vec * L.entries[i].k * L.entries[i].wpb << ",\"when\":\""
-      << (L.entries[i].strided ? kStridedWhen
-          : L.entries[i].fast  ? "scanned extent % vec == 0 and in0/out 16-byte aligned"
-                               : "otherwise")
-      << "\"}";
+  auto list = [&](bool rows) {
+    bool first = true;
+    for (const Entry& e : L.entries) {
+      if (e.team != rows) continue;
+      j << (first ? "" : ",") << "{\"symbol\":\"" << e.symbol << "\",\"vec\":" << e.vec << ",\"k\":" << e.k
+        << ",\"waves\":" << e.wpb << ",\"block\":" << e.threads << ",\"blocks_per_cu\":" << e.blocks_per_cu
+        << ",\"block_tile\":" << 64 * e.vec * e.k * e.wpb << ",\"when\":\""
+        << (e.strided ? kStridedWhen
+            : e.team  ? "scanned extent at most block_tile (the first such entry)"
+            : e.fast  ? "scanned extent % vec == 0 and in0/out 16-byte aligned"
+                      : "otherwise")
+        << "\"}";
+      first = false;
+    }
+  };
+  list(false);
+  j << "],\"row_entries\":[";
+  list(true);
   j << "],\"workspace\":{\"status\":\"tiles * " << kScanStatusWords * 8
     << " bytes, zeroed once\",\"counter\":4,\"stall\":4,\"host_state\":[\"epoch\",\"ticket_base\"]}"
     << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"
@@ -624,7 +650,8 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
                       "association the tile size alone fixes: the same bits on every launch and any grid for one entry. "
                       "The entry follows from the row length and the buffers' alignment: rows of whole 16-byte vectors at "
                       "16-byte-aligned addresses take the staged entry (18432-element tiles), others the register entry "
-                      "(16384-element tiles), whose bits may differ; a strided view runs the serial order. Float Sum / "
+                      "(16384-element tiles), whose bits may differ, and rows that fit a wave's or a block's registers "
+                      "the row entries, whatever their alignment; a strided view runs the serial order. Float Sum / "
                       "Mean fold in f64 within the declared per-prefix bound gamma_(n-1)*sum|x| + 1/2 ulp; Max/Min keep one "
                       "NaN payload and zero sign launch to launch"
                 : kind_is_float(f.dtype) && (f.op0 == UNP_OP_SUM || f.op0 == UNP_OP_MEAN)

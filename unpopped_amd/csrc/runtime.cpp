@@ -906,12 +906,12 @@ int32_t launch(unp_exec* x, size_t entry, uint32_t grid, void** params, hipStrea
 size_t pick(const unp_exec* x, bool fast_ok, bool wide = false) {
   const std::vector<unp::Entry>& es = x->l.entries;
   for (size_t i = 0; i < es.size(); ++i)
-    if (!es[i].strided && es[i].fast == fast_ok && es[i].wide == wide) return i;
+    if (!es[i].strided && !es[i].team && es[i].fast == fast_ok && es[i].wide == wide) return i;
   for (size_t i = 0; i < es.size(); ++i)
-    if (!es[i].strided && !es[i].fast && es[i].wide == wide) return i;
+    if (!es[i].strided && !es[i].team && !es[i].fast && es[i].wide == wide) return i;
   size_t last = 0;
   for (size_t i = 0; i < es.size(); ++i)
-    if (!es[i].strided) last = i;
+    if (!es[i].strided && !es[i].team) last = i;
   return last;
 }
 
@@ -1200,6 +1200,13 @@ int32_t run_scan(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_err
   if (rows == 0 || cols == 0) return UNP_OK;
   const int vec = 16 / (int)unp::kind_bytes(f.dtype);
   uint64_t in = A.buf[0], out = A.buf[1];
+  // A row that fits the registers of a wave, else of a block, needs no tiles.
+  for (size_t i = 0; i < x->l.entries.size(); ++i) {
+    const unp::Entry& en = x->l.entries[i];
+    if (!en.team || cols > 64LL * en.vec * en.k * en.wpb) continue;
+    void* params[] = {&in, &out, &rows, &cols};
+    return launch(x, i, (uint32_t)(x->cu_count * en.blocks_per_cu), params, s, err);
+  }
   const size_t entry = pick(x, cols % vec == 0 && aligned16(in) && aligned16(out));
   const unp::Entry& en = x->l.entries[entry];
   // A block tile: wpb (consumer) waves x 64 lanes x vec x k positions of one row.

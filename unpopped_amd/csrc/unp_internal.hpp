@@ -31,7 +31,7 @@ struct Entry {
   int threads = 0;    // block size of this entry (0: the form's)
   int blocks_per_cu = 0;  // persistent blocks per CU of this entry (0: the form's)
   bool team = false;      // split reduction, innermost run reduced: a wave per output; elementwise: the
-                          // tiled entry (vec: its tile's rows)
+                          // tiled entry (vec: its tile's rows); scan: a row in registers
   int cols = 0;           // output columns per block (dequant GEMM decode entries)
   // Reads and writes its buffers through storage-image strides (unp_hip_exec_launch_views with a
   // view that is not dense row-major); never picked for a pointer launch.
