@@ -1360,13 +1360,13 @@ UNP_DEV void scan_seq(const T* __restrict__ in, T* __restrict__ out, i64 A, i64 
 // columns per block, its rows streamed through a ring of LDS tiles.  The serial order leaves a
 // column one chain of S folds, so one wave (lanes on columns) runs nothing but that chain, out of
 // LDS, while NM mover waves keep the rows coming and going: a lane that loads its own rows waits
-// for memory once per group of loads instead.  2048 x 3000 f32: 34.5 us, 111.6 with scan_seq; 4096 x
-// 8192: 66 us (4.0 TB/s), 355.  What bounds a few strips is the chain: a conversion, an add and a
+// for memory once per group of loads instead.  2048 x 3000 f32: 30.0 us, 111.6 with scan_seq; 4096 x
+// 8192: 67 us (4.0 TB/s), 355.  What bounds a few strips is the chain: a conversion, an add and a
 // conversion in f64 per row, 11 to 12 ns.  From about four strips per CU on a lane per column keeps
 // as much in flight (16 x 300 x 5000: 55 us here, 53 there; 32 x 100 x 8001: 74, 51).
 //
 // Tiles of 16 KiB (64 rows of 4-byte elements) follow each other through NB buffers, across the
-// block's strips (strip = blockIdx.x, += gridDim.x) without a break.  Round r:
+// block's strips (+= gridDim.x) without a break.  Round r:
 //   movers  issue the global->LDS DMA of tile r + D, store tile r - 1, and wait until tile r + 1 has
 //           landed (every tile issues the same operations, clamped to its last row, so the wait is
 //           an exact count that leaves the younger tiles in flight);
@@ -1410,7 +1410,12 @@ UNP_DEV void scan_cols(const T* __restrict__ in, T* __restrict__ out, i64 S, i64
   static_assert((D - 1) * DMA + D * ST < 64, "the wait counts fit vmcnt");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const i64 nt = (S + TR - 1) / TR;
-  const i64 mine = nstrips > blockIdx.x ? (nstrips - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;
+  // Blocks go to the eight XCDs in turn.  Strips that all run at once are dealt out so that neighbours
+  // share an XCD, and the rows are read through its L2: where rows are not whole cache lines, a line
+  // of two strips is then fetched once (2048 x 3000 f32: 30.0 us; 34.8 otherwise).
+  const i64 per_xcd = (nstrips + 7) / 8, slot = blockIdx.x / 8;
+  const i64 first_strip = nstrips >= gridDim.x ? (i64)blockIdx.x : slot < per_xcd ? blockIdx.x % 8 * per_xcd + slot : nstrips;
+  const i64 mine = nstrips > first_strip ? (nstrips - first_strip + gridDim.x - 1) / gridDim.x : 0;
   const i64 N = mine * nt;  // this block's tiles
   if (N == 0) return;
   struct Cursor {  // a tile: its strip, its number in the strip and its buffer
@@ -1424,7 +1429,7 @@ UNP_DEV void scan_cols(const T* __restrict__ in, T* __restrict__ out, i64 S, i64
     }
     c.b = c.b + 1 == NB ? 0 : c.b + 1;
   };
-  const Cursor first = {(i64)blockIdx.x, 0, 0};
+  const Cursor first = {first_strip, 0, 0};
 
   if (wave < NM) {
     const divisor by_ncb(ncb);
@@ -1460,9 +1465,9 @@ UNP_DEV void scan_cols(const T* __restrict__ in, T* __restrict__ out, i64 S, i64
         // Groups past the row (their column is clamped too) are skipped only where an operation also
         // covers the first group: one without a live lane would not be issued, and the count be off.
         if constexpr (WIDE) {
-          if (llive) __builtin_amdgcn_global_load_lds(p, to, 16, 0, 2 /* nt */);
+          if (llive) __builtin_amdgcn_global_load_lds(p, to, 16, 0, 0);
         } else {
-          __builtin_amdgcn_global_load_lds(reinterpret_cast<const u8*>(p) + lane * LB % 16, to, 4, 0, 2);
+          __builtin_amdgcn_global_load_lds(reinterpret_cast<const u8*>(p) + lane * LB % 16, to, 4, 0, 0);
         }
         lo[k] += stride;
       }
