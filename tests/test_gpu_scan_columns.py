@@ -45,3 +45,18 @@ def test_every_prefix_is_the_serial_ones(hip_device, a, s, b, dtype, op, exclusi
         ex.launch(buf.at(shift), buf.at(shift), a, s, b)
         u.synchronize()
         assert np.array_equal(buf.at(shift).download(NT[dtype], x.size).reshape(x.shape), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype,reverse", [("F32", False), ("I32", True), ("I64", False)])
+def test_in_place_with_a_last_strip_of_less_than_a_vector(hip_device, dtype, reverse):
+    """257 strips over 256 blocks: the last one, a single column wide, runs after its neighbour has stored."""
+    a, s, b = 1, 600, 64 * 256 + 1
+    x = values(dtype, a * s * b).reshape(s, b)
+    want = oracle.scan_rows(np.ascontiguousarray(x.T), "Sum", False, reverse).T
+    ex = H.executor(kind="scan", dtype=dtype, rank=3, op="Sum", axis=1, exclusive=False, reverse=reverse)
+    H.say(f"[case] column scan in place {a}x{s}x{b} {dtype} reverse={reverse}")
+    buf = u.DeviceBuffer(x.nbytes)
+    buf.upload(x)
+    ex.launch(buf, buf, a, s, b)
+    u.synchronize()
+    assert np.array_equal(buf.download(NT[dtype], x.size).reshape(x.shape), want)

@@ -1183,10 +1183,13 @@ int32_t run_scan(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_err
     uint64_t in = A.buf[0], out = A.buf[1];
     const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
     // Up to four strips of 64 columns per CU stream through LDS (rows of at least half a strip); more
-    // columns than that keep enough loads in flight with a lane each.
-    const long long ncb = (b0 + 63) / 64, strips = a0 * ncb;
-    if (b0 >= 32 && S >= 16 && strips <= 4LL * x->cu_count) {
-      int32_t wide = b0 % (16 / (long long)unp::kind_bytes(f.dtype)) == 0 && aligned16(in);
+    // columns than that keep enough loads in flight with a lane each.  A last strip of less than a
+    // vector also scans columns of the strip before it, which in place that strip's block may have
+    // stored already: those launches go by columns too.
+    const long long ncb = (b0 + 63) / 64, strips = a0 * ncb, vec = 16 / (long long)unp::kind_bytes(f.dtype);
+    const bool torn = in == out && b0 % 64 > 0 && b0 % 64 < vec;
+    if (b0 >= 32 && S >= 16 && strips <= 4LL * x->cu_count && !torn) {
+      int32_t wide = b0 % vec == 0 && aligned16(in);
       long long n = strips, c = ncb;
       void* params[] = {&in, &out, &S, &b0, &n, &c, &wide};
       return launch(x, 1, grid, params, s, err);
