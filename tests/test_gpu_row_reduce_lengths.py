@@ -64,3 +64,23 @@ def test_two_inputs_nan_and_infinities_in_chunks(hip_device):
     with np.errstate(all="ignore"):
         want = oracle.row_reduce([a, b], stages, epi)
     assert np.array_equal(H.row_reduce([a, b], stages, epi), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("cols", [257, 1281, 4353, 8193])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_in_place_on_an_input_only_the_epilogue_reads(hip_device, cols, dtype):
+    """Ragged rows whose shifted last vector begins a wave: the elements it shares are another wave's, which
+    may have stored them before this one loads them."""
+    if dtype == np.float64:
+        cols = cols // 2 + 1  # the same vector of 2
+    r = np.random.default_rng(43)
+    rows = 700
+    a, b = (r.integers(-8, 9, (rows, cols)).astype(dtype) for _ in range(2))
+    stages = [(X.input(0), "Sum")]
+    epi = X.input(1) * X.konst(3.0) + X.reduced(0)
+    ex = H.row_reduce_executor(H.NP_KIND[dtype], 2, stages, epi, n_inputs=2)
+    H.say(f"[case] row_reduce in place on the epilogue's input {rows}x{cols} {np.dtype(dtype).name}")
+    da, db = u.DeviceBuffer.from_array(a), u.DeviceBuffer.from_array(b)
+    ex.launch(da, db, db, rows, cols)
+    u.synchronize()
+    assert np.array_equal(db.download(dtype, b.size).reshape(b.shape), oracle.row_reduce([a, b], stages, epi))

@@ -3918,6 +3918,15 @@ UNP_DEV void rr_stage(const T* const* rin, const vec<T, VEC> (&xr)[NI][R > 0 ? R
         fold_vec(xv, 0);
       }
     }
+    if constexpr (RAG && R > 0 && S + 1 == NS) {
+      // A shifted last vector shares elements with another lane's, and in place that lane may be in a wave
+      // that stores first: every input of the row has landed in this wave, also one that only the
+      // epilogue reads, before the last barrier lets any wave on to its stores.
+#pragma unroll
+      for (int k = 0; k < NI; ++k)
+#pragma unroll
+        for (int q = 0; q < R; ++q) asm volatile("" ::"v"(__builtin_bit_cast(u32x4_t, xr[k][q])));
+    }
     acc = wave_reduce<double, OP>(acc);
     if (lane == 0) part[wave] = acc;
     __syncthreads();
