@@ -2,12 +2,14 @@
 and their ragged last groups, tiles' last rows, several strips per block, unaligned buffers, in place."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle
 import unpopped_amd as u
-from unpopped_amd import forms as H, synth
+from unpopped_amd import _lib, forms as H, synth
 
 pytestmark = pytest.mark.gpu
 NT = {"F32": np.float32, "F64": np.float64, "I32": np.int32, "I64": np.int64}
@@ -60,3 +62,33 @@ def test_in_place_with_a_last_strip_of_less_than_a_vector(hip_device, dtype, rev
     ex.launch(buf, buf, a, s, b)
     u.synchronize()
     assert np.array_equal(buf.download(NT[dtype], x.size).reshape(x.shape), want)
+
+
+@pytest.mark.parametrize("grid,strips", [(250, 249), (252, 251), (256, 249), (7, 6), (250, 600)])
+def test_every_strip_is_scanned_at_any_grid(hip_device, grid, strips):
+    """The entry launched by hand on grids that are and are not multiples of the eight XCDs."""
+    s, b = 16, 64 * strips
+    x = values("I32", s * b).reshape(s, b)
+    g = u.HipBackend().lower_kernel(H.kernel_for(kind="scan", dtype="I32", rank=3, op="Sum", axis=1))
+    symbol = g.name + "_c"
+    L, m, f, err = _lib.lib(), C.c_void_p(), C.c_void_p(), _lib.Error()
+    co = u.HipCompiler().compile(g.source, g.name)
+    img = C.create_string_buffer(co, len(co))
+    _lib.check(L.unp_hip_module_load(img, len(co), C.byref(m), C.byref(err)), err)
+
+    class Args(C.Structure):
+        _fields_ = [("src", C.c_uint64), ("dst", C.c_uint64), ("S", C.c_int64), ("B", C.c_int64),
+                    ("nstrips", C.c_int64), ("ncb", C.c_int64), ("wide", C.c_int32)]
+
+    try:
+        _lib.check(L.unp_hip_get_function(m, symbol.encode(), C.byref(f), C.byref(err)), err)
+        src, dst = u.DeviceBuffer.from_array(x), u.DeviceBuffer(x.nbytes)
+        dst.fill(0x5A)
+        a = Args(src.ptr, dst.ptr, s, b, strips, strips, 1)
+        H.say(f"[case] column scan by hand, {strips} strips on {grid} blocks")
+        _lib.check(L.unp_hip_launch(f, (C.c_uint32 * 3)(grid, 1, 1), (C.c_uint32 * 3)(576, 1, 1), 0, None, C.byref(a),
+                                    C.sizeof(a), C.byref(err)), err)
+        u.synchronize()
+        assert np.array_equal(dst.download(np.int32, x.size).reshape(s, b), np.cumsum(x, axis=0, dtype=np.int32))
+    finally:
+        L.unp_hip_module_unload(m)

@@ -1412,9 +1412,11 @@ UNP_DEV void scan_cols(const T* __restrict__ in, T* __restrict__ out, i64 S, i64
   const i64 nt = (S + TR - 1) / TR;
   // Blocks go to the eight XCDs in turn.  Strips that all run at once are dealt out so that neighbours
   // share an XCD, and the rows are read through its L2: where rows are not whole cache lines, a line
-  // of two strips is then fetched once (2048 x 3000 f32: 30.0 us; 34.8 otherwise).
+  // of two strips is then fetched once (2048 x 3000 f32: 30.0 us; 34.8 otherwise).  A grid that is no
+  // multiple of eight has XCDs with a block less than that deal needs, and takes the strips in turn.
   const i64 per_xcd = (nstrips + 7) / 8, slot = blockIdx.x / 8;
-  const i64 first_strip = nstrips >= gridDim.x ? (i64)blockIdx.x : slot < per_xcd ? blockIdx.x % 8 * per_xcd + slot : nstrips;
+  const bool in_turn = nstrips >= gridDim.x || gridDim.x % 8 != 0;
+  const i64 first_strip = in_turn ? (i64)blockIdx.x : slot < per_xcd ? blockIdx.x % 8 * per_xcd + slot : nstrips;
   const i64 mine = nstrips > first_strip ? (nstrips - first_strip + gridDim.x - 1) / gridDim.x : 0;
   const i64 N = mine * nt;  // this block's tiles
   if (N == 0) return;
