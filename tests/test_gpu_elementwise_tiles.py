@@ -51,3 +51,32 @@ def test_a_transposition_moves_bits(hip_device, dtype, nt):
         H.say(f"[case] transposition {rows}x{cols} {dtype}")
         got, entry = run(k, [x], (rows, cols), nt)
         assert entry.endswith("_t_e") and got.tobytes() == np.ascontiguousarray(x.T).tobytes()
+
+
+# (output shape, the second input's permutation): tiles mostly inside the extents, with ragged edges on
+# either axis, the second axis turned or not, next to the first or not; then tiles mostly outside, and
+# planes of fewer tiles than CUs.
+ENTRIES = [
+    ((65, 130), [1, 0], "_t_e"), ((130, 65), [1, 0], "_t_e"), ((300, 40), [1, 0], "_t_e"), ((16, 1000), [1, 0], "_t_e"),
+    ((16, 20, 60, 40), [0, 2, 1, 3], "_t_e"), ((60, 300, 33), [1, 0, 2], "_t_e"), ((64, 300, 17), [2, 1, 0], "_t_e"),
+    ((40, 33, 20, 70), [3, 1, 2, 0], "_t_e"), ((300, 60, 65), [1, 0, 2], "_t_e"), ((64, 300, 28), [1, 0, 2], "_t_e"),
+    ((66, 300, 17), [2, 1, 0], "_e"), ((64, 300, 24), [1, 0, 2], "_e"), ((3, 5000), [1, 0], "_e"),
+    ((5000, 17), [1, 0], "_e"), ((5000, 2, 16), [1, 0, 2], "_e"), ((5000, 2, 16), [0, 2, 1], "_e"),
+    ((300, 3, 3, 65), [0, 2, 1, 3], "_e"), ((64, 2, 64), [1, 0, 2], "_e"),
+]
+
+
+@pytest.mark.parametrize("shape,perm,entry", ENTRIES)
+def test_the_entry_follows_the_tiles_share_inside(hip_device, shape, perm, entry):
+    r = np.random.default_rng(33)
+    other = [0] * len(shape)
+    for d, a in enumerate(perm):
+        other[a] = shape[d]
+    ins = [r.normal(size=shape).astype(np.float32), r.normal(size=other).astype(np.float32)]
+    body = {"Sub": [I(0), I(1)]}
+    k = u.lift_elementwise("tiles", "F32", len(shape), body, n_inputs=2, perms=[list(range(len(shape))), perm],
+                           launch=(256, 16))
+    H.say(f"[case] elementwise entry {shape} {perm}")
+    got, ran = run(k, ins, shape, np.float32)
+    assert np.array_equal(got, ins[0] - ins[1].transpose(perm))
+    assert ran == u.HipBackend().lower_kernel(k).name + entry

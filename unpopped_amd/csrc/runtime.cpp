@@ -1402,9 +1402,19 @@ int32_t run_gather(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_e
 
 // The tiled entry's descriptor for strided buffers, if its tiles suit them: an output axis of stride 1
 // and at least 16 elements (D0), and a second axis (J): the one along which the inputs that are not
-// of stride 1 (or 0) along D0 have it, when it has 16 elements too, else the next one outwards.
+// of stride 1 (or 0) along D0 have it, when it has 16 elements too, else the longest other one.
 // Axes of extent 1 are dropped and adjacent axes that every buffer walks as one are merged.
-bool tile_axes(const unp::gather_x_view_host& v, size_t ni, int tj, unp::ew_tile_view_host& d) {
+//
+// A tile costs the same however little of it lies inside the extents: over 4 M elements of two f32
+// inputs and an output the tiled entry takes about 5 + 5.2 / u us, u the share of its elements that
+// is inside.  The strided entry takes 19 us where the inputs are read along D0 (24 x 20833 columns,
+// u = 3/8: 18.9 tiled, 19.1 strided; 16: 26.7, 19.7) and 15 to 27 where the axis next to a short D0
+// is turned, whose lines it finds in its caches (N x 24: 19.1, 16.6; N x 28: 16.5, 17.8); where another
+// axis is turned 26 to 30 (f64 48; u = 1/4: 27.5 and 32 tiled), and down the columns of a long D0 24 to
+// 73 (16 x 250000, u = 1/4: 23.9 tiled, 38.9).  A transposition of one input breaks even lower (N x 24:
+// 12.7 and 14.2).  Planes of fewer tiles than CUs go to the strided entry too, whose lanes are on all of
+// them (8 x 187 x 100: 4.2 us, 5.2 tiled).
+bool tile_axes(const unp::gather_x_view_host& v, size_t ni, int tj, int cus, unp::ew_tile_view_host& d) {
   std::vector<std::vector<long long>> ax;  // per merged axis: extent, output stride, input strides
   for (long long a = 0; a < v.rank; ++a) {
     std::vector<long long> x{v.ext[a], v.ostr[a]};
@@ -1428,13 +1438,18 @@ bool tile_axes(const unp::gather_x_view_host& v, size_t ni, int tj, unp::ew_tile
         d.tr |= 1u << k;
       }
   }
-  if (j == ax.size()) j = d0 > 0 ? d0 - 1 : d0 + 1;
+  const bool turned = j != ax.size();
+  for (size_t a = 0; !turned && a < ax.size(); ++a)
+    if (a != d0 && (j == ax.size() || ax[a][0] >= ax[j][0])) j = a;
   d.e0 = ax[d0][0];
   d.ej = ax[j][0];
   d.oj = ax[j][1];
   for (size_t k = 0; k < ni; ++k) d.i0[k] = ax[d0][2 + k], d.ij[k] = ax[j][2 + k];
   d.t0 = (d.e0 + 63) / 64;
   d.tj = (d.ej + tj - 1) / tj;
+  const double inside = (double)(d.e0 * d.ej) / ((double)(d.t0 * 64) * (double)(d.tj * tj));
+  const double cached = ni == 1 ? 0.33 : 0.375;  // the least share where the strided entry's lines are reused
+  if (inside <= (!turned ? cached : d.e0 >= 64 ? 0.2 : j + 1 == d0 ? cached : 0.249)) return false;
   d.items = d.t0 * d.tj;
   for (size_t a = 0; a < ax.size(); ++a) {
     if (a == d0 || a == j) continue;
@@ -1445,6 +1460,7 @@ bool tile_axes(const unp::gather_x_view_host& v, size_t ni, int tj, unp::ew_tile
     d.items *= ax[a][0];
     ++d.n;
   }
+  if (d.n > 0 && d.items < cus) return false;
   d.inv_t0 = 1.0 / (double)d.t0;
   d.inv_tj = 1.0 / (double)d.tj;
   return true;
@@ -1460,7 +1476,7 @@ int32_t launch_elementwise_strided(unp_exec* x, const std::vector<uint64_t>& ptr
   for (auto& q : p) params.push_back(&q);
   unp::ew_tile_view_host tv;
   const size_t tiled = x->l.entries.size() - 1;
-  if (tile_axes(v, ptrs.size() - 1, x->l.entries[tiled].vec, tv)) {
+  if (tile_axes(v, ptrs.size() - 1, x->l.entries[tiled].vec, x->cu_count, tv)) {
     params.push_back(&tv);
     return launch(x, tiled, (uint32_t)std::min<long long>(tv.items, (long long)x->cu_count * x->l.blocks_per_cu),
                   params.data(), s, err);
