@@ -100,3 +100,33 @@ def test_without_a_workspace_the_bits_are_the_same(hip_device, shape, axes):
     assert L.hipGraphExecDestroy(exe) == 0 and L.hipGraphDestroy(graph) == 0
     for st in streams:
         assert L.hipStreamDestroy(st) == 0
+
+
+# (shape, reduced axes, the entry's tail): few positions under many outputs go a lane per output or vector
+# of columns (fewer elements than a vector, ragged, one and several reduced axes, remainders of the eight
+# in flight), strips of few rows a wave each.
+SHORT = [
+    ((100000, 3, 5), (1,), "mlv"), ((60000, 9, 3), (1,), "mls"), ((70000, 4, 6), (1,), "mlv"),
+    ((3, 30000, 3, 7), (0, 2), "mlv"), ((13, 260001), (0,), "mlv"), ((70000, 1, 4), (1,), "mlv"),
+    ((2, 100000, 2), (0, 2), "gls"), ((3, 60000, 5), (0, 2), "glv"), ((4, 100000, 8), (0, 2), "glv"),
+    ((2, 300, 2, 300, 5), (0, 2, 4), "glv"), ((1, 90001, 9), (0, 2), None),
+    ((1229, 59, 3), (1,), "mws"), ((1130, 47, 4), (1,), "mwv"), ((2000, 100, 7), (1,), "mwv"),
+    ((4, 900, 10, 33), (0, 2), "mwv"), ((1000, 64, 17), (1,), "mwv"),
+    ((1000, 1000, 4), (0, 2), "gwv"), ((2, 4096, 64), (0, 2), "gwv"),
+]
+
+
+@pytest.mark.parametrize("shape,axes,entry", SHORT)
+@pytest.mark.parametrize("dtype", ["F32", "I64"])
+def test_short_reductions_by_lanes_and_waves(hip_device, shape, axes, entry, dtype):
+    nt = {"F32": np.float32, "I64": np.int64}[dtype]
+    x = data(shape, nt)
+    H.say(f"[case] short reduction {shape} over {axes} {dtype}")
+    want = x.astype(np.int64).sum(axis=axes).astype(nt)
+    assert np.array_equal(H.reduce_axes(x, axes, "Sum"), want)
+    ran = H.executor(kind="reduction", dtype=dtype, rank=x.ndim, op="Sum", axes=axes, keepdim=False).last_launch()
+    if dtype == "F32" and entry is not None:
+        assert ran["entry"].rsplit("_", 1)[1] == entry
+    got = H.reduce_expr([x, x], axes, "Sum", X.input(0) * X.input(1)) if dtype == "F32" else None
+    if got is not None:
+        assert np.array_equal(got, (x.astype(np.int64) ** 2).sum(axis=axes).astype(nt))

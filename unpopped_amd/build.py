@@ -85,7 +85,7 @@ CHECK_INSTANTIATIONS = r"""
 #include "unp_device.hip"
 #define KB __launch_bounds__(256)
 // The descriptors the host passes by value (runtime.cpp asserts the same sizes for its images).
-static_assert(sizeof(unp::red_axes) == 54 * 8, "red_axes");
+static_assert(sizeof(unp::red_axes) == 59 * 8, "red_axes");
 static_assert(sizeof(unp::red_view) == 44 * 8, "red_view");
 static_assert(sizeof(unp::scan_view) == 29 * 8, "scan_view");
 static_assert(sizeof(unp::gather_view) == 35 * 8, "gather_view");
@@ -96,8 +96,11 @@ extern "C" __global__ void KB c_rri(const long long* a, long long* b, long long*
 extern "C" __global__ void KB c_ra(const double* a, double* b, long long n, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { unp::reduce_all<double, unp::OP_MEAN, 2, 256, 4>(a, b, n, p, k, e, w); }
 extern "C" __global__ void KB c_rn(const float* a, float* b, float* c, long long r, long long n) { unp::rowreduce_wave<float, unp::OP_MAXNUM, unp::OP_MINNUM, 2, 4, 256, 8, false>(a, b, c, r, n); }
 extern "C" __global__ void KB c_rx(const int* a, int* b, long long n, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { unp::reduce_all<int, unp::OP_XOR, 4, 256, 4>(a, b, n, p, k, e, w); }
-extern "C" __global__ void __launch_bounds__(512) c_rb(const long long* a, long long* b, unp::red_axes d, long long S, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { const long long* in[1] = {a}; unp::xreduce_inner<long long, 1, unp::OP_AND, unp::plain_ops<long long, unp::OP_AND>, 2, 8, 512, 8>(in, b, d, S, p, k, e, w); }
-extern "C" __global__ void __launch_bounds__(512) c_ro(const float* a, float* b, unp::red_axes d, long long S, int l, unsigned long long* p, unsigned* k, unsigned e, unp::waits w) { const float* in[1] = {a}; unp::xreduce_outer<float, 1, unp::OP_SUM, unp::plain_ops<float, unp::OP_SUM>, 4, 512, 8>(in, b, d, S, l, p, k, e, w); }
+extern "C" __global__ void __launch_bounds__(512) c_rb(const long long* a, long long* b, unsigned long long* p, unsigned* k, unsigned e, unp::waits w, unp::red_axes d) { const long long* in[1] = {a}; unp::xreduce_inner<long long, 1, unp::OP_AND, unp::plain_ops<long long, unp::OP_AND>, 2, 8, 512, 8>(in, b, p, k, e, w, d); }
+extern "C" __global__ void __launch_bounds__(512) c_ro(const float* a, float* b, unsigned long long* p, unsigned* k, unsigned e, unp::waits w, unp::red_axes d) { const float* in[1] = {a}; unp::xreduce_outer<float, 1, unp::OP_SUM, unp::plain_ops<float, unp::OP_SUM>, 4, 512, 8>(in, b, p, k, e, w, d); }
+extern "C" __global__ void __launch_bounds__(512) c_rs(const double* a, double* b, unp::red_axes d) { const double* in[1] = {a}; unp::xreduce_outer_wave<double, 1, unp::OP_SUM, unp::plain_ops<double, unp::OP_SUM>, 2, 512, 8>(in, b, d); }
+extern "C" __global__ void KB c_rl(const float* a, float* b, unp::red_axes d) { const float* in[1] = {a}; unp::xreduce_lanes<float, 1, unp::OP_SUM, unp::plain_ops<float, unp::OP_SUM>, 4, true, 256>(in, b, d); }
+extern "C" __global__ void KB c_rm(const double* a, double* b, unp::red_axes d) { const double* in[1] = {a}; unp::xreduce_lanes<double, 1, unp::OP_MAX, unp::plain_ops<double, unp::OP_MAX>, 2, false, 256>(in, b, d); }
 extern "C" __global__ void KB c_rq(const float* a, float* b, unp::red_view d) { unp::reduce_serial<float, unp::OP_MAXNUM, 256>(a, b, d); }
 extern "C" __global__ void KB c_rq2(const long long* a, long long* b, unp::red_view d) { unp::reduce_serial<long long, unp::OP_XOR, 256>(a, b, d); }
 extern "C" __global__ void KB c_rv(const float* a, float* b, unp::red_view d) { unp::reduce_strided<float, unp::OP_SUM, 256>(a, b, d); }

@@ -212,11 +212,12 @@ char reduction_schedule(uint32_t mask, int32_t rank) {
 
 // The entries of a reduction with kept axes after a reduced one or reduced ones around a kept one
 // (schedules 'm' and 'g'), plain or over NI inputs (`x` prefixes the symbols' tails): xreduce_inner
-// when the innermost axis is reduced, a block or a wave per output; xreduce_outer when it is kept.
+// when the innermost axis is reduced, a block or a wave per output; xreduce_outer when it is kept; and for
+// few positions under many outputs xreduce_lanes.
 // Eight waves a block and up to eight 16-byte loads in flight per lane put 64 KiB in flight per CU
-// (column sums of an 8192 x 4096 f32: one such block per CU reads at 79% of a plain read; 2 to 4
-// blocks, 256 or 1024 threads and 4 or 16 loads measured no better).  The inner entries take two
-// blocks per CU, so that one block's closing fold runs under the other's loads.
+// (2 to 4 blocks, 256 or 1024 threads and 4 or 16 loads measured no better for the column sums of an
+// 8192 x 4096 f32).  The inner entries take two blocks per CU, so that one block's closing fold runs
+// under the other's loads.
 static void emit_split(std::ostringstream& src, Lowered& L, int32_t dtype, int NI, int op, const std::string& ops,
                 const std::string& x) {
   const char* T = ctype(dtype);
@@ -224,39 +225,50 @@ static void emit_split(std::ostringstream& src, Lowered& L, int32_t dtype, int N
   const bool inner = (L.axes_mask >> (L.form.rank - 1)) & 1u;
   L.threads = 512;
   L.blocks_per_cu = inner ? 2 : 1;
-  for (int team = 0; team <= (inner ? 1 : 0); ++team)
+  enum { Block, Team, Lane };
+  for (int how : {Block, Team, Lane})
     for (int fast = 1; fast >= 0; --fast) {
       Entry e;
       e.fast = fast;
       e.vec = fast ? V : 1;
-      e.team = team;
-      e.symbol = L.name + "_" + x + (inner ? (team ? "gw" : "g") : "m") + (fast ? "v" : "s");
-      src << "extern \"C\" __global__ void __launch_bounds__(512) " << e.symbol << "(";
+      e.team = how == Team;
+      e.lane = how == Lane;
+      e.threads = how == Lane ? 1024 : 512;
+      e.blocks_per_cu = how == Block ? 0 : 2;
+      e.symbol = L.name + "_" + x + (inner ? "g" : "m") + (how == Team ? "w" : how == Lane ? "l" : "") + (fast ? "v" : "s");
+      src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << e.symbol << "(";
       for (int k = 0; k < NI; ++k) src << "const " << T << "* in" << k << ", ";
-      src << T << "* out, unp::red_axes d, long long S, " << (inner ? "" : "int lpr, ")
-          << "unsigned long long* partials, unsigned* counters, "
-          << "unsigned epoch, unp::waits wt) {\n  const " << T << "* in[" << NI << "] = {";
+      src << T << "* out, ";
+      const bool plain = how == Lane || (how == Team && !inner);
+      if (!plain) src << "unsigned long long* partials, unsigned* counters, unsigned epoch, unp::waits wt, ";
+      src << "unp::red_axes d) {\n  const " << T << "* in[" << NI << "] = {";
       for (int k = 0; k < NI; ++k) src << (k ? ", " : "") << "in" << k;
-      src << "};\n  unp::" << (inner ? "xreduce_inner<" : "xreduce_outer<") << T << ", " << NI << ", " << op << ", "
-          << ops << ", " << e.vec << ", ";
-      if (inner) src << (team ? 1 : 8) << ", ";
-      src << "512, " << U << ">(in, out, d, S, " << (inner ? "" : "lpr, ") << "partials, counters, epoch, wt);\n}\n";
+      src << "};\n  unp::" << (how == Lane ? "xreduce_lanes<" : inner ? "xreduce_inner<" : how == Team ? "xreduce_outer_wave<" : "xreduce_outer<") << T << ", "
+          << NI << ", " << op << ", " << ops << ", " << e.vec << ", ";
+      if (how == Lane)
+        src << (inner ? "true" : "false") << ", 1024>(in, out, d);\n}\n";
+      else
+        src << (inner ? (how == Team ? "1, " : "8, ") : "") << "512, " << U << ">(in, out, "
+            << (plain ? "" : "partials, counters, epoch, wt, ") << "d);\n}\n";
       L.entries.push_back(e);
     }
 }
 static const char* split_policy(uint32_t mask, int32_t rank) {
   return (mask >> (rank - 1)) & 1u
              ? "blocks stride over (chunk of the reduced positions, output) items, the last-ticket block of an "
-               "output folds its chunk partials; short reductions: waves stride over the outputs"
+               "output folds its chunk partials; short reductions: waves or lanes stride over the outputs"
              : "a wave per 64 x vec columns (or whole rows of fewer), blocks stride over (chunk of the reduced "
-               "rows, column strip) items, the last-ticket block of a strip folds its chunk partials";
+               "rows, column strip) items, the last-ticket block of a strip folds its chunk partials; short "
+               "reductions: a wave per strip, or lanes stride over vectors of columns";
 }
 static std::string split_when(const Entry& e) {
-  return std::string(e.team ? "few positions per output, or many outputs; " : "") +
+  return std::string(e.lane   ? "few positions per output under many outputs; "
+                     : e.team ? "few positions per output, or many outputs; "
+                              : "") +
          (e.fast ? "innermost run >= vec elements" : "otherwise");
 }
 static const char* const kSplitWorkspace =
-    "{\"partials\":\"(outputs, or strips * 64 * vec) * chunks * 8 bytes per 4-byte accumulator word (tagged with the "
+    "{\"partials\":\"(outputs, or strips * their columns) * chunks * 8 bytes per 4-byte accumulator word (tagged with the "
     "launch epoch)\",\"counters\":\"(outputs or strips) * 4\",\"stall\":4,\"host_state\":[\"epoch\"]}";
 
 // When the executor picks an entry that reads through storage-image strides.

@@ -220,8 +220,9 @@ template <class T, int N> UNP_DEV vec<T, N> ld_any(const T* p) {
 }
 // The same through the caches, for data that is read again.
 template <class T, int N> UNP_DEV vec<T, N> ld_cached(const T* p) {
-  static_assert(sizeof(T) * N == 16, "16-byte vectors");
-  return __builtin_bit_cast(vec<T, N>, (u32x4_t)*reinterpret_cast<const u32x4_any*>(p));
+  static_assert(sizeof(T) * N == 16 || N == 1, "16-byte vectors, or elements");
+  if constexpr (N == 1) return vec<T, N>{{*p}};
+  else return __builtin_bit_cast(vec<T, N>, (u32x4_t)*reinterpret_cast<const u32x4_any*>(p));
 }
 template <class T, int N> UNP_DEV void st_any(T* p, const vec<T, N>& v) {
   static_assert(sizeof(T) >= 4, "4- and 8-byte elements");
@@ -937,21 +938,33 @@ UNP_DEV void xreduce_all(const T* const* __restrict__ in, T* __restrict__ out, i
 // ---------------------------------------------------------------------------------------
 
 // The axes of one launch, outermost first, adjacent axes of a kind merged and the innermost run
-// taken out: it holds L contiguous elements (reduced for xreduce_inner, kept for xreduce_outer).
+// taken out: it holds L contiguous elements (reduced for xreduce_inner, kept for xreduce_outer).  What
+// every launch reads lies in the first two cache lines, with the reciprocals of its divisors: a launch
+// of a few microseconds waits for each line of its arguments in turn, and a division in f64 at its start
+// takes as long as a load.
 struct red_axes {
-  i64 nk, nr;           // kept / reduced axes besides the innermost run
-  i64 kext[8], kstr[8];
-  i64 rext[8], rstr[8];
-  double kinv[8], rinv[8];  // 1 / extent
   i64 L;
-  i64 runs;             // innermost runs: of one output's positions (xreduce_inner), of the outputs
-  i64 outs, count;      // output elements, reduced positions per output
+  i64 runs;             // innermost runs: of one output's positions (reduced), of the outputs (kept)
+  i64 count, S;         // reduced positions per output, chunks they are cut into
+  i64 per, units;       // parts of a run (vectors, or column strips); outputs, strips or vectors in all
+  double inv_per, inv_units, inv_S;
+  i32 nk, nr;           // kept / reduced axes besides the innermost run
+  i32 lpr, rpi;         // xreduce_outer: lanes per row, rows per load
+  i64 kstr[8], rstr[8];
+  i64 kext[8], rext[8];
+  double kinv[8], rinv[8];  // 1 / extent
 };
 
+// A value that is the same in every lane of a wave, for the compiler to know.
+UNP_DEV i64 uniform(i64 x) {
+  const u32 lo = (u32)__builtin_amdgcn_readfirstlane((int)(u32)x), hi = (u32)__builtin_amdgcn_readfirstlane((int)(u32)((u64)x >> 32));
+  return (i64)((u64)hi << 32 | lo);
+}
+
 // The element offset of position q over n axes, row-major.
-UNP_DEV i64 unravel(i64 q, i64 n, const i64* ext, const i64* str, const double* inv) {
+UNP_DEV i64 unravel(i64 q, int n, const i64* ext, const i64* str, const double* inv) {
   i64 off = 0;
-  for (i64 k = n - 1; k > 0; --k) {
+  for (int k = n - 1; k > 0; --k) {
     i64 c;
     divisor(ext[k], inv[k])(q, q, c);
     off += c * str[k];
@@ -978,7 +991,7 @@ template <class T, int OP> struct plain_ops {
 // 16 bytes at any element address.  The vector index steps by a constant, so its run and place in
 // the run are carried along instead of divided out at each load.
 //
-// Bound by the read (the means of 256 channels of 25088 f32, 26 MB: 7.7 us, 3.3 TB/s; 259 with a
+// Bound by the read (the means of 256 channels of 25088 f32, 26 MB: 6.9 us, 3.7 TB/s; 259 with a
 // wave per output that divides each position's coordinates out).
 //
 // With S > 1 the teams publish their partials and the one that draws an output's last ticket
@@ -986,8 +999,8 @@ template <class T, int OP> struct plain_ops {
 // walks all S chunks of its outputs by itself and folds the same partials in the same order, so
 // the bits do not depend on where the launch ran.
 template <class T, int NI, int OP, class OPS, int VEC, int TEAM, int THREADS, int U>
-UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out, const red_axes& d, i64 S,
-                           u64* __restrict__ partials, u32* __restrict__ counters, u32 epoch, waits wt) {
+UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out, u64* __restrict__ partials,
+                           u32* __restrict__ counters, u32 epoch, waits wt, const red_axes& d) {
   typedef typename OPS::acc Ac;
   typedef fold<Ac, OP> F;
   typedef tagged<Ac> P;
@@ -997,51 +1010,65 @@ UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out,
   __shared__ Ac chunk[TEAM > 1 ? kMaxChunks : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ti = TEAM > 1 ? tid : lane;
-  const i64 nvr = (d.L + VEC - 1) / VEC;  // vectors per run
-  const i64 nv = d.runs * nvr;            // vectors per output
-  const divisor by_run(nvr > 0 ? nvr : 1), by_outs(d.outs), by_chunks(S);
+  const i64 S = d.S;
+  const i64 nvr = d.per;        // vectors per run
+  const i64 nv = d.runs * nvr;  // vectors per output
+  const divisor by_run(nvr > 0 ? nvr : 1, d.inv_per), by_outs(d.units, d.inv_units), by_chunks(S, d.inv_S);
   i64 dq, dr;
   by_run(STEP, dq, dr);
   // The fold of chunk s of the output at element offset `base`, whole in every lane of a wave.
   auto fold_chunk = [&](i64 base, i64 s) {
     const i64 v0 = by_chunks.quo(nv * s), v1 = by_chunks.quo(nv * (s + 1));
     Ac a = F::identity();
-    if (v0 < v1) {
-      i64 q, r;
-      by_run(v0 + ti, q, r);
-      for (i64 v = v0 + ti; v - lane < v1; v += U * STEP) {
-        vec<T, VEC> x[U][NI];
-        int skip[U];  // the vector's leading elements that are not its own
+    i64 v = v0 + ti, q = 0, r = 0;
+    if (v0 < v1) by_run(v, q, r);
+    // N vectors of each input.  `one`: at most one reduced axis before the run, its offset a product.  The
+    // choice is made once, not at each load, whose code would hold both.
+    auto batch = [&](auto one, auto count) {
+      constexpr int N = decltype(count)::value;
+      vec<T, VEC> x[N][NI];
+      int skip[N];  // the vector's leading elements that are not its own
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          // A lane past the chunk's end reads the vector at `base` and ignores it.
-          const bool ok = v + u * STEP < v1;
-          const i64 c = r * VEC, at = c + VEC <= d.L ? c : d.L - VEC;
-          skip[u] = ok ? (int)(c - at) : VEC;
-          const i64 off = base + (ok ? (d.nr <= 1 ? q * d.rstr[0] : unravel(q, d.nr, d.rext, d.rstr, d.rinv)) + at : 0);
+      for (int u = 0; u < N; ++u) {
+        // A lane past the chunk's end reads the vector at `base` and ignores it.
+        const bool ok = v + u * STEP < v1;
+        const i64 c = r * VEC, at = c + VEC <= d.L ? c : d.L - VEC;
+        skip[u] = ok ? (int)(c - at) : VEC;
+        i64 run;
+        if constexpr (decltype(one)::value) run = q * d.rstr[0];
+        else run = unravel(q, d.nr, d.rext, d.rstr, d.rinv);
+        const i64 off = base + (ok ? run + at : 0);
 #pragma unroll
-          for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
-          q += dq;
-          r += dr;
-          if (r >= nvr) {
-            r -= nvr;
-            ++q;
-          }
+        for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
+        q += dq;
+        r += dr;
+        if (r >= nvr) {
+          r -= nvr;
+          ++q;
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) {
-            const Ac b = xfold<T, NI, OP, OPS, VEC>(a, x[u], e);
-            a = e >= skip[u] ? b : a;
-          }
       }
-    }
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const Ac b = xfold<T, NI, OP, OPS, VEC>(a, x[u], e);
+          a = e >= skip[u] ? b : a;
+        }
+      v += N * STEP;
+    };
+    auto walk = [&](auto one) {
+      while (v - lane < v1) {
+        if (v - lane + STEP < v1) batch(one, ic<U>{});
+        else batch(one, ic<1>{});
+      }
+    };
+    if (d.nr <= 1) walk(ic<1>{});
+    else walk(ic<0>{});
     return wave_reduce<Ac, OP>(a);
   };
   if constexpr (TEAM == 1) {
     // Outputs go round the blocks first, so that fewer outputs than waves still reach every CU.
-    for (i64 o = (i64)wave * gridDim.x + blockIdx.x; o < d.outs; o += (i64)gridDim.x * TEAMS) {
+    for (i64 o = (i64)wave * gridDim.x + blockIdx.x; o < d.units; o += (i64)gridDim.x * TEAMS) {
       const Ac a = fold_chunk(unravel(o, d.nk, d.kext, d.kstr, d.kinv), 0);
       if (lane == 0) out[o] = xfinish<T, OP, OPS>(a, d.count);
     }
@@ -1049,7 +1076,7 @@ UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out,
     // One loop for both ways of walking the chunks, so the fold's code is there once: a launch
     // of a few microseconds fetches every instruction it runs from memory.
     const bool alone = S > 1 && partials == nullptr;
-    const i64 n = alone ? divisor(gridDim.x).quo(d.outs - blockIdx.x + gridDim.x - 1) * S : d.outs * S;
+    const i64 n = alone ? divisor(gridDim.x).quo(d.units - blockIdx.x + gridDim.x - 1) * S : d.units * S;
     for (i64 it = alone ? 0 : blockIdx.x; it < n; it += alone ? 1 : gridDim.x) {
       i64 s, o;
       if (alone) {
@@ -1097,201 +1124,313 @@ UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out,
 // The innermost run kept: `L` columns under `count` reduced rows per (outer kept position) a; the
 // shape of every axis set with kept axes after the last reduced one (column sums: one row axis).
 //
-// A wave covers 64 * VEC consecutive columns, or, where all L columns need LPR < 64 lanes, 64 / LPR
-// whole rows at a time.  The last vector of a row starts at L - VEC and stores only the columns the
+// A wave covers 64 * VEC consecutive columns, or, in strips of LPR < 64 lanes' columns, 64 / LPR
+// whole rows at a time.  The last vector of a row starts at L - VEC and passes on only the columns the
 // one before it does not (L >= VEC, any alignment).  The block's WAVES waves split the block's run of
 // rows into consecutive pieces; the blocks of one column strip split the rows into S consecutive
 // chunks.  The (strip, chunk) items are numbered chunk-major and blocks stride over them (a
 // device-class grid), so consecutive blocks take consecutive strips of one chunk and the blocks in
 // flight together read whole rows.  Lane l folds its VEC columns down its rows in ascending order
-// (U rows in flight), the waves' (and packed rows') partials meet in LDS in order.  With S > 1 each
-// block publishes its partials and the block that draws the strip's last ticket folds them: the
-// (packed row, wave) slot g takes the chunks g, g + G, ... (G slots), all in flight together, and
-// the slots meet in order.  The order is fixed by (S, WAVES, U, L), so the result is reproducible.
-// counters[strip] is zero on entry and left zero; the partials carry the launch's `epoch`.  6000 x 2050
-// f32 column norms (49 MB) take 18.2 us, where a wave per column took 59.3.
+// (U rows in flight); the waves' values meet in LDS in wave order and the packed rows' in a tree, a
+// thread per column.  With S > 1 each block publishes its columns and the block that draws the strip's
+// last ticket folds them: group g of its threads takes the chunks g, g + G, ... (G groups of a thread
+// per column), all in flight together, and the groups meet in a tree.  The order is fixed by (S, WAVES,
+// U, L, LPR), so the result is reproducible.  counters[strip] is zero on entry and left zero; the
+// partials carry the launch's `epoch`.  6000 x 2050 f32 column norms (49 MB) take 15.6 us, where a wave
+// per column took 59.3; 8192 x 4096 f32 column sums (134 MB) 23.7 launched one after another and 27 on
+// cold caches.
 // Without a workspace (partials null) each block walks all chunks of its strips by itself in the
 // same association.
-template <class T, int NI, int OP, class OPS, int VEC, int THREADS, int U>
-UNP_DEV void xreduce_outer(const T* const* __restrict__ in, T* __restrict__ out, const red_axes& d, i64 S, int lpr,
-                           u64* __restrict__ partials, u32* __restrict__ counters, u32 epoch, waits wt) {
+//
+// How the lanes of a wave lie on a strip's columns and rows, and their fold of a run of rows.
+template <class T, int NI, int OP, class OPS, int VEC, int U> struct outer_lanes {
   typedef typename OPS::acc Ac;
   typedef fold<Ac, OP> F;
-  typedef tagged<Ac> P;
-  constexpr int WAVES = THREADS / 64, CW = 64 * VEC;
-  __shared__ Ac sh[WAVES][CW], slots[WAVES][CW];
-  __shared__ u32 last;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const i64 B = d.L, R = d.count;
-  const int cw = lpr * VEC, rpi = 64 / lpr;  // columns per strip, rows per load
-  const i64 ncb = divisor(cw).quo(B + cw - 1);
-  const i64 nstrips = d.runs * ncb;
-  const divisor by_ncb(ncb), by_strips(nstrips), by_chunks(S);
-  // Lanes past the last whole row of a load (64 % lpr of them) repeat the first row's.
-  const int sub = lane / lpr < rpi ? lane / lpr : 0, cl = lane % lpr, G = WAVES * rpi;
-  const bool spare = lane >= rpi * lpr;
-  struct Strip {
-    i64 base, out0, c;  // element offset of the strip's rows, its output row, this lane's first column
-    int skip;           // leading columns of the vector that another lane stores
-    bool live;
-  };
-  auto strip_of = [&](i64 strip) {
-    Strip t;
-    i64 a, cb;
-    by_ncb(strip, a, cb);
-    const i64 b0 = cb * cw + (i64)cl * VEC;
-    t.live = b0 < B && !spare;
-    t.c = t.live ? (b0 + VEC <= B ? b0 : B - VEC) : 0;
-    t.skip = (int)(b0 - t.c);
-    t.base = unravel(a, d.nk, d.kext, d.kstr, d.kinv);
-    t.out0 = a * B;
-    return t;
-  };
-  // The fold of every slot's value of this lane's columns, in slot order (slot g: packed row g / WAVES,
-  // wave g % WAVES), the waves' values of one packed row in flight together.
-  auto fold_slots = [&](const Ac (&m)[WAVES][CW], Ac (&a)[VEC]) {
+  int rpi, cw, sub, cl;  // rows per load, columns per strip; this lane's packed row and vector of it
+  bool spare;            // a lane past the last whole row of a load (64 % LPR of them): repeats the first row's
+  UNP_DEV outer_lanes(const red_axes& d, int lane) : rpi(d.rpi), cw(d.lpr * VEC) {
+    const int row = (int)((u32)lane / (u32)d.lpr);
+    spare = row >= rpi;
+    sub = spare ? 0 : row;
+    cl = lane - row * d.lpr;
+  }
+  // Rows [w0, w1) of the strip at column c0 of the rows at `base`; to[p * cw + t] takes packed row p's
+  // fold of column c0 + t.
+  UNP_DEV void fold(const T* const* __restrict__ in, const red_axes& d, i64 base, i64 c0, i64 w0, i64 w1, Ac* to) const {
+    const i64 b0 = c0 + (i64)cl * VEC;
+    const bool live = b0 < d.L && !spare;
+    const i64 c = live ? (b0 + VEC <= d.L ? b0 : d.L - VEC) : 0;
+    const int skip = (int)(b0 - c);  // leading columns of the vector that another lane has
+    Ac a[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) a[e] = F::identity();
-    for (int p = 0; p < rpi; ++p) {
-      Ac v[WAVES][VEC];
+    auto take = [&](const vec<T, VEC> (&x)[U][NI], auto&& ok) {
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) v[w][e] = m[w][(p * lpr + cl) * VEC + e];
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) a[e] = F::apply(a[e], v[w][e]);
-    }
-  };
-  // Chunk s of a strip, folded over the block's waves and packed rows: wave 0's lanes of the first
-  // packed row hold the result.
-  auto fold_chunk = [&](const Strip& t, i64 s, Ac (&a)[VEC]) {
-    const i64 i0 = by_chunks.quo(R * s), i1 = by_chunks.quo(R * (s + 1));
-    const i64 w0 = i0 + (i1 - i0) * wave / WAVES, w1 = i0 + (i1 - i0) * (wave + 1) / WAVES;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) a[e] = F::identity();
-    // U loads a pass, also the last: with a branch around every load to skip those past the piece,
-    // an 8192 x 4096 f32 column sum took 47.9 us instead of 28.4.
-    for (i64 i = w0; i < w1; i += U * rpi) {
-      vec<T, VEC> x[U][NI];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const i64 row = i + u * rpi + sub;
-        const i64 rr = row < w1 ? row : w1 - 1;  // past the piece its last row is read and ignored
-        const i64 off = t.base + t.c + (d.nr <= 1 ? rr * d.rstr[0] : unravel(rr, d.nr, d.rext, d.rstr, d.rinv));
-#pragma unroll
-        for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool ok = t.live && i + u * rpi + sub < w1;
+      for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           const Ac b = xfold<T, NI, OP, OPS, VEC>(a[e], x[u], e);
-          a[e] = ok ? b : a[e];
+          a[e] = ok(u) ? b : a[e];
         }
+    };
+    i64 i = w0;
+    const bool one = d.nr <= 1;
+    if (one) {
+      // Whole passes: a lane's address and a uniform offset per load.  (The pieces' bounds are uniform; as
+      // long as the compiler took them for a lane's own it multiplied every row out per lane, and the f64
+      // column sums of 4096 x 4096 took 38.9 us on cold caches, 33.2 now.)
+      const i64 stride = d.rstr[0], lane0 = base + c + sub * stride;
+      for (; i + U * rpi <= w1; i += U * rpi) {
+        vec<T, VEC> x[U][NI];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + lane0 + (i + u * rpi) * stride);
+        take(x, [](int) { return true; });
       }
     }
+    // U loads a pass, also the last: with a branch around every load to skip those past the piece,
+    // an 8192 x 4096 f32 column sum took 47.9 us instead of 28.4.
+    for (; i < w1; i += U * rpi) {
+      vec<T, VEC> x[U][NI];
+      auto load = [&](auto&& row_offset) {
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) sh[wave][lane * VEC + e] = a[e];
-    __syncthreads();
-    if (wave == 0) fold_slots(sh, a);
-    __syncthreads();  // sh is free again
+        for (int u = 0; u < U; ++u) {
+          const i64 row = i + u * rpi + sub;
+          const i64 off = base + c + row_offset(row < w1 ? row : w1 - 1);  // past the piece its last row is read and ignored
+#pragma unroll
+          for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
+        }
+      };
+      if (one) load([&](i64 row) { return row * d.rstr[0]; });
+      else load([&](i64 row) { return unravel(row, d.nr, d.rext, d.rstr, d.rinv); });
+      take(x, [&](int u) { return i + u * rpi + sub < w1; });
+    }
+    if (live)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e)
+        if (e >= skip) to[sub * cw + cl * VEC + e - skip] = a[e];
+  }
+};
+
+template <class T, int NI, int OP, class OPS, int VEC, int THREADS, int U>
+UNP_DEV void xreduce_outer(const T* const* __restrict__ in, T* __restrict__ out, u64* __restrict__ partials,
+                           u32* __restrict__ counters, u32 epoch, waits wt, const red_axes& d) {
+  typedef typename OPS::acc Ac;
+  typedef fold<Ac, OP> F;
+  typedef tagged<Ac> P;
+  constexpr int WAVES = THREADS / 64;
+  __shared__ Ac sh[WAVES][64 * VEC], slots[THREADS];
+  __shared__ u32 last;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const i64 B = d.L, R = d.count, S = d.S;
+  const outer_lanes<T, NI, OP, OPS, VEC, U> lanes(d, tid & 63);
+  const int cw = lanes.cw, rpi = lanes.rpi, G = THREADS / cw;
+  const divisor by_ncb(d.per, d.inv_per), by_strips(d.units, d.inv_units), by_chunks(S, d.inv_S);
+  // m[p * cw + t] over p < n, folded into m[t], a thread per value.
+  auto tree = [&](Ac* m, int n) {
+    while (n > 1) {
+      const int half = (n + 1) / 2;
+      __syncthreads();
+      if (tid < (n - half) * cw) m[tid] = F::apply(m[tid], m[half * cw + tid]);
+      n = half;
+    }
   };
-  auto store = [&](const Strip& t, const Ac (&a)[VEC]) {
-    if (wave != 0 || lane >= lpr || !t.live) return;
+  // Chunk s of the strip at column c0 of the rows at `base`, folded over the block: thread t < cw holds
+  // column c0 + t.
+  auto fold_chunk = [&](i64 base, i64 c0, i64 s) {
+    const i64 i0 = S == 1 ? 0 : by_chunks.quo(R * s), i1 = S == 1 ? R : by_chunks.quo(R * (s + 1));
+    lanes.fold(in, d, base, c0, uniform(i0 + (i1 - i0) * wave / WAVES), uniform(i0 + (i1 - i0) * (wave + 1) / WAVES),
+               sh[wave]);
+    __syncthreads();
+    Ac r = F::identity();
+    if (tid < rpi * cw) {
+      r = sh[0][tid];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e)
-      if (e >= t.skip) out[t.out0 + t.c + e] = xfinish<T, OP, OPS>(a[e], R);
+      for (int w = 1; w < WAVES; ++w) r = F::apply(r, sh[w][tid]);
+    }
+    if (rpi > 1) {
+      if (tid < rpi * cw) sh[0][tid] = r;  // this thread alone read it
+      tree(sh[0], rpi);
+      if (tid < cw) r = sh[0][tid];
+    }
+    return r;
   };
   // One loop for both ways of walking the chunks, as in xreduce_inner.
   const bool alone = S > 1 && partials == nullptr;
-  const i64 n = alone ? divisor(gridDim.x).quo(nstrips - blockIdx.x + gridDim.x - 1) * S : nstrips * S;
+  const i64 n = alone ? divisor(gridDim.x).quo(d.units - blockIdx.x + gridDim.x - 1) * S : d.units * S;
   for (i64 it = alone ? 0 : blockIdx.x; it < n; it += alone ? 1 : gridDim.x) {
-    i64 s, strip;
+    i64 s = 0, strip = it, at, cb;
     if (alone) {
       by_chunks(it, strip, s);
       strip = strip * gridDim.x + blockIdx.x;
-    } else {
+    } else if (S > 1) {
       by_strips(it, s, strip);
     }
-    const Strip t = strip_of(strip);
-    Ac a[VEC];
-    fold_chunk(t, s, a);
-    if (S == 1) {
-      store(t, a);
-      continue;
-    }
+    by_ncb(strip, at, cb);
+    const i64 c0 = cb * cw;
+    const bool mine = tid < cw && c0 + tid < B;  // this thread's column
+    Ac a = fold_chunk(unravel(at, d.nk, d.kext, d.kstr, d.kinv), c0, s);
+    bool done = S == 1;
     if (alone) {
-      // Chunk s goes to slot s % G, as the closing fold below takes it.
-      if (s == 0) {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) slots[wave][lane * VEC + e] = F::identity();
-        __syncthreads();
+      // Chunk s goes to group s % G, as the closing fold below takes it.
+      if (tid < cw) {
+        if (s == 0)
+          for (int g = 0; g < G; ++g) slots[g * cw + tid] = F::identity();
+        Ac* const slot = &slots[(int)(s % G) * cw + tid];
+        *slot = F::apply(*slot, a);
       }
-      if (wave == 0 && lane < lpr) {
-        const int g = (int)s % G;
-        Ac* const slot = &slots[g % WAVES][(g / WAVES * lpr + cl) * VEC];
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) slot[e] = F::apply(slot[e], a[e]);
-      }
-      if (s == S - 1) {
-        __syncthreads();
-        if (wave == 0) fold_slots(slots, a);
-        store(t, a);
-        __syncthreads();  // slots are the next strip's
-      }
-      continue;
-    }
-    // An item's partials: VEC x W planes of 64 words, word (e, i) of lane l at (e W + i) 64 + l.
-    constexpr i64 ITEM = (i64)CW * P::W;
-    u64* const mine = partials + strip * S * ITEM + cl;
-    if (wave == 0) {
-      if (lane < lpr) {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) P::put(mine + s * ITEM + e * P::W * 64, 64, a[e], epoch);
-      }
-      if (lane == 0) last = arrive_after_stores(&counters[strip]) == (u32)(S - 1) ? 1u : 0u;
-    }
-    __syncthreads();
-    if (last != 0u) {
-      constexpr int Q = 4;  // partials of a slot in flight
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) a[e] = F::identity();
-      for (i64 k = sub * WAVES + wave; k < S; k += Q * G) {
-        Ac v[Q][VEC];
-        bool ok = true;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          const i64 kk = k + q * G < S ? k + q * G : S - 1;
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) ok = P::take(mine + kk * ITEM + e * P::W * 64, 64, epoch, v[q][e]) && ok;
-        }
-        if (!ok) {  // a partial not yet visible: wait for each in turn
+      done = s == S - 1;
+    } else if (S > 1) {
+      // An item's partials: W planes of cw words, a word per column.
+      const i64 item = (i64)cw * P::W;
+      u64* const strip_p = partials + strip * S * item;
+      if (mine) P::put(strip_p + s * item + tid, cw, a, epoch);
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's words are on their way before the ticket
+      __syncthreads();
+      if (tid == 0) last = arrive_after_stores(&counters[strip]) == (u32)(S - 1) ? 1u : 0u;
+      __syncthreads();
+      done = last != 0u;
+      const int g = (int)((u32)tid / (u32)cw), col = tid - g * cw;
+      if (done && g < G) {
+        constexpr int Q = 8;  // partials of a column in flight
+        a = F::identity();
+        const bool live = c0 + col < B;
+        for (i64 k = g; live && k < S; k += Q * G) {
+          Ac v[Q];
+          bool ok = true;
 #pragma unroll
           for (int q = 0; q < Q; ++q) {
             const i64 kk = k + q * G < S ? k + q * G : S - 1;
+            ok = P::take(strip_p + kk * item + col, cw, epoch, v[q]) && ok;
+          }
+          if (!ok) {  // a partial not yet visible: wait for each in turn
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) v[q][e] = P::wait(mine + kk * ITEM + e * P::W * 64, 64, epoch, F::identity(), wt);
+            for (int q = 0; q < Q; ++q) {
+              const i64 kk = k + q * G < S ? k + q * G : S - 1;
+              v[q] = P::wait(strip_p + kk * item + col, cw, epoch, F::identity(), wt);
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            const Ac b = F::apply(a, v[q]);
+            a = k + q * G < S ? b : a;
           }
         }
+        slots[tid] = a;
+      }
+      if (done && tid == 0) __hip_atomic_store(&counters[strip], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (S > 1 && done) {
+      tree(slots, G);
+      __syncthreads();
+      if (tid < cw) a = slots[tid];
+    }
+    if (done && mine) out[at * B + c0 + tid] = xfinish<T, OP, OPS>(a, R);
+    __syncthreads();  // sh, slots and last are the next item's
+  }
+}
+
+// The same with a wave per strip, for strips of few rows: no barrier, no chunks.  2000 x 100 x 7 f32 over
+// the middle axis: 4.7 us, 19.5 with a block per strip.
+template <class T, int NI, int OP, class OPS, int VEC, int THREADS, int U>
+UNP_DEV void xreduce_outer_wave(const T* const* __restrict__ in, T* __restrict__ out, const red_axes& d) {
+  typedef typename OPS::acc Ac;
+  typedef fold<Ac, OP> F;
+  constexpr int WAVES = THREADS / 64;
+  __shared__ Ac sh[WAVES][64 * VEC];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const outer_lanes<T, NI, OP, OPS, VEC, U> lanes(d, lane);
+  const int cw = lanes.cw;
+  const divisor by_ncb(d.per, d.inv_per);
+  Ac* const m = sh[wave];
+  // The wave's own LDS accesses are in order; the compiler keeps them so.
+  auto meet = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (i64 strip = (i64)wave * gridDim.x + blockIdx.x; strip < d.units; strip += (i64)gridDim.x * WAVES) {
+    i64 at, cb;
+    by_ncb(strip, at, cb);
+    const i64 c0 = cb * cw;
+    lanes.fold(in, d, unravel(at, d.nk, d.kext, d.kstr, d.kinv), c0, 0, d.count, m);
+    for (int n = lanes.rpi; n > 1;) {
+      const int half = (n + 1) / 2;
+      meet();
+      for (int t = lane; t < (n - half) * cw; t += 64) m[t] = F::apply(m[t], m[half * cw + t]);
+      n = half;
+    }
+    meet();
+    for (int t = lane; t < cw && c0 + t < d.L; t += 64) out[at * d.L + c0 + t] = xfinish<T, OP, OPS>(m[t], d.count);
+    meet();  // m is the next strip's
+  }
+}
+
+// Few positions under many outputs: a lane per output (the innermost run reduced, INNER) or per vector
+// of one run's columns (kept), which folds its positions in ascending order, eight vectors of each input
+// in flight.  No LDS and no barrier, where a block or a wave for so little spends its time on its start
+// and its close: 100000 x 3 x 5 f32 over the middle axis takes 4.4 us, 2326 in xreduce_outer; 4 x 100000 x 8
+// over the outer two 4.3, 77 in xreduce_inner.
+template <class T, int NI, int OP, class OPS, int VEC, bool INNER, int THREADS>
+UNP_DEV void xreduce_lanes(const T* const* __restrict__ in, T* __restrict__ out, const red_axes& d) {
+  typedef typename OPS::acc Ac;
+  typedef fold<Ac, OP> F;
+  constexpr int C = INNER ? 1 : VEC;  // this lane's outputs
+  const divisor by_per(d.per > 0 ? d.per : 1, d.inv_per);
+  const i64 n = INNER ? d.runs * d.per : d.count;  // vectors to fold
+  for (i64 i = (i64)blockIdx.x * THREADS + threadIdx.x; i < d.units; i += (i64)gridDim.x * THREADS) {
+    i64 run = i, v = 0;
+    if constexpr (!INNER) by_per(i, run, v);
+    const i64 c = INNER || v * VEC + VEC <= d.L ? v * VEC : d.L - VEC;
+    const int mine = (int)(v * VEC - c);  // the first of the lane's columns that is its own
+    const i64 base = unravel(run, d.nk, d.kext, d.kstr, d.kinv) + c;
+    Ac a[C];
 #pragma unroll
-        for (int q = 0; q < Q; ++q)
+    for (int e = 0; e < C; ++e) a[e] = F::identity();
+    i64 q = 0, r = 0;  // INNER: the next vector's run, and its place in it
+    auto batch = [&](auto count, i64 k0) {
+      constexpr int N = decltype(count)::value;
+      vec<T, VEC> x[N][NI];
+      int skip[N];
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) {
-            const Ac b = F::apply(a[e], v[q][e]);
-            a[e] = k + q * G < S ? b : a[e];
+      for (int u = 0; u < N; ++u) {
+        const bool ok = k0 + u < n;  // past the end the last vector is read again and ignored
+        i64 off;
+        if constexpr (INNER) {
+          const i64 at = r * VEC + VEC <= d.L ? r * VEC : d.L - VEC;
+          skip[u] = ok ? (int)(r * VEC - at) : VEC;
+          off = at + (d.nr <= 1 ? q * d.rstr[0] : unravel(q, d.nr, d.rext, d.rstr, d.rinv));
+          if (k0 + u + 1 < n && ++r == d.per) {
+            r = 0;
+            ++q;
           }
+        } else {
+          const i64 row = ok ? k0 + u : n - 1;
+          skip[u] = ok ? 0 : VEC;
+          off = d.nr <= 1 ? row * d.rstr[0] : unravel(row, d.nr, d.rext, d.rstr, d.rinv);
+        }
+#pragma unroll
+        for (int k = 0; k < NI; ++k) x[u][k] = ld_cached<T, VEC>(in[k] + base + off);
       }
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) sh[wave][lane * VEC + e] = a[e];
-      __syncthreads();
-      if (wave == 0) fold_slots(sh, a);
-      store(t, a);
-      if (tid == 0) __hip_atomic_store(&counters[strip], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          Ac& to = a[INNER ? 0 : e];
+          const Ac b = xfold<T, NI, OP, OPS, VEC>(to, x[u], e);
+          to = e >= skip[u] ? b : to;
+        }
+    };
+    i64 k = 0;
+    for (; k + 4 < n; k += 8) batch(ic<8>{}, k);
+    if (k < n) batch(ic<4>{}, k);
+    if constexpr (INNER) {
+      out[i] = xfinish<T, OP, OPS>(a[0], d.count);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e)
+        if (e >= mine) out[run * d.L + c + e] = xfinish<T, OP, OPS>(a[e], d.count);
     }
-    __syncthreads();  // sh and last are the next item's
   }
 }
 
@@ -1301,7 +1440,6 @@ template <class T, int OP, class A> UNP_DEV T scan_out(A v, i64 count) {
   if constexpr (OP == OP_MEAN) return (T)(v / (double)count);
   else return (T)v;
 }
-
 
 // ---------------------------------------------------------------------------------------
 // A scan in the serial lift's own order (lift_scan_opdef, kernel_lift.rs:504-700): along a

@@ -716,11 +716,13 @@ waits_host waits_of(const unp_exec* x) { return waits_host{x->stall, x->wait_tic
 
 // The axes of a row-major input for a split reduction: the innermost run of one kind as L, the kept
 // and the reduced axes before it with their element strides, outermost first.  Axes of extent 1 are
-// dropped and adjacent axes of a kind merged (a merged run's stride is its innermost axis's).
-void fill_red_axes(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask, unp::red_axes_host& d) {
+// dropped and adjacent axes of a kind merged (a merged run's stride is its innermost axis's).  Returns
+// the number of outputs.
+long long fill_red_axes(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask, unp::red_axes_host& d) {
   const bool last = (mask >> (rank - 1)) & 1u;
-  d.L = d.outs = d.count = 1;
-  for (int32_t k = 0; k < rank; ++k) ((mask >> k) & 1u ? d.count : d.outs) *= ext[(size_t)k];
+  long long outs = 1;
+  d.L = d.count = 1;
+  for (int32_t k = 0; k < rank; ++k) ((mask >> k) & 1u ? d.count : outs) *= ext[(size_t)k];
   int32_t k = rank - 1;
   for (; k >= 0 && (((mask >> k) & 1u) != 0) == last; --k) d.L *= ext[(size_t)k];
   long long stride = d.L;
@@ -729,7 +731,7 @@ void fill_red_axes(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask,
     const long long e = ext[(size_t)k];
     if (e == 1) continue;
     const bool red = (mask >> k) & 1u;
-    long long& n = red ? d.nr : d.nk;
+    int32_t& n = red ? d.nr : d.nk;
     long long* const xs = red ? d.rext : d.kext;
     long long* const ss = red ? d.rstr : d.kstr;
     if (n > 0 && red == prev) {
@@ -745,36 +747,37 @@ void fill_red_axes(const std::vector<int64_t>& ext, int32_t rank, uint32_t mask,
   std::reverse(d.kstr, d.kstr + d.nk);
   std::reverse(d.rext, d.rext + d.nr);
   std::reverse(d.rstr, d.rstr + d.nr);
-  for (long long i = 0; i < d.nk; ++i) d.kinv[i] = 1.0 / (double)d.kext[i];
-  for (long long i = 0; i < d.nr; ++i) d.rinv[i] = 1.0 / (double)d.rext[i];
-  const long long total = last ? d.count : d.outs;
+  for (int32_t i = 0; i < d.nk; ++i) d.kinv[i] = 1.0 / (double)d.kext[i];
+  for (int32_t i = 0; i < d.nr; ++i) d.rinv[i] = 1.0 / (double)d.rext[i];
+  const long long total = last ? d.count : outs;
   d.runs = d.L > 0 ? total / d.L : 0;
+  return outs;
 }
 
 // What a split reduction's launch takes, in microseconds, up to a constant: `items` over `grid` blocks
 // of eight waves that stride over them, `loads` 16-byte loads of each lane per item, `folds` rounds
 // of loads of the partials in the closing fold (0: not split).  Blocks read `speed` times the 5
 // TB/s they reach together (8 KiB a load and block), or, where few run, the 27 GB/s one reaches, and
-// wait about 1.2 us for every eight loads; an item pays about 2 us for its start and its fold over
-// the block, a split launch 3.5 us for publishing, the ticket and the store.  Against measurement:
-// 6000 x 2050 f32 column norms 19.4 us at 28 chunks of 256 columns (here 17.9 + the launch), 30.0 at
-// 85; 12158 x 90 I32 column maxima 13.6 at 64 chunks, 15.1 at 256; the means of 256 channels of 25088
-// f32 each 9.5 (7.0 + the launch).
-double split_cost(long long items, long long grid, double loads, double speed, long long folds) {
+// wait about 1.2 us for every eight loads; an item pays `start` (1 us, or 2 where it also folds lanes or
+// packed rows over the block) outside its loads, a split launch 3.5 us for publishing, the ticket and the
+// store.  Against measurement: 6000 x 2050 f32 column norms 15.1 us at 28 chunks of 256 columns (18.2
+// here), 12158 x 90 I32 column maxima 8.9 at 64 chunks, the means of 256 channels of 25088 f32 each 6.9 (7.0).
+double split_cost(long long items, long long grid, double loads, double speed, double start, long long folds) {
   const double together = 8192.0 / 5.0e6 * (double)std::min(items, grid) / speed;
-  const double item = std::max(1.2 * std::ceil(loads / 8.0), loads * std::max(0.3, together)) + 2.0;
+  const double item = std::max(1.2 * std::ceil(loads / 8.0), loads * std::max(0.3, together)) + start;
   return (double)((items + grid - 1) / grid) * item + (folds ? 3.5 + 1.3 * (double)folds : 0.0);
 }
 
-// The number of chunks (1 .. kMaxChunks, at most kSplitRounds whole rounds of items, at least
-// `least` loads each) with the least cost, for `units` outputs or strips of `loads` loads each of
-// which `slots` partials are folded in a round; `best` starts at the cost to beat.
-long long split_chunks(long long units, long long grid, double loads, double speed, long long slots, double& best) {
+// The number of chunks (1 .. kMaxChunks, at most kSplitRounds whole rounds of items, at least a load
+// each) with the least cost, for `units` outputs or strips of `loads` loads each of which `slots`
+// partials are folded in a round; `best` starts at the cost to beat.
+long long split_chunks(long long units, long long grid, double loads, double speed, double start, long long slots,
+                       double& best) {
   long long S = 1;
   const auto take = [&](long long s) {
     if (s < 1 || s > unp::kMaxChunks || (s > 1 && (units * s > (long long)kSplitRounds * grid || loads / (double)s < 1.0)))
       return;
-    const double c = split_cost(units * s, grid, loads / (double)s, speed, s > 1 ? (s + slots - 1) / slots : 0);
+    const double c = split_cost(units * s, grid, loads / (double)s, speed, start, s > 1 ? (s + slots - 1) / slots : 0);
     if (c < best) {
       best = c;
       S = s;
@@ -875,7 +878,7 @@ static_assert(sizeof(unp::red_view_host) == 44 * 8, "red_view_host mirrors the d
 static_assert(sizeof(unp::scan_view_host) == 29 * 8, "scan_view_host mirrors the device's scan_view");
 static_assert(sizeof(unp::ew_tile_view_host) == 114 * 8, "ew_tile_view_host mirrors the device's ew_tile_view");
 static_assert(sizeof(unp::gather_view_host) == 35 * 8, "gather_view_host mirrors the device's gather_view");
-static_assert(sizeof(unp::red_axes_host) == 54 * 8, "red_axes_host mirrors the device's red_axes");
+static_assert(sizeof(unp::red_axes_host) == 59 * 8, "red_axes_host mirrors the device's red_axes");
 
 int32_t launch(unp_exec* x, size_t entry, uint32_t grid, void** params, hipStream_t s, unp_error* err) {
   const uint32_t threads = (uint32_t)(x->l.entries[entry].threads ? x->l.entries[entry].threads : x->l.threads);
@@ -928,58 +931,95 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
   const unp_form& f = x->l.form;
   const bool inner = inner_reduced(x->l);
   unp::red_axes_host d{};
-  fill_red_axes(ext, f.rank, x->l.axes_mask, d);
-  const long long grid = (long long)x->cu_count * x->l.blocks_per_cu;
+  const long long outs = fill_red_axes(ext, f.rank, x->l.axes_mask, d);
+  const long long cus = x->cu_count;
+  const long long grid = cus * x->l.blocks_per_cu;  // of a block per item
   const long long vec = 16 / (long long)unp::kind_bytes(f.dtype);
   const bool fast = d.L >= vec;
   const long long v = fast ? vec : 1;
-  long long S = 1, units = d.outs;
-  bool team = false;
-  int lpr = 64;
+  const long long per = (d.L + v - 1) / v;  // vectors per innermost run
+  const double inputs = (double)(ptrs.size() - 1);
+  bool team = false, lane = false;
   double best = 1e300;
+  d.S = 1;
   if (inner) {
     // A block per (chunk of an) output, or a wave per output.
-    const double loads = (double)(d.runs * ((d.L + v - 1) / v)) / 64.0;
-    S = split_chunks(units, grid, loads / 8.0, 1.0, 64, best);
-    const long long waves = 8 * grid, busy = std::min(units, waves);
-    team = (double)((units + waves - 1) / waves) *
-               std::max(1.2 * std::ceil(loads / 8.0), (double)busy * loads * 1024.0 / 5.0e6) + 2.0 < best;
-    if (team) S = 1;
+    d.per = per;
+    d.units = outs;
+    const double loads = inputs * (double)(d.runs * per) / 64.0;
+    d.S = split_chunks(outs, grid, loads / 8.0, 1.0, 2.0, 64, best);
+    const long long waves = 8 * grid, busy = std::min(outs, waves);
+    const double c = (double)((outs + waves - 1) / waves) *
+                         std::max(1.2 * std::ceil(loads / 8.0), (double)busy * loads * 1024.0 / 5.0e6) + 2.0;
+    if (c < best) {
+      team = true;
+      d.S = 1;
+      best = c;
+    }
   } else {
-    // Strips of 64 lanes' columns, or of 32 or 16 where that gives more blocks without splitting rows:
+    // Strips of 64 lanes' columns, or of fewer where that gives more blocks without splitting rows:
     // narrower ones read slower (28.9, 31.5, 33.8 us for 2000 x 16001 f32 column norms at 64, 32 and
-    // 16 lanes; 53.6 at 8).
-    const long long whole = std::min(64LL, (d.L + v - 1) / v);
-    const struct { long long lanes; double speed; } widths[] = {{64, 1.0}, {32, 0.9}, {16, 0.8}};
+    // 16 lanes; 53.6 at 8); or a wave per strip.
+    const long long whole = std::min(64LL, per);
+    const struct { long long lanes; double speed; } widths[] = {{64, 1.0}, {32, 0.9}, {16, 0.8}, {8, 0.5}, {4, 0.35}};
     for (const auto& w : widths) {
       const long long lanes = std::min(w.lanes, whole);
       if (w.lanes < 64 && w.lanes >= whole) continue;
-      const long long n = d.runs * ((d.L + lanes * v - 1) / (lanes * v)), rpi = 64 / lanes;
-      const double before = best;
-      const long long s = split_chunks(n, grid, (double)d.count / (double)(8 * rpi), w.speed, 4 * 8 * rpi, best);
+      const long long strips = (d.L + lanes * v - 1) / (lanes * v), n = d.runs * strips, rpi = 64 / lanes;
+      const double loads = inputs * (double)d.count / (double)(8 * rpi), before = best;
+      const long long S = split_chunks(n, grid, loads, w.speed, rpi > 1 ? 2.0 : 1.0, 8 * 512 / (lanes * v), best);
+      // A wave per strip.
+      const long long waves = 16 * cus, busy = std::min(n, waves);
+      const double c = (double)((n + waves - 1) / waves) *
+                           (std::max(1.5 * std::ceil(loads), 8.0 * loads * 1024.0 * (double)busy / 4.2e6 / w.speed) + 2.0) + 0.7;
+      const bool by_waves = c < best;
+      if (by_waves) best = c;
       if (best < before) {
-        S = s;
-        units = n;
-        lpr = (int)lanes;
+        team = by_waves;
+        d.S = by_waves ? 1 : S;
+        d.per = strips;
+        d.units = n;
+        d.lpr = (int32_t)lanes;
+        d.rpi = (int32_t)rpi;
       }
     }
   }
+  {
+    // A lane per output or per vector of columns: eight loads in flight each, whose lines it has to
+    // itself only where the run is long.
+    const long long units = inner ? outs : d.runs * per, n = inner ? d.runs * per : d.count;
+    const long long lanes = 2048 * cus, busy = std::min(units, lanes);
+    const double c = (double)((units + lanes - 1) / lanes) *
+                         std::max(1.2 * std::ceil((double)n / 8.0), inputs * (double)busy * (double)n * 16.0 / 3.5e6) + 1.0;
+    if (c < best) {
+      lane = true;
+      team = false;
+      d.S = 1;
+      d.per = per;
+      d.units = units;
+    }
+  }
+  d.inv_per = 1.0 / (double)std::max(1LL, d.per);
+  d.inv_units = 1.0 / (double)d.units;
+  d.inv_S = 1.0 / (double)d.S;
   size_t entry = 0;
-  while (x->l.entries[entry].strided || x->l.entries[entry].fast != fast || x->l.entries[entry].team != team) ++entry;
+  while (x->l.entries[entry].strided || x->l.entries[entry].fast != fast || x->l.entries[entry].team != team ||
+         x->l.entries[entry].lane != lane)
+    ++entry;
   SplitWs w;
-  if (S > 1) {
-    if (units * S > (long long)split_items(x)) {
+  if (d.S > 1) {
+    if (d.units * d.S > (long long)split_items(x)) {
       set_error(err, UNP_INVALID_ARGUMENT, "a split reduction beyond its workspace");
       return UNP_INVALID_ARGUMENT;
     }
-    const size_t bytes = (size_t)(units * S * (inner ? 1 : 64 * v)) * 16;
+    const size_t bytes = (size_t)(d.units * d.S * (inner ? 1 : d.lpr * v)) * 16;
     if (!x->fixed) {
       w = stream_workspace(x, s);
     } else if (f.kind == UNP_FORM_REDUCTION && x->l.red_schedule == 'm' && x->l.rx.plain &&
-               static_fits(x, bytes, false, (size_t)units)) {
+               static_fits(x, bytes, false, (size_t)d.units)) {
       // The plain column reduction takes the static scratch; the others never shared it.
       Ws own;
-      const int32_t rc = workspace(x, bytes, false, (size_t)units, s, own, err);
+      const int32_t rc = workspace(x, bytes, false, (size_t)d.units, s, own, err);
       if (rc != UNP_OK) return rc;
       w.partials = own.ws;
       w.counters = own.counters;
@@ -989,14 +1029,15 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
   waits_host wt = waits_of(x);
   std::vector<void*> params;
   for (uint64_t& p : ptrs) params.push_back(&p);
+  if (!lane && (inner || !team)) {
+    params.push_back(&w.partials);
+    params.push_back(&w.counters);
+    params.push_back(&w.epoch);
+    params.push_back(&wt);
+  }
   params.push_back(&d);
-  params.push_back(&S);
-  if (!inner) params.push_back(&lpr);
-  params.push_back(&w.partials);
-  params.push_back(&w.counters);
-  params.push_back(&w.epoch);
-  params.push_back(&wt);
-  return launch(x, entry, (uint32_t)grid, params.data(), s, err);
+  const unp::Entry& en = x->l.entries[entry];
+  return launch(x, entry, (uint32_t)(cus * (en.blocks_per_cu ? en.blocks_per_cu : x->l.blocks_per_cu)), params.data(), s, err);
 }
 
 // A reduction with a pre-map body over NI inputs or a fused post: NI input buffers of the same

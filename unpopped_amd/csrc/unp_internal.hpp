@@ -30,8 +30,9 @@ struct Entry {
   bool wide = false;  // reduction: the block-per-row schedule (long rows)
   int threads = 0;    // block size of this entry (0: the form's)
   int blocks_per_cu = 0;  // persistent blocks per CU of this entry (0: the form's)
-  bool team = false;      // split reduction, innermost run reduced: a wave per output; elementwise: the
+  bool team = false;      // split reduction: a wave per output or column strip; elementwise: the
                           // tiled entry (vec: its tile's rows); scan: a row in registers
+  bool lane = false;      // split reduction: a lane per output, or per vector of columns
   int cols = 0;           // output columns per block (dequant GEMM decode entries)
   // Reads and writes its buffers through storage-image strides (unp_hip_exec_launch_views with a
   // view that is not dense row-major); never picked for a pointer launch.
@@ -52,12 +53,14 @@ char reduction_schedule(uint32_t mask, int32_t rank);
 
 // The host image of the device's red_axes (the split reductions' argument, passed by value).
 struct red_axes_host {
-  long long nk, nr;
-  long long kext[8], kstr[8];
-  long long rext[8], rstr[8];
-  double kinv[8], rinv[8];
   long long L, runs;
-  long long outs, count;
+  long long count, S;
+  long long per, units;
+  double inv_per, inv_units, inv_S;
+  int32_t nk, nr, lpr, rpi;
+  long long kstr[8], rstr[8];
+  long long kext[8], rext[8];
+  double kinv[8], rinv[8];
 };
 
 // The most chunks a split reduction cuts one output's (or column strip's) positions into.
