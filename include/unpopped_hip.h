@@ -418,6 +418,10 @@ int32_t unp_hip_exec_check(unp_exec* e, unp_error* err);
 /* The last launch's geometry and chosen entry point (for reports). */
 int32_t unp_hip_exec_last_launch(const unp_exec* e, uint32_t grid[3], uint32_t block[3],
                                  char* entry, size_t entry_len);
+/* The last launch's split: the chunks each output's positions (a column strip's rows, a row) were cut
+ * into, and whether blocks shared them (1) or one block walked them all (0: one chunk, or no
+ * workspace). */
+int32_t unp_hip_exec_last_chunks(const unp_exec* e, int64_t* chunks, int32_t* shared);
 void unp_hip_exec_destroy(unp_exec* e);
 
 #ifdef __cplusplus

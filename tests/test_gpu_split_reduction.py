@@ -130,3 +130,110 @@ def test_short_reductions_by_lanes_and_waves(hip_device, shape, axes, entry, dty
     got = H.reduce_expr([x, x], axes, "Sum", X.input(0) * X.input(1)) if dtype == "F32" else None
     if got is not None:
         assert np.array_equal(got, (x.astype(np.int64) ** 2).sum(axis=axes).astype(nt))
+
+
+class Streams(list):
+    """n HIP streams, destroyed at the end."""
+
+    def __init__(self, n):
+        for _ in range(n):
+            st = C.c_void_p()
+            assert _lib.lib().hipStreamCreate(C.byref(st)) == 0
+            self.append(st)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        u.synchronize()
+        for st in self:
+            assert _lib.lib().hipStreamDestroy(st) == 0
+
+
+FORMS = [("column", (4000, 300), (0,)), ("channel", (16, 8, 40000), (0, 2)), ("rows", (3, 60001), (1,))]
+
+
+def fresh(kind, shape, axes):
+    """An executor no launch has been made with yet."""
+    if kind == "rows":
+        stages, epi = X.softmax()
+        k = u.lift_row_reduce("fresh", "F32", 2, stages, epi, launch=H.CALLER_LAUNCH)
+    else:
+        k = u.lift_reduction("fresh", "F32", len(shape), "Sum", axes=axes, launch=H.CALLER_LAUNCH)
+    outs = int(np.prod(shape)) if kind == "rows" else int(np.prod([n for d, n in enumerate(shape) if d not in axes]))
+    return u.Executor(u.HipBackend().lower_kernel(k)), outs
+
+
+@pytest.mark.parametrize("kind,shape,axes", FORMS)
+def test_first_launches_on_new_streams_allocate_nothing(hip_device, kind, shape, axes):
+    """Made while another stream captures in global mode, where an allocation or a synchronisation is an error
+    and ends the capture; each has a workspace, on streams past the executor's own ones too."""
+    x = synth.normal_f32(3, int(np.prod(shape))).reshape(shape)
+    L = _lib.lib()
+    ex, outs = fresh(kind, shape, axes)
+    din, first = u.DeviceBuffer.from_array(x), u.DeviceBuffer(outs * 4)
+    u.synchronize()
+    H.say(f"[case] split launches during another stream's capture: {kind}")
+    with Streams(7) as streams:
+        got = [u.DeviceBuffer(outs * 4) for _ in streams]
+        assert L.hipStreamBeginCapture(streams[0], 0) == 0
+        shared = []
+        try:
+            for st, o in list(zip(streams, got))[1:]:
+                ex.launch(din, o, *shape, stream=st.value)
+                shared.append((ex.last_launch()["shared"], ex.last_launch()["chunks"] > 1))
+        finally:
+            graph = C.c_void_p()
+            ended = L.hipStreamEndCapture(streams[0], C.byref(graph))
+        assert ended == 0 and shared == [(True, True)] * 6
+        L.hipGraphDestroy(graph)
+        ex.launch(din, first, *shape)
+        ex.check()
+        want = first.download(np.uint32, outs)
+        for o in got[1:]:
+            assert np.array_equal(o.download(np.uint32, outs), want)
+
+
+@pytest.mark.parametrize("kind,shape,axes", FORMS)
+def test_overlapping_launches_on_many_streams(hip_device, kind, shape, axes):
+    """Seven streams and the per-thread one, each with its own input, launched on in turn without a wait."""
+    L = _lib.lib()
+    n = int(np.prod(shape))
+    ex, outs = fresh(kind, shape, axes)
+    xs = [u.DeviceBuffer.from_array(synth.normal_f32(60 + i, n)) for i in range(8)]
+    got = [u.DeviceBuffer(outs * 4) for _ in xs]
+    want = []
+    for x, o in zip(xs, got):
+        ex.launch(x, o, *shape)
+        ex.check()
+        want.append(o.download(np.uint32, outs))
+        o.fill(0)
+    u.synchronize()
+    H.say(f"[case] overlapping split launches: {kind}")
+    with Streams(7) as streams:
+        handles = [st.value for st in streams] + [2]  # hipStreamPerThread
+        for _ in range(10):
+            for x, o, st in zip(xs, got, handles):
+                ex.launch(x, o, *shape, stream=st)
+                assert ex.last_launch()["shared"]
+        ex.check()
+    for o, w in zip(got, want):
+        assert np.array_equal(o.download(np.uint32, outs), w)
+
+
+def test_a_stream_per_request_keeps_its_workspace(hip_device):
+    shape, axes = (4000, 300), (0,)
+    ex, outs = fresh("column", shape, axes)
+    x = u.DeviceBuffer.from_array(synth.normal_f32(3, int(np.prod(shape))))
+    o = u.DeviceBuffer(outs * 4)
+    ex.launch(x, o, *shape)
+    ex.check()
+    want = o.download(np.uint32, outs)
+    H.say("[case] a stream per launch")
+    for _ in range(20):
+        o.fill(0)
+        u.synchronize()
+        with Streams(1) as (st,):
+            ex.launch(x, o, *shape, stream=st.value)
+            assert ex.last_launch()["shared"]
+        assert np.array_equal(o.download(np.uint32, outs), want)

@@ -471,7 +471,10 @@ class Executor:
         b = (C.c_uint32 * 3)()
         name = C.create_string_buffer(256)
         _lib.lib().unp_hip_exec_last_launch(self._h, g, b, name, 256)
-        return {"grid": list(g), "block": list(b), "entry": name.value.decode()}
+        chunks, shared = C.c_int64(), C.c_int32()
+        _lib.lib().unp_hip_exec_last_chunks(self._h, C.byref(chunks), C.byref(shared))
+        return {"grid": list(g), "block": list(b), "entry": name.value.decode(), "chunks": int(chunks.value),
+                "shared": bool(shared.value)}
 
     def __del__(self):
         h = getattr(self, "_h", None)

@@ -141,6 +141,7 @@ def lib() -> C.CDLL:
         "unp_hip_exec_set_wait_limit": (i32, [P, u32]),
         "unp_hip_exec_check": (i32, [P, E]),
         "unp_hip_exec_last_launch": (i32, [P, C.POINTER(u32), C.POINTER(u32), C.c_char_p, sz]),
+        "unp_hip_exec_last_chunks": (i32, [P, C.POINTER(C.c_int64), C.POINTER(i32)]),
         "unp_hip_exec_destroy": (None, [P]),
     }
     for name, (res, args) in sig.items():

@@ -86,12 +86,11 @@ struct unp_event {
   hipEvent_t e = nullptr;
 };
 
-// One stream's workspace of a split reduction: launches on a stream follow one another, so each may
-// use the words of the one before it, told apart by the epoch.
-struct StreamWs {
+// A workspace of a split reduction, used by one launch at a time: ticket counters (left zero by every
+// launch), then the partials, told apart from an earlier launch's by the epoch.
+struct SplitSlot {
   hipStream_t stream = nullptr;
-  bool bound = false;             // to `stream`
-  uint8_t* base = nullptr;        // ticket counters (left zero by every launch), then the partials
+  bool bound = false;  // to `stream`, whose launches follow one another
   uint32_t epoch = 0;
 };
 
@@ -106,8 +105,15 @@ struct unp_exec {
   void* ws = nullptr;  // scan: tile status words; full reduction: block partials
   size_t ws_bytes = 0;
   uint32_t* counter = nullptr;
-  // The workspaces of a split reduction, one per stream the executor has launched it on.
-  std::vector<StreamWs> stream_ws;
+  // The workspaces of a split reduction (kSplitSlots of them, allocated with the executor) and the end of
+  // the last launch that used the last one.
+  uint8_t* split_base = nullptr;
+  std::vector<SplitSlot> slots;
+  hipEvent_t slot_done = nullptr;
+  // The last launch's chunks per output (or strip, or row), and whether its blocks shared them.
+  long long chunks = 1;
+  bool shared = false;
+  bool slot_used = false;
   uint32_t epoch = 0;
   uint32_t ticket_base = 0;
   // Bounded waits: the word a kernel that gave up waiting counts into, read and cleared by
@@ -133,9 +139,10 @@ struct unp_exec {
 namespace {
 
 // A split reduction's workspace.  The items (outputs or column strips, times chunks) of a launch that
-// splits are at most kSplitItems = 4 rounds of its grid (split_chunks): each has a ticket counter
-// at most, and its partials: one value, or a strip's 64 * vec of them, in 16 bytes at most.
-constexpr size_t kSplitRounds = 4, kMaxStreams = 4;
+// splits are at most kSplitRounds rounds of its grid (split_chunks): each has a ticket counter
+// at most, and its partials: one value, or a strip's 64 * vec of them, in 16 bytes at most.  Three
+// rounds of 256 blocks of 256 columns fit the static scratch too.
+constexpr size_t kSplitRounds = 3, kSplitSlots = 4;
 bool inner_reduced(const unp::Lowered& l) { return (l.axes_mask >> (l.form.rank - 1)) & 1u; }
 size_t split_items(const unp_exec* x) { return kSplitRounds * (size_t)x->cu_count * (size_t)x->l.blocks_per_cu; }
 size_t split_counter_bytes(const unp_exec* x) { return (split_items(x) * sizeof(uint32_t) + 255) / 256 * 256; }
@@ -152,17 +159,14 @@ bool splits(const unp_exec* x) {
   return x->l.form.kind == UNP_FORM_REDUCTION && (x->l.red_schedule == 'g' || x->l.red_schedule == 'm');
 }
 
-hipError_t add_stream_ws(unp_exec* x) {
-  StreamWs w;
-  hipError_t e = hipMalloc((void**)&w.base, split_bytes(x));
-  if (e != hipSuccess) return e;
-  if ((e = hipMemset(w.base, 0, split_bytes(x))) == hipSuccess) e = hipDeviceSynchronize();
-  if (e != hipSuccess) {
-    hipFree(w.base);
-    return e;
-  }
-  x->stream_ws.push_back(w);
-  return hipSuccess;
+hipError_t make_slots(unp_exec* x) {
+  const size_t bytes = kSplitSlots * split_bytes(x);
+  hipError_t e = hipMalloc((void**)&x->split_base, bytes);
+  if (e == hipSuccess) e = hipMemset(x->split_base, 0, bytes);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&x->slot_done, hipEventDisableTiming);
+  x->slots.resize(kSplitSlots);
+  return e;
 }
 
 }  // namespace
@@ -500,7 +504,7 @@ int32_t unp_hip_exec_create(const unp_generated* g, unp_exec** out, unp_error* e
       per_cu = 0;
     x->resident.push_back(per_cu);
   }
-  if (splits(x) && (e = add_stream_ws(x)) != hipSuccess) {
+  if (splits(x) && (e = make_slots(x)) != hipSuccess) {
     unp_hip_exec_destroy(x);
     return hip_fail(err, "hipMalloc(split reduction workspace)", e);
   }
@@ -513,8 +517,8 @@ void unp_hip_exec_destroy(unp_exec* x) {
   if (!x) return;
   if (x->ws) hipFree(x->ws);
   if (x->counter) hipFree(x->counter);
-  for (const StreamWs& w : x->stream_ws)
-    if (w.base) hipFree(w.base);
+  if (x->split_base) hipFree(x->split_base);
+  if (x->slot_done) hipEventDestroy(x->slot_done);
   if (x->stall) hipFree(x->stall);
   for (void* p : x->stage)
     if (p) hipFree(p);
@@ -555,6 +559,13 @@ int32_t unp_hip_exec_set_timing(unp_exec* x, unp_event* start, unp_event* stop) 
   if (!x || (start == nullptr) != (stop == nullptr)) return UNP_INVALID_ARGUMENT;
   x->t_start = start ? start->e : nullptr;
   x->t_stop = stop ? stop->e : nullptr;
+  return UNP_OK;
+}
+
+int32_t unp_hip_exec_last_chunks(const unp_exec* x, int64_t* chunks, int32_t* shared) {
+  if (!x) return UNP_INVALID_ARGUMENT;
+  if (chunks) *chunks = x->chunks;
+  if (shared) *shared = x->shared ? 1 : 0;
   return UNP_OK;
 }
 
@@ -789,52 +800,64 @@ long long split_chunks(long long units, long long grid, double loads, double spe
   return S;
 }
 
-// The workspace of a split launch on stream s: the stream's own, bound on its first launch (the
-// one made with the executor first, then up to kMaxStreams).  None (null words) for a stream past
-// those, for the per-thread stream (one handle, a stream per thread), under capture (a replay
+// The workspace of a split launch on stream s.  All of them are there from the start, so that a launch
+// neither allocates nor synchronises (which would break another stream's capture).  The first streams
+// an executor is launched on have one each; the last one serves all others in turn, a program's that
+// makes a stream per request among them, and the per-thread stream (one handle, a stream per thread): a
+// launch there waits, on the GPU, for the one before it.  (hipStreamDestroy returns once the stream's work
+// has ended, so a later stream that is given a bound one's handle follows it too.)  A column sum of
+// 12158 x 90 f32 takes 8.5 us on a stream's own and 11.9 in turn, 380 without.  None (null words) under capture (a replay
 // would carry one epoch for ever, and the graph the addresses) and in a no-allocation launch; the
 // kernel then folds all chunks of an output in one block, to the same bits.
 struct SplitWs {
   void* partials = nullptr;
   void* counters = nullptr;
   uint32_t epoch = 0;
+  bool in_turn = false;  // the last one: finish_split marks the launch's end
 };
 
-SplitWs stream_workspace(unp_exec* x, hipStream_t s) {
-  SplitWs w;
-  if (x->fixed || s == hipStreamPerThread) return w;
+int32_t split_workspace(unp_exec* x, hipStream_t s, SplitWs& w, unp_error* err) {
+  if (x->fixed) return UNP_OK;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();  // the null stream while another stream captures: not an error of this launch
-    return w;
+    return UNP_OK;
   }
-  if (st != hipStreamCaptureStatusNone) return w;
-  StreamWs* own = nullptr;
-  for (StreamWs& c : x->stream_ws)
-    if (c.bound && c.stream == s) own = &c;
-  for (StreamWs& c : x->stream_ws)
-    if (!own && !c.bound) own = &c;
-  if (!own) {
-    if (x->stream_ws.size() >= kMaxStreams || add_stream_ws(x) != hipSuccess) {
-      (void)hipGetLastError();
-      return w;
+  if (st != hipStreamCaptureStatusNone) return UNP_OK;
+  size_t at = kSplitSlots - 1;
+  for (size_t i = 0; s != hipStreamPerThread && i < kSplitSlots - 1; ++i)
+    if (!x->slots[i].bound || x->slots[i].stream == s) {
+      at = i;
+      x->slots[i].bound = true;
+      x->slots[i].stream = s;
+      break;
     }
-    own = &x->stream_ws.back();
+  SplitSlot& own = x->slots[at];
+  uint8_t* const base = x->split_base + at * split_bytes(x);
+  w.in_turn = at == kSplitSlots - 1;
+  if (w.in_turn && x->slot_used) {
+    const hipError_t e = hipStreamWaitEvent(s, x->slot_done, 0);
+    if (e != hipSuccess) return hip_fail(err, "hipStreamWaitEvent(split workspace)", e);
   }
-  own->bound = true;
-  own->stream = s;
-  if (own->epoch == 0xffffffffu) {
+  if (own.epoch == 0xffffffffu) {
     // The words start zeroed and no launch has epoch 0; clear them before the epoch wraps.
-    if (hipMemsetAsync(own->base, 0, split_bytes(x), s) != hipSuccess) {
-      (void)hipGetLastError();
-      return w;
-    }
-    own->epoch = 0;
+    const hipError_t e = hipMemsetAsync(base, 0, split_bytes(x), s);
+    if (e != hipSuccess) return hip_fail(err, "hipMemsetAsync(split workspace)", e);
+    own.epoch = 0;
   }
-  w.epoch = ++own->epoch;
-  w.counters = own->base;
-  w.partials = own->base + split_counter_bytes(x);
-  return w;
+  w.epoch = ++own.epoch;
+  w.counters = base;
+  w.partials = base + split_counter_bytes(x);
+  return UNP_OK;
+}
+
+// After the launch's kernels, whether or not they all went out.
+int32_t finish_split(unp_exec* x, const SplitWs& w, hipStream_t s, int32_t rc, unp_error* err) {
+  if (!w.in_turn) return rc;
+  const hipError_t e = hipEventRecord(x->slot_done, s);
+  if (e != hipSuccess) return rc != UNP_OK ? rc : hip_fail(err, "hipEventRecord(split workspace)", e);
+  x->slot_used = true;
+  return rc;
 }
 
 // Appends axis (e, is, os) to a descriptor's list, merged into the previous axis when the two
@@ -1013,13 +1036,13 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
       return UNP_INVALID_ARGUMENT;
     }
     const size_t bytes = (size_t)(d.units * d.S * (inner ? 1 : d.lpr * v)) * 16;
-    if (!x->fixed) {
-      w = stream_workspace(x, s);
-    } else if (f.kind == UNP_FORM_REDUCTION && x->l.red_schedule == 'm' && x->l.rx.plain &&
+    int32_t rc = split_workspace(x, s, w, err);
+    if (rc != UNP_OK) return rc;
+    if (x->fixed && f.kind == UNP_FORM_REDUCTION && x->l.red_schedule == 'm' && x->l.rx.plain &&
                static_fits(x, bytes, false, (size_t)d.units)) {
       // The plain column reduction takes the static scratch; the others never shared it.
       Ws own;
-      const int32_t rc = workspace(x, bytes, false, (size_t)d.units, s, own, err);
+      rc = workspace(x, bytes, false, (size_t)d.units, s, own, err);
       if (rc != UNP_OK) return rc;
       w.partials = own.ws;
       w.counters = own.counters;
@@ -1037,7 +1060,11 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
   }
   params.push_back(&d);
   const unp::Entry& en = x->l.entries[entry];
-  return launch(x, entry, (uint32_t)(cus * (en.blocks_per_cu ? en.blocks_per_cu : x->l.blocks_per_cu)), params.data(), s, err);
+  x->chunks = d.S;
+  x->shared = w.partials != nullptr;
+  const int32_t rc =
+      launch(x, entry, (uint32_t)(cus * (en.blocks_per_cu ? en.blocks_per_cu : x->l.blocks_per_cu)), params.data(), s, err);
+  return finish_split(x, w, s, rc, err);
 }
 
 // A reduction with a pre-map body over NI inputs or a fused post: NI input buffers of the same
@@ -1317,11 +1344,13 @@ int32_t run_row_reduce(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, u
     const size_t first = 7, stages = sp.ops.size();
     const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
     SplitWs w;
-    if (!whole && rows <= kRowChunks / chunks) w = stream_workspace(x, s);
+    if (!whole && rows <= kRowChunks / chunks && (rc = split_workspace(x, s, w, err)) != UNP_OK) return rc;
+    x->chunks = chunks;
+    x->shared = w.partials != nullptr;
     if (!w.partials) return launch(x, first + stages + 1, grid, params.data(), s, err);
     params.push_back(&w.partials);
     for (size_t st = 0; st <= stages && rc == UNP_OK; ++st) rc = launch(x, first + st, grid, params.data(), s, err);
-    return rc;
+    return finish_split(x, w, s, rc, err);
   }
   const size_t entry = cols < vec ? 6 : (aligned ? 0 : 3) + held_by;
   // As many blocks as the CUs hold at once (at most blocks_per_cu each), so no blocks start late
@@ -1946,6 +1975,8 @@ int32_t invalid(unp_error* err, const std::string& what) {
 int32_t begin_launch(unp_exec* x, unp_error* err) {
   set_error(err, UNP_OK, "");
   x->t_first = true;
+  x->chunks = 1;
+  x->shared = false;
   int cur = -1;
   if (hipGetDevice(&cur) != hipSuccess || cur != x->device)
     return invalid(err, "the executor was created on another device");
