@@ -389,10 +389,11 @@ int32_t unp_hip_exec_launch_views(unp_exec* e, const unp_view* views, size_t nvi
                                   size_t nscalars, void* stream, unp_error* err);
 /* No reference counterpart: it exists for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  unp_hip_exec_launch with every
- * workspace the executor would allocate (scan tile status and ticket counter, reduction partials and
- * counters, the dequant GEMM's repacked activations) taken from one static device array of
- * UNP_STATIC_SCRATCH_BYTES per GPU instead; the call allocates and frees nothing.  A launch whose
- * workspace does not fit is refused with UNP_INVALID_ARGUMENT before anything runs.  Each call
+ * workspace the executor would use (scan tile status and ticket counter, reduction partials and
+ * counters, a row reduction's chunk partials, the dequant GEMM's repacked activations) taken from one
+ * static device array of UNP_STATIC_SCRATCH_BYTES per GPU instead; the call allocates and frees nothing.
+ * A launch whose workspace does not fit is refused with UNP_INVALID_ARGUMENT before anything runs; a
+ * split reduction, which can do without one, goes unsplit to the same bits instead.  Each call
  * clears the part of the array it uses on its stream first; calls that overlap on one GPU share the
  * array and race, so a caller serialises them. */
 #define UNP_STATIC_SCRATCH_BYTES (4u << 20)

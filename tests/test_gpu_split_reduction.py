@@ -237,3 +237,22 @@ def test_a_stream_per_request_keeps_its_workspace(hip_device):
             ex.launch(x, o, *shape, stream=st.value)
             assert ex.last_launch()["shared"]
         assert np.array_equal(o.download(np.uint32, outs), want)
+
+
+@pytest.mark.parametrize("kind,shape,axes", FORMS + [("body", (4000, 300), (0,))])
+def test_a_no_allocation_launch_splits_in_the_static_scratch(hip_device, kind, shape, axes):
+    x = u.DeviceBuffer.from_array(synth.normal_f32(3, int(np.prod(shape))))
+    if kind == "body":
+        ex, outs = H.reduce_expr_executor("F32", 2, "Sum", axes, X.input(0) * X.konst(0.75)), shape[1]
+    else:
+        ex, outs = fresh(kind, shape, axes)
+    a, b = u.DeviceBuffer(outs * 4), u.DeviceBuffer(outs * 4)
+    H.say(f"[case] static split launch: {kind}")
+    ex.launch(x, a, *shape)
+    for _ in range(2):
+        b.fill(0)
+        ex.launch_static(x, b, *shape)
+        last = ex.last_launch()
+        ex.check()
+        assert last["shared"] and last["chunks"] > 1
+        assert np.array_equal(b.download(np.uint32, outs), a.download(np.uint32, outs))

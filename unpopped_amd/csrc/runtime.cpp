@@ -807,8 +807,9 @@ long long split_chunks(long long units, long long grid, double loads, double spe
 // launch there waits, on the GPU, for the one before it.  (hipStreamDestroy returns once the stream's work
 // has ended, so a later stream that is given a bound one's handle follows it too.)  A column sum of
 // 12158 x 90 f32 takes 8.5 us on a stream's own and 11.9 in turn, 380 without.  None (null words) under capture (a replay
-// would carry one epoch for ever, and the graph the addresses) and in a no-allocation launch; the
-// kernel then folds all chunks of an output in one block, to the same bits.
+// would carry one epoch for ever, and the graph the addresses); the kernel then folds all chunks of an
+// output in one block, to the same bits.  A no-allocation launch takes `bytes` of partials and `counters`
+// tickets from the static scratch (split_items keeps them within it).
 struct SplitWs {
   void* partials = nullptr;
   void* counters = nullptr;
@@ -816,8 +817,16 @@ struct SplitWs {
   bool in_turn = false;  // the last one: finish_split marks the launch's end
 };
 
-int32_t split_workspace(unp_exec* x, hipStream_t s, SplitWs& w, unp_error* err) {
-  if (x->fixed) return UNP_OK;
+int32_t split_workspace(unp_exec* x, hipStream_t s, size_t bytes, size_t counters, SplitWs& w, unp_error* err) {
+  if (x->fixed) {
+    if (!static_fits(x, bytes, false, counters)) return UNP_OK;
+    Ws own;
+    const int32_t rc = workspace(x, bytes, false, counters, s, own, err);
+    w.partials = own.ws;
+    w.counters = own.counters;
+    w.epoch = 1;
+    return rc;
+  }
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();  // the null stream while another stream captures: not an error of this launch
@@ -1036,18 +1045,8 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
       return UNP_INVALID_ARGUMENT;
     }
     const size_t bytes = (size_t)(d.units * d.S * (inner ? 1 : d.lpr * v)) * 16;
-    int32_t rc = split_workspace(x, s, w, err);
+    const int32_t rc = split_workspace(x, s, bytes, (size_t)d.units, w, err);
     if (rc != UNP_OK) return rc;
-    if (x->fixed && f.kind == UNP_FORM_REDUCTION && x->l.red_schedule == 'm' && x->l.rx.plain &&
-               static_fits(x, bytes, false, (size_t)d.units)) {
-      // The plain column reduction takes the static scratch; the others never shared it.
-      Ws own;
-      rc = workspace(x, bytes, false, (size_t)d.units, s, own, err);
-      if (rc != UNP_OK) return rc;
-      w.partials = own.ws;
-      w.counters = own.counters;
-      w.epoch = 1;
-    }
   }
   waits_host wt = waits_of(x);
   std::vector<void*> params;
@@ -1344,7 +1343,8 @@ int32_t run_row_reduce(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, u
     const size_t first = 7, stages = sp.ops.size();
     const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
     SplitWs w;
-    if (!whole && rows <= kRowChunks / chunks && (rc = split_workspace(x, s, w, err)) != UNP_OK) return rc;
+    if (!whole && rows <= kRowChunks / chunks && (rc = split_workspace(x, s, (size_t)(rows * chunks) * stages * 8, 0, w, err)) != UNP_OK)
+      return rc;
     x->chunks = chunks;
     x->shared = w.partials != nullptr;
     if (!w.partials) return launch(x, first + stages + 1, grid, params.data(), s, err);
