@@ -256,3 +256,43 @@ def test_a_no_allocation_launch_splits_in_the_static_scratch(hip_device, kind, s
         ex.check()
         assert last["shared"] and last["chunks"] > 1
         assert np.array_equal(b.download(np.uint32, outs), a.download(np.uint32, outs))
+
+
+# Every lane layout of the strips: one column, fewer lanes than a wave, ragged, whole strips, several reduced
+# axes, kept axes before the reduced one.
+CAPTURED = [((40000, 1), (0,)), ((40000, 3), (0,)), ((40000, 6), (0,)), ((12158, 90), (0,)), ((9001, 37), (0,)),
+            ((6000, 2050), (0,)), ((3, 20000, 22), (1,)), ((30, 2, 700, 2, 70), (0, 2))]
+
+
+@pytest.mark.parametrize("body", [False, True])
+@pytest.mark.parametrize("shape,axes", CAPTURED)
+def test_captured_column_reductions_replay_to_the_same_bits(hip_device, shape, axes, body):
+    """Captured once and replayed between eager launches: a plain one over one run of axes splits in a workspace
+    of its own, the others fold all chunks of their columns in one block."""
+    x = u.DeviceBuffer.from_array(synth.normal_f32(3, int(np.prod(shape))))
+    outs = int(np.prod([n for d, n in enumerate(shape) if d not in axes]))
+    if body:
+        ex = H.reduce_expr_executor("F32", len(shape), "Sum", axes, X.input(0) * X.konst(0.75))
+    else:
+        ex, _ = fresh("column", shape, axes)
+    L, a, b, graph, exe = _lib.lib(), u.DeviceBuffer(outs * 4), u.DeviceBuffer(outs * 4), C.c_void_p(), C.c_void_p()
+    H.say(f"[case] captured column reduction {shape} over {axes} body={body}")
+    ex.launch(x, a, *shape)
+    ex.check()
+    assert ex.last_launch()["shared"] and ex.last_launch()["chunks"] > 1
+    want = a.download(np.uint32, outs)
+    with Streams(1) as (st,):
+        assert L.hipStreamBeginCapture(st, 0) == 0
+        ex.launch(x, b, *shape, stream=st.value)
+        assert ex.last_launch()["shared"] == (not body and len(axes) == 1)
+        assert L.hipStreamEndCapture(st, C.byref(graph)) == 0
+        assert L.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(4):
+            b.fill(0)
+            u.synchronize()
+            assert L.hipGraphLaunch(exe, st) == 0
+            ex.launch(x, a, *shape)
+            ex.check()
+            assert np.array_equal(b.download(np.uint32, outs), want)
+            assert np.array_equal(a.download(np.uint32, outs), want)
+        assert L.hipGraphExecDestroy(exe) == 0 and L.hipGraphDestroy(graph) == 0

@@ -85,7 +85,7 @@ CHECK_INSTANTIATIONS = r"""
 #include "unp_device.hip"
 #define KB __launch_bounds__(256)
 // The descriptors the host passes by value (runtime.cpp asserts the same sizes for its images).
-static_assert(sizeof(unp::red_axes) == 59 * 8, "red_axes");
+static_assert(sizeof(unp::red_axes) == 60 * 8, "red_axes");
 static_assert(sizeof(unp::red_view) == 44 * 8, "red_view");
 static_assert(sizeof(unp::scan_view) == 29 * 8, "scan_view");
 static_assert(sizeof(unp::gather_view) == 35 * 8, "gather_view");
@@ -99,6 +99,7 @@ extern "C" __global__ void KB c_rx(const int* a, int* b, long long n, unsigned l
 extern "C" __global__ void __launch_bounds__(512) c_rb(const long long* a, long long* b, unsigned long long* p, unsigned* k, unsigned e, unp::waits w, unp::red_axes d) { const long long* in[1] = {a}; unp::xreduce_inner<long long, 1, unp::OP_AND, unp::plain_ops<long long, unp::OP_AND>, 2, 8, 512, 8>(in, b, p, k, e, w, d); }
 extern "C" __global__ void __launch_bounds__(512) c_ro(const float* a, float* b, unsigned long long* p, unsigned* k, unsigned e, unp::waits w, unp::red_axes d) { const float* in[1] = {a}; unp::xreduce_outer<float, 1, unp::OP_SUM, unp::plain_ops<float, unp::OP_SUM>, 4, 512, 8>(in, b, p, k, e, w, d); }
 extern "C" __global__ void __launch_bounds__(512) c_rs(const double* a, double* b, unp::red_axes d) { const double* in[1] = {a}; unp::xreduce_outer_wave<double, 1, unp::OP_SUM, unp::plain_ops<double, unp::OP_SUM>, 2, 512, 8>(in, b, d); }
+extern "C" __global__ void __launch_bounds__(512) c_rz(const int* a, int* b, unp::red_axes d) { const int* in[1] = {a}; unp::xreduce_outer_alone<int, 1, unp::OP_MAX, unp::plain_ops<int, unp::OP_MAX>, 1, 512, 8>(in, b, d); }
 extern "C" __global__ void KB c_rl(const float* a, float* b, unp::red_axes d) { const float* in[1] = {a}; unp::xreduce_lanes<float, 1, unp::OP_SUM, unp::plain_ops<float, unp::OP_SUM>, 4, true, 256>(in, b, d); }
 extern "C" __global__ void KB c_rm(const double* a, double* b, unp::red_axes d) { const double* in[1] = {a}; unp::xreduce_lanes<double, 1, unp::OP_MAX, unp::plain_ops<double, unp::OP_MAX>, 2, false, 256>(in, b, d); }
 extern "C" __global__ void KB c_rq(const float* a, float* b, unp::red_view d) { unp::reduce_serial<float, unp::OP_MAXNUM, 256>(a, b, d); }

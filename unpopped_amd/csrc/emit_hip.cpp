@@ -225,25 +225,27 @@ static void emit_split(std::ostringstream& src, Lowered& L, int32_t dtype, int N
   const bool inner = (L.axes_mask >> (L.form.rank - 1)) & 1u;
   L.threads = 512;
   L.blocks_per_cu = inner ? 2 : 1;
-  enum { Block, Team, Lane };
-  for (int how : {Block, Team, Lane})
+  enum { Block, Team, Lane, Alone };
+  for (int how : {Block, Team, Lane, Alone})
     for (int fast = 1; fast >= 0; --fast) {
+      if (how == Alone && inner) continue;
       Entry e;
       e.fast = fast;
       e.vec = fast ? V : 1;
       e.team = how == Team;
       e.lane = how == Lane;
+      e.wide = how == Alone;
       e.threads = how == Lane ? 1024 : 512;
       e.blocks_per_cu = how == Block ? 0 : 2;
-      e.symbol = L.name + "_" + x + (inner ? "g" : "m") + (how == Team ? "w" : how == Lane ? "l" : "") + (fast ? "v" : "s");
+      e.symbol = L.name + "_" + x + (inner ? "g" : "m") + (how == Team ? "w" : how == Lane ? "l" : how == Alone ? "a" : "") + (fast ? "v" : "s");
       src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << e.symbol << "(";
       for (int k = 0; k < NI; ++k) src << "const " << T << "* in" << k << ", ";
       src << T << "* out, ";
-      const bool plain = how == Lane || (how == Team && !inner);
+      const bool plain = how == Lane || how == Alone || (how == Team && !inner);
       if (!plain) src << "unsigned long long* partials, unsigned* counters, unsigned epoch, unp::waits wt, ";
       src << "unp::red_axes d) {\n  const " << T << "* in[" << NI << "] = {";
       for (int k = 0; k < NI; ++k) src << (k ? ", " : "") << "in" << k;
-      src << "};\n  unp::" << (how == Lane ? "xreduce_lanes<" : inner ? "xreduce_inner<" : how == Team ? "xreduce_outer_wave<" : "xreduce_outer<") << T << ", "
+      src << "};\n  unp::" << (how == Lane ? "xreduce_lanes<" : inner ? "xreduce_inner<" : how == Team ? "xreduce_outer_wave<" : how == Alone ? "xreduce_outer_alone<" : "xreduce_outer<") << T << ", "
           << NI << ", " << op << ", " << ops << ", " << e.vec << ", ";
       if (how == Lane)
         src << (inner ? "true" : "false") << ", 1024>(in, out, d);\n}\n";
@@ -264,6 +266,7 @@ static const char* split_policy(uint32_t mask, int32_t rank) {
 static std::string split_when(const Entry& e) {
   return std::string(e.lane   ? "few positions per output under many outputs; "
                      : e.team ? "few positions per output, or many outputs; "
+                     : e.wide ? "split, without a workspace; "
                               : "") +
          (e.fast ? "innermost run >= vec elements" : "otherwise");
 }

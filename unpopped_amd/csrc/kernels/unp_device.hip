@@ -950,6 +950,7 @@ struct red_axes {
   double inv_per, inv_units, inv_S;
   i32 nk, nr;           // kept / reduced axes besides the innermost run
   i32 lpr, rpi;         // xreduce_outer: lanes per row, rows per load
+  i32 alone, pad;       // xreduce_outer_alone: lanes of a strip
   i64 kstr[8], rstr[8];
   i64 kext[8], rext[8];
   double kinv[8], rinv[8];  // 1 / extent
@@ -1139,8 +1140,6 @@ UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out,
 // partials carry the launch's `epoch`.  6000 x 2050 f32 column norms (49 MB) take 15.6 us, where a wave
 // per column took 59.3; 8192 x 4096 f32 column sums (134 MB) 23.7 launched one after another and 27 on
 // cold caches.
-// Without a workspace (partials null) each block walks all chunks of its strips by itself in the
-// same association.
 //
 // How the lanes of a wave lie on a strip's columns and rows, and their fold of a run of rows.
 template <class T, int NI, int OP, class OPS, int VEC, int U> struct outer_lanes {
@@ -1256,32 +1255,15 @@ UNP_DEV void xreduce_outer(const T* const* __restrict__ in, T* __restrict__ out,
     }
     return r;
   };
-  // One loop for both ways of walking the chunks, as in xreduce_inner.
-  const bool alone = S > 1 && partials == nullptr;
-  const i64 n = alone ? divisor(gridDim.x).quo(d.units - blockIdx.x + gridDim.x - 1) * S : d.units * S;
-  for (i64 it = alone ? 0 : blockIdx.x; it < n; it += alone ? 1 : gridDim.x) {
+  for (i64 it = blockIdx.x; it < d.units * S; it += gridDim.x) {
     i64 s = 0, strip = it, at, cb;
-    if (alone) {
-      by_chunks(it, strip, s);
-      strip = strip * gridDim.x + blockIdx.x;
-    } else if (S > 1) {
-      by_strips(it, s, strip);
-    }
+    if (S > 1) by_strips(it, s, strip);
     by_ncb(strip, at, cb);
     const i64 c0 = cb * cw;
     const bool mine = tid < cw && c0 + tid < B;  // this thread's column
     Ac a = fold_chunk(unravel(at, d.nk, d.kext, d.kstr, d.kinv), c0, s);
     bool done = S == 1;
-    if (alone) {
-      // Chunk s goes to group s % G, as the closing fold below takes it.
-      if (tid < cw) {
-        if (s == 0)
-          for (int g = 0; g < G; ++g) slots[g * cw + tid] = F::identity();
-        Ac* const slot = &slots[(int)(s % G) * cw + tid];
-        *slot = F::apply(*slot, a);
-      }
-      done = s == S - 1;
-    } else if (S > 1) {
+    if (S > 1) {
       // An item's partials: W planes of cw words, a word per column.
       const i64 item = (i64)cw * P::W;
       u64* const strip_p = partials + strip * S * item;
@@ -1328,6 +1310,97 @@ UNP_DEV void xreduce_outer(const T* const* __restrict__ in, T* __restrict__ out,
     }
     if (done && mine) out[at * B + c0 + tid] = xfinish<T, OP, OPS>(a, R);
     __syncthreads();  // sh, slots and last are the next item's
+  }
+}
+
+// The same without a workspace, to the same bits: a block walks all chunks of the columns of `alone` lanes
+// by itself (8, or 4 where that leaves more than half of the CUs idle).  A group of those lanes folds one
+// piece (a chunk's rows of one wave and packed row of xreduce_outer), as many pieces at a time as the block
+// has groups; then its threads put the pieces together in xreduce_outer's order.  `per` and `units` count
+// these narrower strips.  6000 x 2050 f32 column norms, captured: 41.8 us (191.8 with the wide strips in one
+// block each), 8192 x 4096 44.6 (194.4).
+template <class T, int NI, int OP, class OPS, int VEC, int THREADS, int U>
+UNP_DEV void xreduce_outer_alone(const T* const* __restrict__ in, T* __restrict__ out, const red_axes& d) {
+  typedef typename OPS::acc Ac;
+  typedef fold<Ac, OP> F;
+  constexpr int WAVES = 8;  // of xreduce_outer's blocks, whose 512 threads also set the groups that fold the chunks
+  __shared__ Ac sh[THREADS * VEC], slots[512];
+  const int tid = threadIdx.x;
+  const i64 R = d.count, S = d.S;
+  const int aw = d.alone, cols = aw * VEC, rpi = d.rpi, G = 512 / (d.lpr * VEC);
+  const int PC = WAVES * rpi, CP = THREADS / aw / PC;  // pieces of a chunk, chunks at a time
+  const divisor by_per(d.per, d.inv_per), by_chunks(S, d.inv_S);
+  const int gi = (int)((u32)tid / (u32)aw), cl = tid - gi * aw;            // this lane's group and vector
+  const int c = (int)((u32)gi / (u32)PC), p = (gi - c * PC) / WAVES, w = (gi - c * PC) % WAVES;  // its chunk and piece
+  const int row = (int)((u32)tid / (u32)cols), col = tid - row * cols;     // a thread per value below
+  for (i64 strip = blockIdx.x; strip < d.units; strip += gridDim.x) {
+    i64 at, cb;
+    by_per(strip, at, cb);
+    const i64 c0 = cb * cols, b0 = c0 + (i64)cl * VEC;
+    const bool live = b0 < d.L && c < CP;
+    const i64 lc = live ? (b0 + VEC <= d.L ? b0 : d.L - VEC) : 0;
+    const int skip = (int)(b0 - lc);
+    const i64 base = unravel(at, d.nk, d.kext, d.kstr, d.kinv) + lc;
+    Ac slot = F::identity();  // group `row`'s fold of column `col`
+    for (i64 s0 = 0; s0 < S; s0 += CP) {
+      const i64 s = s0 + c;
+      if (live && s < S) {
+        const i64 i0 = by_chunks.quo(R * s), i1 = by_chunks.quo(R * (s + 1));
+        const i64 w0 = i0 + (i1 - i0) * w / WAVES, w1 = i0 + (i1 - i0) * (w + 1) / WAVES;
+        Ac a[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) a[e] = F::identity();
+        for (i64 i = w0 + p; i < w1; i += U * rpi) {
+          vec<T, VEC> x[U][NI];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const i64 rr = i + u * rpi < w1 ? i + u * rpi : i;  // past the piece a row of it is read and ignored
+            const i64 off = base + (d.nr <= 1 ? rr * d.rstr[0] : unravel(rr, d.nr, d.rext, d.rstr, d.rinv));
+#pragma unroll
+            for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+              const Ac b = xfold<T, NI, OP, OPS, VEC>(a[e], x[u], e);
+              a[e] = i + u * rpi < w1 ? b : a[e];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          if (e >= skip) sh[gi * cols + cl * VEC + e - skip] = a[e];
+      }
+      __syncthreads();
+      // Value (chunk k, packed row q) of column `col`: the waves' pieces in order, then a tree over q.
+      const int k = (int)((u32)row / (u32)rpi), q = row - k * rpi;
+      Ac* const v = sh + (k * PC + q * WAVES) * cols + col;
+      if (k < CP) {
+        Ac r = v[0];
+        for (int i = 1; i < WAVES; ++i) r = F::apply(r, v[i * cols]);
+        v[0] = r;
+      }
+      for (int n = rpi; n > 1;) {
+        const int half = (n + 1) / 2;
+        __syncthreads();
+        if (k < CP && q < n - half) v[0] = F::apply(v[0], v[half * WAVES * cols]);
+        n = half;
+      }
+      __syncthreads();
+      if (row < G)
+        for (int i = 0; i < CP && s0 + i < S; ++i)
+          if ((int)((s0 + i) % G) == row) slot = F::apply(slot, sh[i * PC * cols + col]);
+      __syncthreads();  // sh is the next pass's
+    }
+    if (row < G) slots[row * cols + col] = slot;
+    for (int n = G; n > 1;) {
+      const int half = (n + 1) / 2;
+      __syncthreads();
+      if (row < n - half) slots[row * cols + col] = F::apply(slots[row * cols + col], slots[(row + half) * cols + col]);
+      n = half;
+    }
+    if (row == 0 && c0 + col < d.L) out[at * d.L + c0 + col] = xfinish<T, OP, OPS>(slots[col], R);
+    __syncthreads();  // slots are the next strip's
   }
 }
 

@@ -143,6 +143,8 @@ namespace {
 // at most, and its partials: one value, or a strip's 64 * vec of them, in 16 bytes at most.  Three
 // rounds of 256 blocks of 256 columns fit the static scratch too.
 constexpr size_t kSplitRounds = 3, kSplitSlots = 4;
+// One more for captured column reductions (below).
+constexpr size_t kCaptureSlot = kSplitSlots;
 bool inner_reduced(const unp::Lowered& l) { return (l.axes_mask >> (l.form.rank - 1)) & 1u; }
 size_t split_items(const unp_exec* x) { return kSplitRounds * (size_t)x->cu_count * (size_t)x->l.blocks_per_cu; }
 size_t split_counter_bytes(const unp_exec* x) { return (split_items(x) * sizeof(uint32_t) + 255) / 256 * 256; }
@@ -160,7 +162,7 @@ bool splits(const unp_exec* x) {
 }
 
 hipError_t make_slots(unp_exec* x) {
-  const size_t bytes = kSplitSlots * split_bytes(x);
+  const size_t bytes = (kSplitSlots + 1) * split_bytes(x);
   hipError_t e = hipMalloc((void**)&x->split_base, bytes);
   if (e == hipSuccess) e = hipMemset(x->split_base, 0, bytes);
   if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -806,10 +808,14 @@ long long split_chunks(long long units, long long grid, double loads, double spe
 // makes a stream per request among them, and the per-thread stream (one handle, a stream per thread): a
 // launch there waits, on the GPU, for the one before it.  (hipStreamDestroy returns once the stream's work
 // has ended, so a later stream that is given a bound one's handle follows it too.)  A column sum of
-// 12158 x 90 f32 takes 8.5 us on a stream's own and 11.9 in turn, 380 without.  None (null words) under capture (a replay
-// would carry one epoch for ever, and the graph the addresses); the kernel then folds all chunks of an
-// output in one block, to the same bits.  A no-allocation launch takes `bytes` of partials and `counters`
-// tickets from the static scratch (split_items keeps them within it).
+// 12158 x 90 f32 takes 8.5 us on a stream's own and 11.9 in turn.
+//
+// Under capture a replay would carry one epoch for ever.  A plain column reduction, whose launches have
+// always shared the executor's words, takes a workspace kept for captures, cleared by kernels in front
+// of it.  The other forms' graphs may be replayed on several streams at once, as they kept no words before
+// they were split: none (null words), and a block folds all chunks of its outputs, to the same bits.
+// A no-allocation launch takes `bytes` of partials and `counters` tickets from the static scratch
+// (split_items keeps them within it).
 struct SplitWs {
   void* partials = nullptr;
   void* counters = nullptr;
@@ -832,7 +838,15 @@ int32_t split_workspace(unp_exec* x, hipStream_t s, size_t bytes, size_t counter
     (void)hipGetLastError();  // the null stream while another stream captures: not an error of this launch
     return UNP_OK;
   }
-  if (st != hipStreamCaptureStatusNone) return UNP_OK;
+  if (st != hipStreamCaptureStatusNone) {
+    if (x->l.form.kind != UNP_FORM_REDUCTION || x->l.red_schedule != 'm' || !x->l.rx.plain) return UNP_OK;
+    uint8_t* const base = x->split_base + kCaptureSlot * split_bytes(x);
+    w.counters = base;
+    w.partials = base + split_counter_bytes(x);
+    w.epoch = 1;
+    const int32_t rc = unp::scratch_clear(base, up256(counters * sizeof(uint32_t)), s, err);
+    return rc != UNP_OK ? rc : unp::scratch_clear(w.partials, up256(bytes), s, err);
+  }
   size_t at = kSplitSlots - 1;
   for (size_t i = 0; s != hipStreamPerThread && i < kSplitSlots - 1; ++i)
     if (!x->slots[i].bound || x->slots[i].stream == s) {
@@ -910,7 +924,7 @@ static_assert(sizeof(unp::red_view_host) == 44 * 8, "red_view_host mirrors the d
 static_assert(sizeof(unp::scan_view_host) == 29 * 8, "scan_view_host mirrors the device's scan_view");
 static_assert(sizeof(unp::ew_tile_view_host) == 114 * 8, "ew_tile_view_host mirrors the device's ew_tile_view");
 static_assert(sizeof(unp::gather_view_host) == 35 * 8, "gather_view_host mirrors the device's gather_view");
-static_assert(sizeof(unp::red_axes_host) == 59 * 8, "red_axes_host mirrors the device's red_axes");
+static_assert(sizeof(unp::red_axes_host) == 60 * 8, "red_axes_host mirrors the device's red_axes");
 
 int32_t launch(unp_exec* x, size_t entry, uint32_t grid, void** params, hipStream_t s, unp_error* err) {
   const uint32_t threads = (uint32_t)(x->l.entries[entry].threads ? x->l.entries[entry].threads : x->l.threads);
@@ -1031,13 +1045,8 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
       d.units = units;
     }
   }
-  d.inv_per = 1.0 / (double)std::max(1LL, d.per);
   d.inv_units = 1.0 / (double)d.units;
   d.inv_S = 1.0 / (double)d.S;
-  size_t entry = 0;
-  while (x->l.entries[entry].strided || x->l.entries[entry].fast != fast || x->l.entries[entry].team != team ||
-         x->l.entries[entry].lane != lane)
-    ++entry;
   SplitWs w;
   if (d.S > 1) {
     if (d.units * d.S > (long long)split_items(x)) {
@@ -1048,10 +1057,24 @@ int32_t run_split(unp_exec* x, const std::vector<int64_t>& ext, std::vector<uint
     const int32_t rc = split_workspace(x, s, bytes, (size_t)d.units, w, err);
     if (rc != UNP_OK) return rc;
   }
+  const bool alone = !inner && d.S > 1 && !w.partials;
+  if (alone) {
+    for (int32_t lanes : {8, 4}) {
+      d.alone = std::min(lanes, d.lpr);
+      d.per = (d.L + d.alone * v - 1) / (d.alone * v);
+      d.units = d.runs * d.per;
+      if (2 * d.units >= cus) break;
+    }
+  }
+  d.inv_per = 1.0 / (double)std::max(1LL, d.per);
+  size_t entry = 0;
+  while (x->l.entries[entry].strided || x->l.entries[entry].fast != fast || x->l.entries[entry].team != team ||
+         x->l.entries[entry].lane != lane || x->l.entries[entry].wide != alone)
+    ++entry;
   waits_host wt = waits_of(x);
   std::vector<void*> params;
   for (uint64_t& p : ptrs) params.push_back(&p);
-  if (!lane && (inner || !team)) {
+  if (!lane && !alone && (inner || !team)) {
     params.push_back(&w.partials);
     params.push_back(&w.counters);
     params.push_back(&w.epoch);

@@ -27,7 +27,7 @@ struct Entry {
   int k = 1;          // vectors per lane per tile (scan)
   int wpb = 1;        // waves per ticket group (scan)
   bool fast = false;  // the 16-byte-aligned path
-  bool wide = false;  // reduction: the block-per-row schedule (long rows)
+  bool wide = false;  // row fold: the block-per-row schedule (long rows); outer reduction: no workspace
   int threads = 0;    // block size of this entry (0: the form's)
   int blocks_per_cu = 0;  // persistent blocks per CU of this entry (0: the form's)
   bool team = false;      // split reduction: a wave per output or column strip; elementwise: the
@@ -57,7 +57,7 @@ struct red_axes_host {
   long long count, S;
   long long per, units;
   double inv_per, inv_units, inv_S;
-  int32_t nk, nr, lpr, rpi;
+  int32_t nk, nr, lpr, rpi, alone, pad;
   long long kstr[8], rstr[8];
   long long kext[8], rext[8];
   double kinv[8], rinv[8];
