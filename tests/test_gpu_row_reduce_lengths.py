@@ -14,6 +14,11 @@ from unpopped_amd import expr as X, forms as H
 pytestmark = pytest.mark.gpu
 
 
+def ran(ex):
+    """The last launch's entry, without the kernel's name."""
+    return ex.last_launch()["entry"][len(ex.kernel.name):]
+
+
 @pytest.mark.parametrize("rows,cols", [(3, 1), (5, 3), (4, 4), (3, 5), (2, 1023), (2300, 37), (3, 4095), (3, 4097),
                                        (2, 8191), (2, 8193), (600, 8195), (2, 16383), (2, 16385), (1, 50001),
                                        (3, 20480), (1, 300001), (520, 16388)])
@@ -66,9 +71,9 @@ def test_two_inputs_nan_and_infinities_in_chunks(hip_device):
     assert np.array_equal(H.row_reduce([a, b], stages, epi), want, equal_nan=True)
 
 
-@pytest.mark.parametrize("cols", [257, 1281, 4353, 8193])
+@pytest.mark.parametrize("cols,entry", [(257, "_s"), (1281, "_s"), (2305, "_c4_s"), (4353, "_c_s"), (8193, "_c512_s")])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-def test_in_place_on_an_input_only_the_epilogue_reads(hip_device, cols, dtype):
+def test_in_place_on_an_input_only_the_epilogue_reads(hip_device, cols, entry, dtype):
     """Ragged rows whose shifted last vector begins a wave: the elements it shares are another wave's, which
     may have stored them before this one loads them."""
     if dtype == np.float64:
@@ -83,4 +88,31 @@ def test_in_place_on_an_input_only_the_epilogue_reads(hip_device, cols, dtype):
     da, db = u.DeviceBuffer.from_array(a), u.DeviceBuffer.from_array(b)
     ex.launch(da, db, db, rows, cols)
     u.synchronize()
+    assert ran(ex) == entry
     assert np.array_equal(db.download(dtype, b.size).reshape(b.shape), oracle.row_reduce([a, b], stages, epi))
+
+
+# The entry at the ends of every range, for a chain that keeps a stage's values (softmax) and one that does not.
+@pytest.mark.parametrize("which,rows,cols,shift,entry", [
+    ("softmax", 9, 3, 0, "_s"), ("softmax", 9, 447, 0, "_s"), ("softmax", 9, 448, 0, "_c4"), ("softmax", 9, 448, 4, "_c4_s"),
+    ("softmax", 9, 449, 0, "_c4_s"), ("softmax", 9, 4096, 0, "_c4"), ("softmax", 9, 4095, 0, "_c4_s"),
+    ("softmax", 9, 4097, 0, "_c_s"), ("softmax", 9, 4100, 0, "_c"), ("softmax", 9, 8191, 0, "_c_s"),
+    ("softmax", 9, 8192, 0, "_c"), ("softmax", 9, 8196, 0, "_c512_v"), ("softmax", 9, 8195, 0, "_c512_s"),
+    ("softmax", 9, 16384, 0, "_c512_v"), ("softmax", 9, 16384, 4, "_c512_s"), ("softmax", 9, 16385, 0, "_p_v"),
+    ("softmax", 447, 16388, 0, "_p_v"), ("softmax", 448, 16388, 0, "_a_v"), ("softmax", 449, 16389, 4, "_a_v"),
+    ("rms_norm", 9, 2047, 0, "_s"), ("rms_norm", 9, 2049, 0, "_c4_s"), ("rms_norm", 9, 2048, 4, "_c4_s"),
+    ("rms_norm", 9, 64, 0, "_c4"), ("rms_norm", 9, 64, 4, "_s"), ("rms_norm", 3, 70001, 4, "_p_v"),
+])
+def test_the_entry_follows_the_length_and_the_alignment(hip_device, which, rows, cols, shift, entry):
+    stages, epi = getattr(X, which)()
+    x = np.random.default_rng(44).normal(size=(rows, cols)).astype(np.float32)
+    ex = H.row_reduce_executor("F32", 2, stages, epi)
+    H.say(f"[case] row_reduce entry {which} {rows}x{cols} +{shift}")
+    src, dst = u.DeviceBuffer(x.nbytes + 64), u.DeviceBuffer(x.nbytes + 64)
+    src.at(shift).upload(x)
+    ex.launch(src.at(shift), dst.at(shift), rows, cols)
+    u.synchronize()
+    assert ran(ex) == entry
+    assert ex.last_launch()["shared"] == (entry == "_p_v")
+    few = slice(0, 9)
+    assert ulps(dst.at(shift).download(np.float32, x.size).reshape(x.shape)[few], oracle.row_reduce([x[few]], stages, epi)).max() <= 2

@@ -1833,6 +1833,7 @@ int32_t lower_row_reduce(const RowReduceSpec& sp, Lowered& L, std::string& why) 
   src << header(L.name, f);
   src << "struct " << ops << " {\n  static constexpr int op[" << NS << "] = {";
   for (size_t st = 0; st < NS; ++st) src << (st ? ", " : "") << sp.ops[st];
+  L.rr_cached = cached >= 0;
   src << "};\n  static constexpr int cached = " << cached << ";\n"
       << "  template <int S> static __device__ __forceinline__ double pre(const double* x, const double* r);\n"
       << "  static __device__ __forceinline__ double epi(const double* x, const double* r) { (void)x; (void)r; return "
@@ -1912,11 +1913,11 @@ int32_t lower_row_reduce(const RowReduceSpec& sp, Lowered& L, std::string& why) 
       if (!in(e)) continue;
       j << (first ? "" : ",") << "{\"symbol\":\"" << e.symbol << "\",\"vec\":" << e.vec
         << ",\"row_in_registers\":" << (e.k ? "true" : "false") << ",\"when\":\""
-        << (e.team ? (e.symbol == L.name + "_a_v" ? "longer rows, two or more per CU, or without a workspace"
+        << (e.team ? (e.symbol == L.name + "_a_v" ? "longer rows, 7 for every 4 CUs or more, or without a workspace"
                                                   : "longer rows: the stages in order, then the epilogue")
             : e.threads == 512 ? "256 * vec * 8 < cols <= 512 * vec * 8"
             : e.k ? (e.k == 4 ? "vec <= cols <= 256 * vec * 4" : "256 * vec * 4 < cols <= 256 * vec * 8")
-                  : "cols < vec")
+                  : std::string("cols < vec, or unaligned and cols < ") + (L.rr_cached ? "448" : "512 * vec"))
         << (e.k ? (e.fast ? ", cols % vec == 0 and every buffer 16-byte aligned" : ", otherwise") : "") << "\"}";
       first = false;
     }

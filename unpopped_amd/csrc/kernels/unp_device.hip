@@ -4131,10 +4131,10 @@ UNP_DEV void rr_stage(const T* const* rin, const vec<T, VEC> (&xr)[NI][R > 0 ? R
         fold_vec(xv, 0);
       }
     }
-    if constexpr (RAG && R > 0 && S + 1 == NS) {
+    if constexpr (RAG && R > 0 && S == 0) {
       // A shifted last vector shares elements with another lane's, and in place that lane may be in a wave
-      // that stores first: every input of the row has landed in this wave, also one that only the
-      // epilogue reads, before the last barrier lets any wave on to its stores.
+      // that stores first: every input of the row has landed in this wave, also one that no stage waits
+      // for, before the first barrier.
 #pragma unroll
       for (int k = 0; k < NI; ++k)
 #pragma unroll
@@ -4267,13 +4267,14 @@ template <class T, int NI, int NS, class OPS, int THREADS, int VEC> struct rr_ch
   const T* const* in;
   T* out;
   i64 cols, C, nvec;
+  divisor by_chunks;
   UNP_DEV rr_chunks(const T* const* in_, T* out_, i64 cols_, i64 C_)
-      : in(in_), out(out_), cols(cols_), C(C_), nvec((cols_ + VEC - 1) / VEC) {}
+      : in(in_), out(out_), cols(cols_), C(C_), nvec((cols_ + VEC - 1) / VEC), by_chunks(C_) {}
 
   // fn(vector's first element, its leading elements that are another vector's, the inputs) over
   // chunk c of a row, R vectors of each input in flight.
   template <class Fn> UNP_DEV void each(i64 row, i64 c, Fn&& fn) const {
-    const i64 v0 = nvec * c / C, v1 = nvec * (c + 1) / C;
+    const i64 v0 = by_chunks.quo(nvec * c), v1 = by_chunks.quo(nvec * (c + 1));
     for (i64 v = v0; v < v1; v += THREADS * R) {
       vec<T, VEC> x[R][NI];
       i64 at[R];
@@ -4292,8 +4293,8 @@ template <class T, int NI, int NS, class OPS, int THREADS, int VEC> struct rr_ch
     }
   }
 
-  // Chunk c of a row folded by stage S, in every thread (`sh`: a slot per wave).
-  template <int S> UNP_DEV double fold(i64 row, i64 c, const double (&red)[NS], double* sh) const {
+  // Chunk c of a row folded by stage S over each wave.
+  template <int S> UNP_DEV double fold(i64 row, i64 c, const double (&red)[NS]) const {
     typedef unp::fold<double, OPS::op[S]> F;
     double acc = F::identity();
     each(row, c, [&](i64, int skip, const vec<T, VEC> (&v)[NI]) {
@@ -4307,7 +4308,15 @@ template <class T, int NI, int NS, class OPS, int THREADS, int VEC> struct rr_ch
         acc = e >= skip ? b : acc;
       }
     });
-    return block_reduce<double, OPS::op[S], THREADS>(acc, sh);
+    return wave_reduce<double, OPS::op[S]>(acc);
+  }
+
+  // A chunk's waves, in wave order.
+  template <int S> static UNP_DEV double meet(const double* w) {
+    double a = w[0];
+#pragma unroll
+    for (int i = 1; i < THREADS / 64; ++i) a = unp::fold<double, OPS::op[S]>::apply(a, w[i]);
+    return a;
   }
 
   // Stage S of a row from its chunks' partials, in every lane.
@@ -4346,25 +4355,26 @@ template <class T, int NI, int NS, class OPS, int THREADS, int VEC> struct rr_ch
 template <class T, int NI, int NS, class OPS, int THREADS, int VEC, int S>
 UNP_DEV void rr_chunk_stage(const T* const* in, T* out, i64 rows, i64 cols, i64 C, double* part) {
   const rr_chunks<T, NI, NS, OPS, THREADS, VEC> ch(in, out, cols, C);
-  __shared__ double sh[THREADS / 64];
-  const divisor by_chunks(C);
-  for (i64 item = blockIdx.x; item < rows * C; item += gridDim.x) {
+  __shared__ double sh[2][THREADS / 64];
+  int par = 0;
+  for (i64 item = blockIdx.x; item < rows * C; item += gridDim.x, par ^= 1) {
     i64 row, c;
-    by_chunks(item, row, c);
+    ch.by_chunks(item, row, c);
     double red[NS] = {};
     unroll_for<S>([&](auto t) { red[t.value] = ch.template finish<t.value>(part + (t.value * rows + row) * C); });
-    const double a = ch.template fold<S>(row, c, red, sh);
-    if (threadIdx.x == 0) part[(S * rows + row) * C + c] = a;
+    const double a = ch.template fold<S>(row, c, red);
+    if ((threadIdx.x & 63) == 0) sh[par][threadIdx.x >> 6] = a;
+    __syncthreads();  // the other half is the next item's; this one's reader passes its barrier first
+    if (threadIdx.x == 0) part[(S * rows + row) * C + c] = ch.template meet<S>(sh[par]);
   }
 }
 
 template <class T, int NI, int NS, class OPS, int THREADS, int VEC>
 UNP_DEV void rr_chunk_epilogue(const T* const* in, T* out, i64 rows, i64 cols, i64 C, const double* part) {
   const rr_chunks<T, NI, NS, OPS, THREADS, VEC> ch(in, out, cols, C);
-  const divisor by_chunks(C);
   for (i64 item = blockIdx.x; item < rows * C; item += gridDim.x) {
     i64 row, c;
-    by_chunks(item, row, c);
+    ch.by_chunks(item, row, c);
     double red[NS];
     unroll_for<NS>([&](auto t) { red[t.value] = ch.template finish<t.value>(part + (t.value * rows + row) * C); });
     ch.epilogue(row, c, red);
@@ -4374,14 +4384,20 @@ UNP_DEV void rr_chunk_epilogue(const T* const* in, T* out, i64 rows, i64 cols, i
 template <class T, int NI, int NS, class OPS, int THREADS, int VEC>
 UNP_DEV void rr_chunk_rows(const T* const* in, T* out, i64 rows, i64 cols, i64 C) {
   const rr_chunks<T, NI, NS, OPS, THREADS, VEC> ch(in, out, cols, C);
-  __shared__ double sh[THREADS / 64], part[kMaxChunks];
+  constexpr int WAVES = THREADS / 64;
+  static_assert(THREADS >= kMaxChunks, "a thread per chunk");
+  __shared__ double sh[kMaxChunks][WAVES], part[kMaxChunks];
+  const int tid = threadIdx.x;
   for (i64 row = blockIdx.x; row < rows; row += gridDim.x) {
     double red[NS] = {};
     unroll_for<NS>([&](auto t) {
+      // No wave waits for the others between the chunks.
       for (i64 c = 0; c < C; ++c) {
-        const double a = ch.template fold<t.value>(row, c, red, sh);
-        if (threadIdx.x == 0) part[c] = a;
+        const double a = ch.template fold<t.value>(row, c, red);
+        if ((tid & 63) == 0) sh[c][tid >> 6] = a;
       }
+      __syncthreads();
+      if (tid < C) part[tid] = ch.template meet<t.value>(sh[tid]);
       __syncthreads();
       red[t.value] = ch.template finish<t.value>(part);
       __syncthreads();  // `part` is the next stage's

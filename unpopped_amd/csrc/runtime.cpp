@@ -1357,11 +1357,12 @@ int32_t run_row_reduce(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, u
   // stage, the epilogue, and the whole row in one block.
   const size_t held_by = cols <= 256LL * vec * 4 ? 0 : cols <= 256LL * vec * 8 ? 1 : 2;
   if (cols > 512LL * vec * 8) {
-    // Two rows per CU or more: each in one block, which finds them in its caches again (600 x 40000 f32
-    // softmax 86 us, 96 in chunks of 4096); fewer: chunks of up to four vectors per thread of a block, on every CU.
-    const bool whole = rows >= 2LL * x->cu_count;
-    const long long nvec = (cols + vec - 1) / vec, most = whole ? 8192 : 1024;
-    long long chunks = std::min(unp::kMaxChunks, (nvec + most - 1) / most);
+    // Seven rows for every four CUs or more: each in one block, which finds them in its caches again
+    // (33000 f32 softmax: 450 rows 56 us, 59 in chunks; 400 rows 56 and 52); fewer: chunks of up to four
+    // vectors per thread of a block, on every CU.
+    const bool whole = 4 * rows >= 7LL * x->cu_count;
+    const long long nvec = (cols + vec - 1) / vec;
+    long long chunks = whole ? 1 : std::min(unp::kMaxChunks, (nvec + 1023) / 1024);
     params.push_back(&chunks);
     const size_t first = 7, stages = sp.ops.size();
     const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
@@ -1375,7 +1376,13 @@ int32_t run_row_reduce(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, u
     for (size_t st = 0; st <= stages && rc == UNP_OK; ++st) rc = launch(x, first + st, grid, params.data(), s, err);
     return finish_split(x, w, s, rc, err);
   }
-  const size_t entry = cols < vec ? 6 : (aligned ? 0 : 3) + held_by;
+  // The in-register entries work through all four vectors of a thread however few of them the row has,
+  // so a short unaligned row is quicker element by element: f32 RMS norms of 63492 x 63 33.2 us (149.6 in
+  // registers), 3910 x 1023 9.2 (13.2), 1332 x 3001 11.2 (7.6).  Where a stage's values are kept for the
+  // epilogue the passes would work them out twice: softmax 15686 x 255 28.4 (31.5), 7827 x 511 19.4 (20.0),
+  // 3910 x 1023 18.9 (13.0).
+  const bool few = !aligned && cols < (x->l.rr_cached ? 448 : 512 * vec);
+  const size_t entry = few || cols < vec ? 6 : (aligned ? 0 : 3) + held_by;
   // As many blocks as the CUs hold at once (at most blocks_per_cu each), so no blocks start late
   // as a tail that runs at a fraction of the occupancy.
   const int held = x->resident[entry];

@@ -174,6 +174,7 @@ struct Lowered {
   bool serial_scan = false;
   int32_t scan_axis = 0;
   RowReduceSpec rr;  // UNP_FORM_ROW_REDUCE only
+  bool rr_cached = false;  // its in-register entries keep a stage's values for the epilogue
   ReductionExpr rx;  // UNP_FORM_REDUCTION and UNP_FORM_SCAN: the pre-map body and the post
   GatherExpr gx;     // UNP_FORM_GATHER: the inputs and body
   ElementwiseExpr ew;  // UNP_FORM_ELEMENTWISE: the inputs, their permutations and the body
