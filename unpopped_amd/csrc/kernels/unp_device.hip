@@ -511,7 +511,9 @@ UNP_DEV void rowreduce_wave(const T* __restrict__ in, T* __restrict__ out0, T* _
       }
     }
     if constexpr (RAG) {
-      if (cols < VEC) {  // less than a vector: an element per lane
+      // An element per lane at most, also where a row is less than a vector (10^6 rows of 3 f64 322 us, 388
+      // by vectors; 100000 of 7 f32 25.5, 36.4).
+      if (cols <= 64) {
         if (lane < cols) {
           a0 = F0::apply(a0, (A0)p[lane]);
           if constexpr (NOUT > 1) a1 = F1::apply(a1, (A1)p[lane]);
