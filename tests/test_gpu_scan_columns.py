@@ -92,3 +92,24 @@ def test_every_strip_is_scanned_at_any_grid(hip_device, grid, strips):
         assert np.array_equal(dst.download(np.int32, x.size).reshape(s, b), np.cumsum(x, axis=0, dtype=np.int32))
     finally:
         L.unp_hip_module_unload(m)
+
+
+# A strip per CU at most, two over 200 rows, four over 512, each at its last strip and the next; rows of half a
+# strip; a last strip of less than a vector in place.
+@pytest.mark.parametrize("a,s,b,in_place,tail", [
+    (1, 16, 64 * 256, False, "_c"), (1, 16, 64 * 256 + 1, False, "_q"), (1, 199, 64 * 300, False, "_q"),
+    (1, 200, 64 * 300, False, "_c"), (1, 200, 64 * 512, False, "_c"), (1, 200, 64 * 513, False, "_q"),
+    (2, 512, 64 * 400, False, "_c"), (1, 511, 64 * 600, False, "_q"), (1, 512, 64 * 1025, False, "_q"),
+    (1, 15, 64, False, "_q"), (1, 16, 32, False, "_c"), (1, 16, 31, False, "_q"), (300, 20, 33, False, "_q"),
+    (1, 100, 65, False, "_c"), (1, 100, 65, True, "_q"), (1, 100, 68, True, "_c"),
+])
+def test_the_entry_follows_the_strips(hip_device, a, s, b, in_place, tail):
+    x = values("I32", a * s * b).reshape(a, s, b)
+    ex = H.executor(kind="scan", dtype="I32", rank=3, op="Sum", axis=1, exclusive=False, reverse=False)
+    H.say(f"[case] column scan entry {a}x{s}x{b} in_place={in_place}")
+    src = u.DeviceBuffer.from_array(x)
+    dst = src if in_place else u.DeviceBuffer(x.nbytes)
+    ex.launch(src, dst, a, s, b)
+    u.synchronize()
+    assert ex.last_launch()["entry"] == ex.kernel.name + tail
+    assert np.array_equal(dst.download(np.int32, x.size).reshape(x.shape), np.cumsum(x, axis=1, dtype=np.int32))

@@ -548,7 +548,7 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
     j << "],\"launch\":{\"block\":[1024,1,1],\"grid\":\"cu_count*1\",\"grid_policy\":\"device-class constant; one "
       << "lane per column of the input seen as A x S x B around the scanned axis, lanes or blocks of 64 columns stride "
       << "over the columns\"},\"entries\":[{\"symbol\":\"" << c.symbol
-      << "\",\"block\":576,\"when\":\"B >= 32, S >= 16, at most 4 strips of 64 columns per CU, and not in place with a last strip of less than 16 bytes\"},{\"symbol\":\"" << e.symbol
+      << "\",\"block\":576,\"when\":\"B >= 32, S >= 16, at most one strip of 64 columns per CU, or two where S >= 200 (8-byte elements 100), or four where S >= 512 (400), and not in place with a last strip of less than 16 bytes\"},{\"symbol\":\"" << e.symbol
       << "\",\"when\":\"otherwise\"},{\"symbol\":\""
       << L.entries.back().symbol << "\",\"when\":\"" << kStridedWhen << "\"}],\"workspace\":null"
       << ",\"compiler_args\":[\"--offload-arch=gfx950\",\"-O3\",\"-Xclang\",\"-target-feature\",\"-Xclang\",\"-packed-fp32-ops\"]"

@@ -1272,13 +1272,20 @@ int32_t run_scan(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_err
     if (a0 == 0 || S == 0 || b0 == 0) return UNP_OK;
     uint64_t in = A.buf[0], out = A.buf[1];
     const uint32_t grid = (uint32_t)(x->cu_count * x->l.blocks_per_cu);
-    // Up to four strips of 64 columns per CU stream through LDS (rows of at least half a strip); more
-    // columns than that keep enough loads in flight with a lane each.  A last strip of less than a
+    // Strips of 64 columns stream through LDS (rows of at least half a strip) where the chain of one
+    // column bounds the launch: a strip per CU, or more where the rows pay for the tiles of 64 that each strip's
+    // start and end leave part empty.  A lane per column keeps enough loads in flight by itself from about four
+    // strips per CU on.  F32, lanes / strips: 128 x 250 strips 6.2 / 5.6 us, 128 x 300 6.2 / 8.5, 200 x 500
+    // 15.0 / 10.9, 200 x 1000 18.8 / 21.5, 500 x 1000 42.8 / 43.7, 1000 x 1000 116 / 82; I64 128 x 300 10.8 / 9.8,
+    // 500 x 1000 88.7 / 79.9.  A last strip of less than a
     // vector also scans columns of the strip before it, which in place that strip's block may have
     // stored already: those launches go by columns too.
     const long long ncb = (b0 + 63) / 64, strips = a0 * ncb, vec = 16 / (long long)unp::kind_bytes(f.dtype);
     const bool torn = in == out && b0 % 64 > 0 && b0 % 64 < vec;
-    if (b0 >= 32 && S >= 16 && strips <= 4LL * x->cu_count && !torn) {
+    const long long cus = x->cu_count;
+    const bool chain = strips <= cus || (strips <= 2 * cus && S >= (vec == 4 ? 200 : 100)) ||
+                       (strips <= 4 * cus && S >= (vec == 4 ? 512 : 400));
+    if (b0 >= 32 && S >= 16 && chain && !torn) {
       int32_t wide = b0 % vec == 0 && aligned16(in);
       long long n = strips, c = ncb;
       void* params[] = {&in, &out, &S, &b0, &n, &c, &wide};
