@@ -53,3 +53,24 @@ def test_normal_values_keep_their_bits_and_the_bound(hip_device, rows, cols):
     bound = 2 * (k / (1 - k)) * np.cumsum(np.abs(x.astype(np.float64)), axis=1)
     want = oracle.scan_rows(x, "Sum").astype(np.float64)
     assert (np.abs(runs[0].astype(np.float64) - want) <= bound + np.spacing(np.abs(runs[0])).astype(np.float64)).all()
+
+
+# A wave's and a block's registers, the staged tiles, and the register tiles at one per CU and past it.
+@pytest.mark.parametrize("dtype,rows,cols,tail", [
+    ("I32", 3, 1024, "_r1"), ("I32", 3, 1025, "_r8"), ("I32", 3, 16384, "_r8"), ("I32", 3, 16388, "_v"),
+    ("I32", 1, 16385, "_s1"), ("I32", 128, 16385, "_s1"), ("I32", 129, 16385, "_s"), ("I32", 1, 256 * 16384 - 1, "_s1"),
+    ("I32", 1, 256 * 16384 + 1, "_s"), ("F32", 1, 16385, "_s"), ("I64", 3, 8192, "_r8"), ("I64", 3, 8193, "_s"),
+    ("I64", 3, 8194, "_v")])
+def test_the_entry_follows_the_row(hip_device, dtype, rows, cols, tail):
+    x = synth.int16_i32(13, rows * cols).astype(NT[dtype]).reshape(rows, cols)
+    op = "Max" if dtype == "F32" else "Sum"
+    H.say(f"[case] row scan entry {rows}x{cols} {dtype}")
+    for reverse, exclusive in ((False, False), (True, True)):
+        ex = H.executor(kind="scan", dtype=dtype, rank=2, op=op, reverse=reverse,
+                        exclusive=exclusive)
+        din, dout = u.DeviceBuffer.from_array(x), u.DeviceBuffer(x.nbytes)
+        ex.launch(din, dout, rows, cols)
+        ex.check()
+        assert ex.last_launch()["entry"] == ex.kernel.name + tail
+        want = oracle.scan_rows(x, op, exclusive, reverse)
+        assert np.array_equal(dout.download(NT[dtype], x.size).reshape(x.shape), want)

@@ -1307,7 +1307,9 @@ int32_t run_scan(unp_exec* x, const unp_arg* a, size_t n, hipStream_t s, unp_err
     void* params[] = {&in, &out, &rows, &cols};
     return launch(x, i, (uint32_t)(x->cu_count * en.blocks_per_cu), params, s, err);
   }
-  const size_t entry = pick(x, cols % vec == 0 && aligned16(in) && aligned16(out));
+  size_t entry = pick(x, cols % vec == 0 && aligned16(in) && aligned16(out));
+  // At most a tile per CU of the register scan (16384 positions): the entry after it, where there is one.
+  if (!x->l.entries[entry].fast && x->l.entries[entry + 1].lane && rows * ((cols + 16383) / 16384) <= x->cu_count) ++entry;
   const unp::Entry& en = x->l.entries[entry];
   // A block tile: wpb (consumer) waves x 64 lanes x vec x k positions of one row.
   const long long tile = 64LL * en.vec * en.k * en.wpb;

@@ -32,7 +32,7 @@ struct Entry {
   int blocks_per_cu = 0;  // persistent blocks per CU of this entry (0: the form's)
   bool team = false;      // split reduction: a wave per output or column strip; elementwise: the
                           // tiled entry (vec: its tile's rows); scan: a row in registers
-  bool lane = false;      // split reduction: a lane per output, or per vector of columns
+  bool lane = false;      // split reduction: a lane per output, or per vector of columns; scan: few tiles
   int cols = 0;           // output columns per block (dequant GEMM decode entries)
   // Reads and writes its buffers through storage-image strides (unp_hip_exec_launch_views with a
   // view that is not dense row-major); never picked for a pointer launch.
