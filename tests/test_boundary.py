@@ -933,3 +933,38 @@ def test_general_gather_lift_follows_the_gather_lift():
     with pytest.raises(_lib.UnpError) as e:
         u.HipBackend().lower_kernel(ki)
     assert e.value.kind == "UnsupportedKernel"
+
+
+def test_a_failed_launch_reports_its_own_threads_error():
+    """Two threads in Executor.launch at once: one call's message is not the other's to clear."""
+    import threading
+
+    ex = u.Executor.__new__(u.Executor)
+    ex._h = None
+    step = threading.Barrier(2, timeout=20)
+    said = {}
+
+    def launch(handle, words, nargs, stream, perr):  # unp_hip_exec_launch as far as the error goes
+        fails = threading.current_thread().name == "fails"
+        if not fails:
+            step.wait()
+        perr._obj.detail = b"this launch failed" if fails else b""
+        if fails:
+            step.wait()
+        step.wait()
+        return _lib.HIP_ERROR if fails else _lib.OK
+
+    ex._launch = launch
+
+    def call():
+        try:
+            ex.launch(1)
+        except u.UnpError as e:
+            said[threading.current_thread().name] = str(e)
+
+    threads = [threading.Thread(target=call, name=n) for n in ("fails", "works")]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert list(said) == ["fails"] and "this launch failed" in said["fails"]

@@ -15,6 +15,7 @@ from __future__ import annotations
 import ctypes as C
 import json
 import struct
+import threading
 from dataclasses import dataclass
 
 import numpy as np
@@ -387,6 +388,17 @@ class _ArgWords(dict):
 _ARG_WORDS = _ArgWords()
 
 
+class _CallError(threading.local):
+    """A thread's unp_error for launches: made once, and no other thread's call writes into it."""
+
+    def __init__(self):
+        self.value = _lib.Error()
+        self.ref = C.byref(self.value)
+
+
+_CALL_ERROR = _CallError()
+
+
 class Executor:
     """A lowered kernel compiled, loaded and ready to launch on the current device."""
 
@@ -396,10 +408,7 @@ class Executor:
         err = _lib.Error()
         check(_lib.lib().unp_hip_exec_create(kernel._handle, C.byref(h), C.byref(err)), err)
         self._h = h
-        # One caller at a time: launches share an error and look nothing up.
-        self._err = err
-        self._perr = C.byref(err)
-        self._launch = _lib.lib().unp_hip_exec_launch
+        self._launch = _lib.lib().unp_hip_exec_launch  # launches look nothing up
 
     @staticmethod
     def _args(args):
@@ -417,9 +426,9 @@ class Executor:
         words = []
         for a in args:
             words += (1, a.ptr) if isinstance(a, DeviceBuffer) else (0, int(a) & 0xFFFFFFFFFFFFFFFF)
-        rc = self._launch(self._h, _ARG_WORDS[len(args)](*words), len(args), stream, self._perr)
+        rc = self._launch(self._h, _ARG_WORDS[len(args)](*words), len(args), stream, _CALL_ERROR.ref)
         if rc:
-            check(rc, self._err)
+            check(rc, _CALL_ERROR.value)
 
     def launch_static(self, *args, stream: int = 0) -> None:
         """``launch`` with every workspace in the library's static device scratch
