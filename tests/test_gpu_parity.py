@@ -456,7 +456,7 @@ def test_scan_unaligned_takes_the_register_path(hip_device):
     dout = u.DeviceBuffer(x.nbytes)
     ex.launch(din, dout, 1, x.shape[1])
     u.synchronize()
-    assert ex.last_launch()["entry"].endswith("_s")
+    assert ex.last_launch()["entry"] == ex.kernel.name + "_1_s"
     assert np.array_equal(dout.download(np.int32, x.size).reshape(x.shape), oracle.scan_rows(x, "Sum"))
 
 
@@ -1209,7 +1209,8 @@ def test_row_reduce_two_inputs_rank_three(hip_device):
 def test_row_reduce_entries_and_reproducibility(hip_device):
     """Each entry runs where it should, and a launch repeats bit for bit."""
     stages, epi = X.softmax()
-    for shape, suffix in (((8, 4096), "_c4"), ((8, 6000), "_c"), ((8, 8196), "_v"), ((8, 4099), "_s")):
+    for shape, suffix in (((8, 4096), "_c4"), ((8, 6000), "_c"), ((8, 8196), "_c512_v"), ((8, 4099), "_c_s"),
+                          ((8, 20000), "_p_v")):
         H.say(f"[case] row_reduce entry {suffix} {shape}")
         x = rng(37).normal(size=shape).astype(np.float32)
         ex = H.row_reduce_executor("F32", 2, stages, epi)
@@ -1219,7 +1220,7 @@ def test_row_reduce_entries_and_reproducibility(hip_device):
             ex.launch(din, dout, *shape)
             u.synchronize()
             outs.append(dout.download(np.float32, x.size).reshape(shape))
-        assert ex.last_launch()["entry"].endswith(suffix)
+        assert ex.last_launch()["entry"] == ex.kernel.name + suffix
         assert np.array_equal(outs[0], outs[1])
         assert ulps(outs[0], oracle.row_reduce([x], stages, epi)).max() <= 2
 

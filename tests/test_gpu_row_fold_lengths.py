@@ -28,3 +28,19 @@ def test_sums_and_maxima_of_rows_of_any_length(hip_device, rows, cols, dtype, nt
         u.synchronize()
         assert np.array_equal(s.download(nt, rows), want) and np.array_equal(t.download(nt, rows), want)
         assert np.array_equal(m.download(nt, rows), x.max(axis=1))
+
+
+@pytest.mark.parametrize("rows,cols,shift,tail", [
+    (7, 64, 0, "_wv"), (7, 64, 4, "_ws"), (7, 63, 0, "_ws"), (300, 4096, 0, "_wv"), (256, 4095, 0, "_ws"),
+    (256, 4096, 0, "_bv"), (256, 4096, 4, "_bs"), (256, 4097, 0, "_bs"), (257, 4096, 0, "_wv"),
+    (257, 32768, 0, "_wv"), (257, 32772, 0, "_bv"), (257, 32769, 0, "_bs")])
+def test_the_entry_follows_the_rows(hip_device, rows, cols, shift, tail):
+    x = (synth.int16_i32(9, rows * cols) - 9).astype(np.float32).reshape(rows, cols)
+    ex = H.executor(kind="reduction", dtype="F32", rank=2, op="Sum", reduced_from=1)
+    H.say(f"[case] row fold entry {rows}x{cols} +{shift}")
+    src, dst = u.DeviceBuffer(x.nbytes + 64), u.DeviceBuffer(rows * 4)
+    src.at(shift).upload(x)
+    ex.launch(src.at(shift), dst, rows, cols)
+    u.synchronize()
+    assert ex.last_launch()["entry"] == ex.kernel.name + tail
+    assert np.array_equal(dst.download(np.float32, rows), x.astype(np.int64).sum(axis=1).astype(np.float32))

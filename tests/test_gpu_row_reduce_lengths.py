@@ -69,6 +69,8 @@ def test_two_inputs_nan_and_infinities_in_chunks(hip_device):
     with np.errstate(all="ignore"):
         want = oracle.row_reduce([a, b], stages, epi)
     assert np.array_equal(H.row_reduce([a, b], stages, epi), want, equal_nan=True)
+    last = H.row_reduce_executor("F32", 2, stages, epi, n_inputs=2).last_launch()
+    assert last["entry"].endswith("_p_v") and last["chunks"] == 5 and last["shared"]
 
 
 @pytest.mark.parametrize("cols,entry", [(257, "_s"), (1281, "_s"), (2305, "_c4_s"), (4353, "_c_s"), (8193, "_c512_s")])

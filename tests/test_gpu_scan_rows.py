@@ -58,7 +58,7 @@ def test_normal_values_keep_their_bits_and_the_bound(hip_device, rows, cols):
 # A wave's and a block's registers, the staged tiles, and the register tiles at one per CU and past it.
 @pytest.mark.parametrize("dtype,rows,cols,tail", [
     ("I32", 3, 1024, "_r1"), ("I32", 3, 1025, "_r8"), ("I32", 3, 16384, "_r8"), ("I32", 3, 16388, "_v"),
-    ("I32", 1, 16385, "_s1"), ("I32", 128, 16385, "_s1"), ("I32", 129, 16385, "_s"), ("I32", 1, 256 * 16384 - 1, "_s1"),
+    ("I32", 1, 16385, "_1_s"), ("I32", 128, 16385, "_1_s"), ("I32", 129, 16385, "_s"), ("I32", 1, 256 * 16384 - 1, "_1_s"),
     ("I32", 1, 256 * 16384 + 1, "_s"), ("F32", 1, 16385, "_s"), ("I64", 3, 8192, "_r8"), ("I64", 3, 8193, "_s"),
     ("I64", 3, 8194, "_v")])
 def test_the_entry_follows_the_row(hip_device, dtype, rows, cols, tail):

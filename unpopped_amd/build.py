@@ -85,7 +85,7 @@ CHECK_INSTANTIATIONS = r"""
 #include "unp_device.hip"
 #define KB __launch_bounds__(256)
 // The descriptors the host passes by value (runtime.cpp asserts the same sizes for its images).
-static_assert(sizeof(unp::red_axes) == 60 * 8, "red_axes");
+static_assert(sizeof(unp::red_axes) == 61 * 8, "red_axes");
 static_assert(sizeof(unp::red_view) == 44 * 8, "red_view");
 static_assert(sizeof(unp::scan_view) == 29 * 8, "scan_view");
 static_assert(sizeof(unp::gather_view) == 35 * 8, "gather_view");

@@ -564,7 +564,7 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
   //      wave streaming the next tile into LDS by DMA plus NC consumer waves, one block per
   //      CU (two LDS buffers of one 72 KiB tile each);
   //  _s  anything else: the register scan, 16384-element tiles in 16-byte vectors at any alignment;
-  //  _s1 the same an element per lane, for i32 with at most a tile per CU: there the time is
+  //  _1_s the same an element per lane, for i32 with at most a tile per CU: there the time is
   //      one tile's and the look-back's, which the vectors lengthen (i32: one row of 100001 10.2 us,
   //      13.2 in vectors, 16 of 100001 12.4 and 16.3; 256 of 131073 99.0 and 69.5).
   // Rows of at most 1024 and 16384 elements of 4 bytes (half as many of 8) fit a wave's or a block's
@@ -604,7 +604,7 @@ static int32_t lower_scan(const unp_form& f, Lowered& L, std::string& why) {
     e.k = 16384 / (64 * e.vec * e.wpb);
     e.threads = 64 * e.wpb;
     e.blocks_per_cu = wide_carry ? 1 : 3;
-    e.symbol = L.name + (few ? "_s1" : "_s");
+    e.symbol = L.name + (few ? "_1_s" : "_s");
     src << "extern \"C\" __global__ void __launch_bounds__(" << e.threads << ") " << e.symbol << "(const " << T
         << "* in, " << T << "* out, long long rows, long long cols, unsigned long long* status, "
         << "unsigned* counter, unsigned ticket_base, unsigned epoch, unp::waits wt) {\n  unp::scan_lookback<" << T << ", " << f.op0

@@ -940,16 +940,17 @@ UNP_DEV void xreduce_all(const T* const* __restrict__ in, T* __restrict__ out, i
 // ---------------------------------------------------------------------------------------
 
 // The axes of one launch, outermost first, adjacent axes of a kind merged and the innermost run
-// taken out: it holds L contiguous elements (reduced for xreduce_inner, kept for xreduce_outer).  What
-// every launch reads lies in the first two cache lines, with the reciprocals of its divisors: a launch
-// of a few microseconds waits for each line of its arguments in turn, and a division in f64 at its start
-// takes as long as a load.
+// taken out: it holds L contiguous elements (reduced for xreduce_inner, kept for xreduce_outer).  What every
+// launch reads lies in the first three cache lines of its arguments, with the reciprocals of its divisors: a
+// launch of a few microseconds waits for each line of its arguments in turn, and a division in f64 at its
+// start takes as long as a load.
 struct red_axes {
   i64 L;
   i64 runs;             // innermost runs: of one output's positions (reduced), of the outputs (kept)
   i64 count, S;         // reduced positions per output, chunks they are cut into
   i64 per, units;       // parts of a run (vectors, or column strips); outputs, strips or vectors in all
   double inv_per, inv_units, inv_S;
+  i64 step;             // rstr[0]
   i32 nk, nr;           // kept / reduced axes besides the innermost run
   i32 lpr, rpi;         // xreduce_outer: lanes per row, rows per load
   i32 alone, pad;       // xreduce_outer_alone: lanes of a strip
@@ -1038,7 +1039,7 @@ UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out,
         const i64 c = r * VEC, at = c + VEC <= d.L ? c : d.L - VEC;
         skip[u] = ok ? (int)(c - at) : VEC;
         i64 run;
-        if constexpr (decltype(one)::value) run = q * d.rstr[0];
+        if constexpr (decltype(one)::value) run = q * d.step;
         else run = unravel(q, d.nr, d.rext, d.rstr, d.rinv);
         const i64 off = base + (ok ? run + at : 0);
 #pragma unroll
@@ -1180,7 +1181,7 @@ template <class T, int NI, int OP, class OPS, int VEC, int U> struct outer_lanes
       // Whole passes: a lane's address and a uniform offset per load.  (The pieces' bounds are uniform; as
       // long as the compiler took them for a lane's own it multiplied every row out per lane, and the f64
       // column sums of 4096 x 4096 took 38.9 us on cold caches, 33.2 now.)
-      const i64 stride = d.rstr[0], lane0 = base + c + sub * stride;
+      const i64 stride = d.step, lane0 = base + c + sub * stride;
       for (; i + U * rpi <= w1; i += U * rpi) {
         vec<T, VEC> x[U][NI];
 #pragma unroll
@@ -1203,7 +1204,7 @@ template <class T, int NI, int OP, class OPS, int VEC, int U> struct outer_lanes
           for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
         }
       };
-      if (one) load([&](i64 row) { return row * d.rstr[0]; });
+      if (one) load([&](i64 row) { return row * d.step; });
       else load([&](i64 row) { return unravel(row, d.nr, d.rext, d.rstr, d.rinv); });
       take(x, [&](int u) { return i + u * rpi + sub < w1; });
     }
@@ -1357,7 +1358,7 @@ UNP_DEV void xreduce_outer_alone(const T* const* __restrict__ in, T* __restrict_
 #pragma unroll
           for (int u = 0; u < U; ++u) {
             const i64 rr = i + u * rpi < w1 ? i + u * rpi : i;  // past the piece a row of it is read and ignored
-            const i64 off = base + (d.nr <= 1 ? rr * d.rstr[0] : unravel(rr, d.nr, d.rext, d.rstr, d.rinv));
+            const i64 off = base + (d.nr <= 1 ? rr * d.step : unravel(rr, d.nr, d.rext, d.rstr, d.rinv));
 #pragma unroll
             for (int k = 0; k < NI; ++k) x[u][k] = ld_any<T, VEC>(in[k] + off);
           }
@@ -1474,7 +1475,7 @@ UNP_DEV void xreduce_lanes(const T* const* __restrict__ in, T* __restrict__ out,
         if constexpr (INNER) {
           const i64 at = r * VEC + VEC <= d.L ? r * VEC : d.L - VEC;
           skip[u] = ok ? (int)(r * VEC - at) : VEC;
-          off = at + (d.nr <= 1 ? q * d.rstr[0] : unravel(q, d.nr, d.rext, d.rstr, d.rinv));
+          off = at + (d.nr <= 1 ? q * d.step : unravel(q, d.nr, d.rext, d.rstr, d.rinv));
           if (k0 + u + 1 < n && ++r == d.per) {
             r = 0;
             ++q;
@@ -1482,7 +1483,7 @@ UNP_DEV void xreduce_lanes(const T* const* __restrict__ in, T* __restrict__ out,
         } else {
           const i64 row = ok ? k0 + u : n - 1;
           skip[u] = ok ? 0 : VEC;
-          off = d.nr <= 1 ? row * d.rstr[0] : unravel(row, d.nr, d.rext, d.rstr, d.rinv);
+          off = d.nr <= 1 ? row * d.step : unravel(row, d.nr, d.rext, d.rstr, d.rinv);
         }
 #pragma unroll
         for (int k = 0; k < NI; ++k) x[u][k] = ld_cached<T, VEC>(in[k] + base + off);

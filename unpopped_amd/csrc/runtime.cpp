@@ -762,6 +762,7 @@ long long fill_red_axes(const std::vector<int64_t>& ext, int32_t rank, uint32_t 
   std::reverse(d.rstr, d.rstr + d.nr);
   for (int32_t i = 0; i < d.nk; ++i) d.kinv[i] = 1.0 / (double)d.kext[i];
   for (int32_t i = 0; i < d.nr; ++i) d.rinv[i] = 1.0 / (double)d.rext[i];
+  d.step = d.rstr[0];
   const long long total = last ? d.count : outs;
   d.runs = d.L > 0 ? total / d.L : 0;
   return outs;
@@ -924,7 +925,7 @@ static_assert(sizeof(unp::red_view_host) == 44 * 8, "red_view_host mirrors the d
 static_assert(sizeof(unp::scan_view_host) == 29 * 8, "scan_view_host mirrors the device's scan_view");
 static_assert(sizeof(unp::ew_tile_view_host) == 114 * 8, "ew_tile_view_host mirrors the device's ew_tile_view");
 static_assert(sizeof(unp::gather_view_host) == 35 * 8, "gather_view_host mirrors the device's gather_view");
-static_assert(sizeof(unp::red_axes_host) == 60 * 8, "red_axes_host mirrors the device's red_axes");
+static_assert(sizeof(unp::red_axes_host) == 61 * 8, "red_axes_host mirrors the device's red_axes");
 
 int32_t launch(unp_exec* x, size_t entry, uint32_t grid, void** params, hipStream_t s, unp_error* err) {
   const uint32_t threads = (uint32_t)(x->l.entries[entry].threads ? x->l.entries[entry].threads : x->l.threads);

@@ -57,6 +57,7 @@ struct red_axes_host {
   long long count, S;
   long long per, units;
   double inv_per, inv_units, inv_S;
+  long long step;
   int32_t nk, nr, lpr, rpi, alone, pad;
   long long kstr[8], rstr[8];
   long long kext[8], rext[8];
