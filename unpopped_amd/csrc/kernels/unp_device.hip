@@ -1141,7 +1141,7 @@ UNP_DEV void xreduce_inner(const T* const* __restrict__ in, T* __restrict__ out,
 // per column), all in flight together, and the groups meet in a tree.  The order is fixed by (S, WAVES,
 // U, L, LPR), so the result is reproducible.  counters[strip] is zero on entry and left zero; the
 // partials carry the launch's `epoch`.  6000 x 2050 f32 column norms (49 MB) take 15.6 us, where a wave
-// per column took 59.3; 8192 x 4096 f32 column sums (134 MB) 23.7 launched one after another and 27 on
+// per column took 59.3; 8192 x 4096 f32 column sums (134 MB) 23.7 launched one after another and 27.2 on
 // cold caches.
 //
 // How the lanes of a wave lie on a strip's columns and rows, and their fold of a run of rows.
@@ -1179,8 +1179,8 @@ template <class T, int NI, int OP, class OPS, int VEC, int U> struct outer_lanes
     const bool one = d.nr <= 1;
     if (one) {
       // Whole passes: a lane's address and a uniform offset per load.  (The pieces' bounds are uniform; as
-      // long as the compiler took them for a lane's own it multiplied every row out per lane, and the f64
-      // column sums of 4096 x 4096 took 38.9 us on cold caches, 33.2 now.)
+      // long as the compiler took them for a lane's own it multiplied every row out per lane, and the f32
+      // column maxima of 8192 x 4096 took 28.6 us on cold caches, 27.6 now.)
       const i64 stride = d.step, lane0 = base + c + sub * stride;
       for (; i + U * rpi <= w1; i += U * rpi) {
         vec<T, VEC> x[U][NI];
