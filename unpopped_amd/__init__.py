@@ -15,8 +15,8 @@ from __future__ import annotations
 import ctypes as C
 import json
 import struct
-import threading
 from dataclasses import dataclass
+from threading import get_ident
 
 import numpy as np
 
@@ -388,15 +388,16 @@ class _ArgWords(dict):
 _ARG_WORDS = _ArgWords()
 
 
-class _CallError(threading.local):
-    """A thread's unp_error for launches: made once, and no other thread's call writes into it."""
+class _CallErrors(dict):
+    """A thread's reference to its unp_error for launches, by the thread's number: made once, and no other
+    running thread's call writes into it."""
 
-    def __init__(self):
-        self.value = _lib.Error()
-        self.ref = C.byref(self.value)
+    def __missing__(self, thread: int):
+        self[thread] = C.byref(_lib.Error())
+        return self[thread]
 
 
-_CALL_ERROR = _CallError()
+_CALL_ERRORS = _CallErrors()
 
 
 class Executor:
@@ -426,9 +427,10 @@ class Executor:
         words = []
         for a in args:
             words += (1, a.ptr) if isinstance(a, DeviceBuffer) else (0, int(a) & 0xFFFFFFFFFFFFFFFF)
-        rc = self._launch(self._h, _ARG_WORDS[len(args)](*words), len(args), stream, _CALL_ERROR.ref)
+        err = _CALL_ERRORS[get_ident()]
+        rc = self._launch(self._h, _ARG_WORDS[len(args)](*words), len(args), stream, err)
         if rc:
-            check(rc, _CALL_ERROR.value)
+            check(rc, err._obj)
 
     def launch_static(self, *args, stream: int = 0) -> None:
         """``launch`` with every workspace in the library's static device scratch
