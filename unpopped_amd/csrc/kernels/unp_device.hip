@@ -1278,29 +1278,36 @@ UNP_DEV void xreduce_outer(const T* const* __restrict__ in, T* __restrict__ out,
       done = last != 0u;
       const int g = (int)((u32)tid / (u32)cw), col = tid - g * cw;
       if (done && g < G) {
-        constexpr int Q = 8;  // partials of a column in flight
         a = F::identity();
-        const bool live = c0 + col < B;
-        for (i64 k = g; live && k < S; k += Q * G) {
-          Ac v[Q];
-          bool ok = true;
-#pragma unroll
-          for (int q = 0; q < Q; ++q) {
-            const i64 kk = k + q * G < S ? k + q * G : S - 1;
-            ok = P::take(strip_p + kk * item + col, cw, epoch, v[q]) && ok;
-          }
-          if (!ok) {  // a partial not yet visible: wait for each in turn
+        // Q partials of a column in flight.  The words come from beyond L2, and with eight always asked for,
+        // also of two, the closing fold of an f64 4096 x 4096 took 3.4 us instead of 2.1.
+        auto close = [&](auto n) {
+          constexpr int Q = decltype(n)::value;
+          for (i64 k = g; k < S; k += Q * G) {
+            Ac v[Q];
+            bool ok = true;
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
               const i64 kk = k + q * G < S ? k + q * G : S - 1;
-              v[q] = P::wait(strip_p + kk * item + col, cw, epoch, F::identity(), wt);
+              ok = P::take(strip_p + kk * item + col, cw, epoch, v[q]) && ok;
+            }
+            if (!ok) {  // a partial not yet visible: wait for each in turn
+#pragma unroll
+              for (int q = 0; q < Q; ++q) {
+                const i64 kk = k + q * G < S ? k + q * G : S - 1;
+                v[q] = P::wait(strip_p + kk * item + col, cw, epoch, F::identity(), wt);
+              }
+            }
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+              const Ac b = F::apply(a, v[q]);
+              a = k + q * G < S ? b : a;
             }
           }
-#pragma unroll
-          for (int q = 0; q < Q; ++q) {
-            const Ac b = F::apply(a, v[q]);
-            a = k + q * G < S ? b : a;
-          }
+        };
+        if (c0 + col < B) {
+          if (S <= 2 * G) close(ic<2>{});
+          else close(ic<8>{});
         }
         slots[tid] = a;
       }
